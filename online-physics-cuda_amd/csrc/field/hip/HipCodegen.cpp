@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdio>
 #include <set>
+#include <tuple>
 #include <functional>
 #include <sstream>
 
@@ -22,9 +23,18 @@ typedef long long i64;
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef unsigned long long u64;
 #define IDX(x, y, z) ((i64)(z) * k.nxy + (i64)(y) * k.nx + (i64)(x))
-#define AT(slot, x, y, z) k.A[(i64)(slot) * k.cells + IDX(x, y, z)]
-#define CELL_HEAD const int x = (int)(blockIdx.x * blockDim.x + threadIdx.x); const int y = (int)(blockIdx.y * blockDim.y + threadIdx.y); \
-    const int z = (int)blockIdx.z; if (x >= k.nx || y >= k.ny) return;
+// A row's first cell, and a cell of it: where y and z are the wave's own (CELL_HEAD) the row is scalar arithmetic and a
+// read needs one 32-bit offset of a lane.
+#define ROW(y, z) ((i64)(z) * k.nxy + (i64)(y) * k.nx)
+#define AT(slot, x, y, z) (k.A + ((i64)(slot) * k.cells + ROW(y, z)))[(unsigned)(x)]
+// A thread a cell, a wave 64 cells of one row: a 256-thread block takes four rows of a plane, or of a lattice with fewer
+// than four (flat) a row of four planes. y and z are the same in all a wave's lanes, and nothing here reads the block's
+// size (two of its three numbers come by a vector load that every wave would wait for).
+#define CELL_XYZ const int x = (int)(blockIdx.x * 64u + (threadIdx.x & 63u)); \
+    const int cell_row = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)); \
+    const int y = k.ny < 4 ? (int)blockIdx.y : (int)(blockIdx.y * 4u) + cell_row; \
+    const int z = k.ny < 4 ? (int)(blockIdx.z * 4u) + cell_row : (int)blockIdx.z;
+#define CELL_HEAD CELL_XYZ if (x >= k.nx || y >= k.ny || z >= k.nz) return;
 // A cell's coordinates from its index: 32-bit divisions while the lattice has fewer than 2^31 cells (a 64-bit division
 // is a long software sequence on the card).
 __device__ __forceinline__ void cell_xyz(const K& k, i64 i, int& x, int& y, int& z)
@@ -45,8 +55,12 @@ __device__ __forceinline__ int ez(const K& k, int v) { return max(0, min(v, k.nz
 // reads HBM; a window's LDS holds every coordinate within its reach at the clamped cell's value, so there the
 // coordinate goes unclamped and the neighbours' addresses stay constant offsets of the cell's.
 #define LX(v) (M::kClamps ? ex(k, (v)) : (v))
-#define LY(v) (M::kClamps ? ey(k, (v)) : (v))
-#define LZ(v) (M::kClamps ? ez(k, (v)) : (v))
+#define LY(v) (M::kClamps ? EY(v) : (v))
+#define LZ(v) (M::kClamps ? EZ(v) : (v))
+// M::kInner: the cell's row lies further from the lattice's y and z edges than the law reads, so nothing there is clamped.
+#define EX(v) ex(k, (v))
+#define EY(v) (M::kInner ? (v) : ey(k, (v)))
+#define EZ(v) (M::kInner ? (v) : ez(k, (v)))
 __device__ __forceinline__ bool finite_d(double v) { return __builtin_isfinite(v); }
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return max(lo, min(v, hi)); }
 // a / h, a / h^2, a / (h * span): when the divisor is a power of two (flags, set by the host) the quotient is the exact
@@ -60,9 +74,22 @@ template <class M> __device__ __forceinline__ double div_hh(const K& k, double a
 {
     return (M::kPow2 || (k.flags & 2)) ? a * k.inv_hh : a / (k.h * k.h);
 }
+// A span of no cells (an axis one cell long) divides a cell's difference with itself: NaN, as 0 / 0 or NaN * inf.
 template <class M> __device__ __forceinline__ double div_hs(const K& k, double a, int span)
 {
-    return (M::kPow2 || (k.flags & 1)) && span > 0 ? a * (span == 1 ? k.inv_h : 0.5 * k.inv_h) : a / (k.h * (double)span);
+    if (M::kPow2) return a * (span == 2 ? 0.5 * k.inv_h : (span == 1 ? k.inv_h : __builtin_inf()));
+    return (k.flags & 1) && span > 0 ? a * (span == 1 ? k.inv_h : 0.5 * k.inv_h) : a / (k.h * (double)span);
+}
+// The same quotients of a float, rounded to float: by a power of two both the double product and the float one are exact
+// (or overflow, or flush, alike), so the float product serves. The host sets the flags only where the reciprocals are
+// normal floats.
+template <class M> __device__ __forceinline__ float div_h1(const K& k, float a)
+{
+    return M::kPow2 ? a * (float)k.inv_h : fe_rf(k.h == 0.0 ? 0.0 : div_h<M>(k, (double)a));
+}
+template <class M> __device__ __forceinline__ float div_hh1(const K& k, float a)
+{
+    return M::kPow2 ? a * (float)k.inv_hh : fe_rf(k.h == 0.0 ? 0.0 : div_hh<M>(k, (double)a));
 }
 // Where a value is read from (struct Direct, generated after this prelude: the field's array in HBM; a window kernel
 // has its own, an LDS ring of planes).
@@ -153,7 +180,7 @@ __device__ __forceinline__ void range_fold(unsigned nout, unsigned nnan, u64 fb,
         const u64 other = __shfl_xor(fb, o);
         fb = other < fb ? other : fb;
     }
-    const int t = (int)(threadIdx.y * blockDim.x + threadIdx.x), w = t >> 6, nw = (int)((blockDim.x * blockDim.y + 63) >> 6);
+    const int t = (int)threadIdx.x, w = t >> 6, nw = 4;
     if ((t & 63) == 0) { rn[w] = nout; rb[w] = nnan; rf[w] = fb; }
     __syncthreads();
     if (t == 0) {
@@ -169,10 +196,9 @@ __device__ __forceinline__ void range_fold(unsigned nout, unsigned nnan, u64 fb,
 // index of a bad one (integer atomics: the order does not matter). A clamped field's finite strays are clamped instead.
 extern "C" __global__ void k_range(K k, int field, double lo, double hi, int clamp, unsigned* rec, u64* first)
 {
-    const int x = (int)(blockIdx.x * blockDim.x + threadIdx.x); const int y = (int)(blockIdx.y * blockDim.y + threadIdx.y);
-    const int z = (int)blockIdx.z;
+    CELL_XYZ
     unsigned nout = 0, nnan = 0; u64 fb = ~0ull;
-    if (x < k.nx && y < k.ny) {
+    if (x < k.nx && y < k.ny && z < k.nz) {
         const i64 i = IDX(x, y, z);
         const float v = k.now[field][i];
         const double d = (double)v;
@@ -421,34 +447,40 @@ public:
         const int nf = std::max(1, lay_.fields);
         out_ << "// generated by the Field Engine's --hip emitter for gfx950\n";
         out_ << FE_EXACT_HELPERS_TEXT;
-        // The params travel by value in the arguments (the kernarg segment is read-only: the compiler hoists every read
+        // The params (and KF, the face conductance between two cells of a param's value: the harmonic mean 2 k k / (k + k) as
+        // the CPU computes it) travel by value in the arguments (the kernarg segment is read-only: the compiler hoists every read
         // of them out of loops), so a step's launches carry the values they were queued with.
         const int np = std::max(1, static_cast<int>(law_.param_values.size()));
         const int nu = std::max(1, lay_.uniforms);
         out_ << "struct K {\n    float* now[" << nf << "];\n    float* nxt[" << nf << "];\n"
              << "    const double* U;\n    float* A;\n    double* S;\n    double* L;\n    unsigned* C;\n    const float* N;\n"
              << "    long long nxy;\n    long long cells;\n    double h;\n    double dt;\n    double inv_h;\n    double inv_hh;\n"
-             << "    int nx;\n    int ny;\n    int nz;\n    int flags;\n    double P[" << np << "];\n};\n";
-        lay_.kernel_arg_bytes = (2 * nf + 6) * 8 + 6 * 8 + 4 * 4 + 8 * np;
+             << "    int nx;\n    int ny;\n    int nz;\n    int flags;\n    double P[" << np << "];\n    double KF[" << np << "];\n};\n";
+        lay_.kernel_arg_bytes = (2 * nf + 6) * 8 + 6 * 8 + 4 * 4 + 16 * np;
         out_ << "#define FE_BOUND_SLOTS " << kBoundSlots << "\n";
         out_ << kPrelude;
         // Reductions' results are read once a kernel into registers (a load inside the z loop would be repeated and,
         // waited for, would drain the loads in flight).
         out_ << "struct Direct {\n    static constexpr bool kClamps = true;\n    static constexpr bool kExact = true;\n"
-             << "    static constexpr bool kPow2 = false;\n    __device__ void flag(bool) const {}\n    double u[" << nu << "];\n"
+             << "    static constexpr bool kPow2 = false;\n    static constexpr bool kInner = false;\n    static constexpr bool bad = false;\n"
+             << "    __device__ void flag(bool) const {}\n    double u[" << nu << "];\n"
              << "    __device__ explicit Direct(const K& k) { for (int q = 0; q < " << nu << "; ++q) u[q] = " << (lay_.uniforms > 0 ? "k.U[q]" : "0.0")
              << "; }\n"
-             << "    template <int F> __device__ __forceinline__ float fld(const K& k, int x, int y, int z) const { return k.now[F][IDX(x, y, z)]; }\n"
-             << "    template <int F> __device__ __forceinline__ float fld_any(const K& k, int x, int y, int z) const { return k.now[F][IDX(x, y, z)]; }\n"
+             << "    template <int F> __device__ __forceinline__ float fld(const K& k, int x, int y, int z) const { return (k.now[F] + ROW(y, z))[(unsigned)x]; }\n"
+             << "    template <int F> __device__ __forceinline__ float fld_any(const K& k, int x, int y, int z) const { return fld<F>(k, x, y, z); }\n"
              << "};\n"
-             // The direct view specialised: W32, reads with 32-bit index arithmetic (lattices of fewer than 2^31 cells: a
-             // 64-bit product a read is several instructions, and a law's gather makes dozens of reads a cell); P2, h a
-             // power of two, so a division by h or h^2 is the exact product with the reciprocal and no division is left
-             // in the code (a run-time choice between the two would have the card compute both).
-             << "template <bool W32, bool P2> struct DirectT : Direct {\n    static constexpr bool kPow2 = P2;\n"
+             // The direct view specialised: W32, a row's first cell and a cell's byte offset in it in 32-bit
+             // arithmetic (lattices of fewer than 2^30 cells); P2, h a power of two, so a division by h or h^2 is the exact product with the reciprocal and no
+             // division is left in the code (a run-time choice between the two would have the card compute both); IN, a
+             // row away from the lattice's y and z edges (M::kInner), in the fast forms (a cell they flag is taken again
+             // in the exact ones).
+             << "template <bool W32, bool P2, bool IN = false> struct DirectT : Direct {\n    static constexpr bool kPow2 = P2;\n"
+             << "    static constexpr bool kInner = IN;\n    static constexpr bool kExact = !IN;\n    mutable bool bad = false;\n"
+             << "    __device__ __forceinline__ void flag(bool b) const { if (IN) bad = bad || b; }\n"
              << "    __device__ explicit DirectT(const K& k) : Direct(k) {}\n"
              << "    template <int F> __device__ __forceinline__ float fld(const K& k, int x, int y, int z) const\n"
-             << "    { return W32 ? k.now[F][(unsigned)z * (unsigned)k.nxy + (unsigned)y * (unsigned)k.nx + (unsigned)x] : k.now[F][IDX(x, y, z)]; }\n"
+             << "    {\n        if (W32) return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(k.now[F] + ((unsigned)z * (unsigned)k.nxy + (unsigned)y * (unsigned)k.nx)) + (unsigned)x * 4u);\n"
+             << "        return (k.now[F] + ROW(y, z))[(unsigned)x];\n    }\n"
              << "    template <int F> __device__ __forceinline__ float fld_any(const K& k, int x, int y, int z) const { return fld<F>(k, x, y, z); }\n"
              << "};\n"
              << "#define FE_POW2(k) (((k).flags & 3) == 3)\n";
@@ -579,7 +611,7 @@ private:
     // or through LX/LY/LZ when the argument is a field itself (the memory it is read from decides).
     std::string cl(int arg, int a, const std::string& v) const
     {
-        static const char* direct[3] = {"ex(k, ", "ey(k, ", "ez(k, "};
+        static const char* direct[3] = {"EX(", "EY(", "EZ("};
         static const char* leaf[3] = {"LX(", "LY(", "LZ("};
         const bool is_leaf = at(arg).op == Op::Field && lay_.stages.count(arg) == 0;
         return std::string(is_leaf ? leaf[a] : direct[a]) + v + ")";
@@ -674,11 +706,12 @@ private:
             // Zero times anything is zero on the CPU, without looking at the anything (src/field/Law.cpp:804-843).
             const int a = in.args[0];
             const int b = in.args[1];
-            if (scalar(a) || scalar(b)) {
-                const int s = scalar(a) ? a : b;
-                f << "    const double s = s" << s << "(k, m);\n    if (s == 0.0) return 0.0f;\n";
+            const std::string one = narrow(in), product = one.empty() ? "fe_rf(" + d(a) + " * " + d(b) + ")" : one;
+            if (scalar(a) || scalar(b)) { // a select, not a branch: the reads behind the product stay with the others
+                f << "    const float p = " << product << ";\n    return s" << (scalar(a) ? a : b) << "(k, m) == 0.0 ? 0.0f : p;\n";
+            } else {
+                f << "    return " << product << ";\n";
             }
-            f << "    return fe_rf(" << d(a) << " * " << d(b) << ");\n";
             break;
         }
         case Op::Lap: {
@@ -698,8 +731,9 @@ private:
             const int axis = in.op == Op::Gx ? 0 : (in.op == Op::Gy ? 1 : 2);
             const char* c = axis == 0 ? "x" : (axis == 1 ? "y" : "z");
             const char* cnt = axis == 0 ? "k.nx" : (axis == 1 ? "k.ny" : "k.nz");
-            const std::string hi = std::string(c) + " + 1 < " + cnt + " ? " + c + " + 1 : " + c;
-            const std::string lo = std::string(c) + " > 0 ? " + c + " - 1 : " + c;
+            const std::string inner = axis == 0 ? "" : "M::kInner || ";
+            const std::string hi = inner + c + " + 1 < " + cnt + " ? " + c + " + 1 : " + c;
+            const std::string lo = inner + c + " > 0 ? " + c + " - 1 : " + c;
             f << "    const int hi = " << hi << ";\n    const int lo = " << lo << ";\n";
             const std::string ahi = axis == 0 ? d(in.args[0], "hi") : (axis == 1 ? d(in.args[0], "x", "hi") : d(in.args[0], "x", "y", "hi"));
             const std::string alo = axis == 0 ? d(in.args[0], "lo") : (axis == 1 ? d(in.args[0], "x", "lo") : d(in.args[0], "x", "y", "lo"));
@@ -726,8 +760,12 @@ private:
             // it is literally the +x flux of the cell before it (shared when a lane computes both cells).
             f << "    const double c = " << d(fa) << ";\n";
             if (scalar(kk)) {
-                f << "    const double kv = s" << kk << "(k, m);\n"
-                  << "    const double kf = (kv + kv) > 0.0 ? 2.0 * kv * kv / (kv + kv) : 0.0;\n";
+                if (at(kk).op == Op::Param) {
+                    f << "    const double kf = k.KF[" << at(kk).index << "];\n"; // the same quotient, taken by the host
+                } else {
+                    f << "    const double kv = s" << kk << "(k, m);\n"
+                      << "    const double kf = (kv + kv) > 0.0 ? 2.0 * kv * kv / (kv + kv) : 0.0;\n";
+                }
             } else {
                 f << "    const double ka = " << d(kk) << ";\n";
             }
@@ -774,7 +812,8 @@ private:
               << "    const double zl = " << d(fa, "x", "y", cl(fa, 2, "z - 1")) << "; const double zh = "
               << d(fa, "x", "y", cl(fa, 2, "z + 1")) << ";\n";
             auto up = [&](const char* speed, const char* c, const char* cnt, const char* lo, const char* hi) {
-                return std::string("(") + speed + " > 0.0 ? (" + c + " > 0 ? div_h<M>(k, " + speed + " * (c - " + lo + ")) : 0.0) : (" + c +
+                const std::string inner = c[0] == 'x' ? "" : "M::kInner || ";
+                return std::string("(") + speed + " > 0.0 ? (" + inner + c + " > 0 ? div_h<M>(k, " + speed + " * (c - " + lo + ")) : 0.0) : (" + inner + c +
                     " + 1 < " + cnt + " ? div_h<M>(k, " + speed + " * (" + hi + " - c)) : 0.0))";
             };
             f << "    double o = " << up("u", "x", "k.nx", "xl", "xh") << ";\n"
@@ -784,13 +823,56 @@ private:
             break;
         }
         case Op::ShiftT: {
+            // The cells whose clamped read is this one: a run an axis (run_to), one cell long away from the lattice's
+            // edges (in a row clear of them the axis is the cell shifted back). By one cell along one axis a run has two
+            // cells at most, both read without a branch (clamped, the values dropped where the run is shorter): the sum
+            // from +0 of one or two floats in double, rounded, is the float sum. Other shifts walk their runs.
             const Runtime walk(runtime_);
-            f << "    int lx, hx, ly, hy, lz, hz;\n"
-              << "    run_to(x, " << in.offset[0] << ", k.nx, lx, hx); run_to(y, " << in.offset[1] << ", k.ny, ly, hy); run_to(z, "
-              << in.offset[2] << ", k.nz, lz, hz);\n"
-              << "    double s = 0.0;\n"
-              << "    for (int zz = lz; zz <= hz; ++zz) for (int yy = ly; yy <= hy; ++yy) for (int xx = lx; xx <= hx; ++xx) s += "
-              << d(in.args[0], "xx", "yy", "zz") << ";\n"
+            static const char* axes[3] = {"x", "y", "z"};
+            int moved = 0, along = 0, far = 0;
+            std::string inner[3], cells[3], loops;
+            for (int q = 0; q < 3; ++q) {
+                inner[q] = cells[q] = axes[q];
+                if (in.offset[q] == 0) {
+                    continue;
+                }
+                ++moved;
+                along = q;
+                far = std::max(far, std::abs(in.offset[q]));
+                inner[q] = std::string(axes[q]) + " - (" + std::to_string(in.offset[q]) + ")";
+                cells[q] = std::string(axes[q]) + axes[q];
+            }
+            if (moved == 0) {
+                f << "    return fe_rf(0.0 + " << d(in.args[0]) << ");\n";
+                break;
+            }
+            if (in.offset[0] == 0) {
+                f << "    if constexpr (M::kInner) return fe_rf(0.0 + " << d(in.args[0], inner[0], inner[1], inner[2]) << ");\n";
+            }
+            for (int q = 0; q < 3; ++q) {
+                if (in.offset[q] != 0) {
+                    const std::string a = axes[q];
+                    f << "    int l" << a << ", h" << a << "; run_to(" << a << ", " << in.offset[q] << ", k.n" << a << ", l" << a << ", h" << a << ");\n";
+                }
+            }
+            if (moved == 1 && far == 1) {
+                const std::string a = axes[along];
+                std::string one[3] = {"x", "y", "z"}, two[3] = {"x", "y", "z"};
+                one[along] = "clampi(l" + a + ", 0, k.n" + a + " - 1)";
+                two[along] = "clampi(h" + a + ", 0, k.n" + a + " - 1)";
+                f << "    const float one = " << v(in.args[0], one[0], one[1], one[2]) << ", two = " << v(in.args[0], two[0], two[1], two[2]) << ";\n"
+                  << "    const float s = 0.0f + one;\n"
+                  << "    return l" << a << " > h" << a << " ? 0.0f : (l" << a << " < h" << a << " ? s + two : s);\n";
+                break;
+            }
+            f << "    double s = 0.0;\n    ";
+            for (int q = 2; q >= 0; --q) {
+                if (in.offset[q] != 0) {
+                    const std::string a = axes[q];
+                    f << "for (int " << a << a << " = l" << a << "; " << a << a << " <= h" << a << "; ++" << a << a << ") ";
+                }
+            }
+            f << "s += " << d(in.args[0], cells[0], cells[1], cells[2]) << ";\n"
               << "    return fe_rf(s);\n";
             break;
         }
@@ -905,9 +987,11 @@ private:
             net_faces(in, f);
             break;
         }
-        default:
-            f << "    return fe_rf(" << arith(in, id) << ");\n";
+        default: {
+            const std::string single = narrow(in);
+            f << "    return " << (single.empty() ? "fe_rf(" + arith(in, id) + ")" : single) << ";\n";
             break;
+        }
         }
         f << "}\n";
         out_ << f.str();
@@ -1060,6 +1144,66 @@ private:
 
     // An element-wise op in double over its arguments at (x, y, z), as the CPU's lambdas compute it
     // (src/field/Law.cpp:782-857): std::min/std::max/std::clamp comparisons, not fmin/fmax.
+    bool by_h(const ir::Inst& in) const { return at(in.args[1]).op == Op::Cell; }
+    bool by_hh(const ir::Inst& in) const
+    {
+        const ir::Inst& q = at(in.args[1]);
+        return q.op == Op::Mul && at(q.args[0]).op == Op::Cell && at(q.args[1]).op == Op::Cell;
+    }
+
+    // An argument as a float where it is one exactly: a cell value, or a number that a float holds (normal, or zero).
+    // Empty otherwise.
+    std::string single(int id) const
+    {
+        if (!scalar(id)) {
+            return v(id);
+        }
+        const ir::Inst& q = at(id);
+        const float f = static_cast<float>(q.number);
+        if (q.op != Op::Const || static_cast<double>(f) != q.number || (f != 0.0f && !std::isnormal(f))) {
+            return "";
+        }
+        char text[64];
+        std::snprintf(text, sizeof(text), "(%af)", static_cast<double>(f));
+        return text;
+    }
+
+    // The single-precision form of an element-wise node whose arguments are all floats, or empty. The CPU widens them,
+    // computes in double and rounds once to float; for one sum, difference, product or quotient of two floats that is the
+    // correctly rounded float result (a double holds more than twice a float's digits, so the second rounding changes
+    // nothing), which the float instruction gives directly; comparisons and sign changes are exact either way. It saves a
+    // conversion an argument, one for the result and the register pairs: the transport law's adjoint on 256^3 (an
+    // elementwise and upwind law, bound by its instructions) went from 529 to 333-374 us a gather,
+    // with shift_t's two unconditional reads and the inner rows' forms.
+    std::string narrow(const ir::Inst& in) const
+    {
+        if (in.op == Op::Div && !scalar(in.args[0]) && (by_h(in) || by_hh(in))) {
+            return std::string(by_h(in) ? "div_h1" : "div_hh1") + "<M>(k, " + v(in.args[0]) + ")";
+        }
+        std::vector<std::string> a;
+        for (const int q : in.args) {
+            a.push_back(single(q));
+            if (a.back().empty()) {
+                return "";
+            }
+        }
+        switch (in.op) {
+        case Op::Neg: return "(-" + a[0] + ")";
+        case Op::Abs: return "__builtin_fabsf(" + a[0] + ")";
+        case Op::Step: return "(" + a[0] + " > 0.0f ? 1.0f : 0.0f)";
+        case Op::Pos: return "([](float q) { return q < 0.0f ? 0.0f : q; })(" + a[0] + ")";
+        case Op::Add: return "(" + a[0] + " + " + a[1] + ")";
+        case Op::Sub: return "(" + a[0] + " - " + a[1] + ")";
+        case Op::Mul: return "(" + a[0] + " * " + a[1] + ")";
+        case Op::Min: return "([](float p, float q) { return q < p ? q : p; })(" + a[0] + ", " + a[1] + ")";
+        case Op::Max: return "([](float p, float q) { return p < q ? q : p; })(" + a[0] + ", " + a[1] + ")";
+        case Op::Clamp:
+            return "([](float q, float lo, float h) { const float hi = lo < h ? h : lo; return q < lo ? lo : (hi < q ? hi : q); })(" + a[0] +
+                ", " + a[1] + ", " + a[2] + ")";
+        default: return "";
+        }
+    }
+
     std::string arith(const ir::Inst& in, int id) const
     {
         auto a = [&](std::size_t i) { return d(in.args[i]); };
@@ -1077,11 +1221,8 @@ private:
         case Op::Div: {
             // A division by h or h * h (the lattice spacing): the product with the reciprocal where that is a power of
             // two (the quotient's bits, as div_h and div_hh give the stencils), no division on the card.
-            const ir::Inst& q = at(in.args[1]);
-            const bool by_h = q.op == Op::Cell;
-            const bool by_hh = q.op == Op::Mul && at(q.args[0]).op == Op::Cell && at(q.args[1]).op == Op::Cell;
-            if (by_h || by_hh) {
-                return std::string("(k.h == 0.0 ? 0.0 : ") + (by_h ? "div_h" : "div_hh") + "<M>(k, " + a(0) + "))";
+            if (by_h(in) || by_hh(in)) {
+                return std::string("(k.h == 0.0 ? 0.0 : ") + (by_h(in) ? "div_h" : "div_hh") + "<M>(k, " + a(0) + "))";
             }
             return "([](double p, double q) { return q == 0.0 ? 0.0 : p / q; })(" + a(0) + ", " + a(1) + ")";
         }
@@ -1737,32 +1878,48 @@ private:
             code.swaps = targets;
         }
         const int nt = static_cast<int>(targets.size());
-        // The direct kernel: a thread a cell; `<gather>_32` the same with 32-bit reads (lattices under 2^31 cells).
-        g << "template <class M> __device__ __forceinline__ void d_" << code.gather << "(const K& k, int x, int y, int z)\n{\n"
+        // The direct kernel: a thread a cell; `<gather>_32` the same with 32-bit reads (lattices under 2^30 cells).
+        // False, and nothing written, for a cell the fast forms flag.
+        g << "template <class M> __device__ __forceinline__ bool d_" << code.gather << "(const K& k, int x, int y, int z)\n{\n"
           << "    const M m(k);\n    float o[" << nt << "], n[" << nt << "];\n    " << cellfn << "(k, m, x, y, z, o, n);\n"
-          << "    const i64 i = IDX(x, y, z);\n";
+          << "    if (m.bad) return false;\n    const i64 row = ROW(y, z);\n";
         for (int q = 0; q < nt; ++q) {
             const std::string t = std::to_string(targets[static_cast<std::size_t>(q)]);
             const std::string qs = std::to_string(q);
             g << "    { const bool ch = __float_as_uint(o[" << qs << "]) != __float_as_uint(n[" << qs << "]);\n";
             if (code.in_place) {
-                g << "      if (ch) k.now[" << t << "][i] = n[" << qs << "];\n";
+                g << "      if (ch) (k.now[" << t << "] + row)[(unsigned)x] = n[" << qs << "];\n";
             } else {
-                g << "      k.nxt[" << t << "][i] = n[" << qs << "];\n";
+                g << "      (k.nxt[" << t << "] + row)[(unsigned)x] = n[" << qs << "];\n";
             }
             g << "      mark(k, " << t << ", ch); }\n";
         }
-        g << "}\n";
-        for (const bool w32 : {false, true}) {
-            const std::string w = w32 ? "true" : "false";
-            g << "extern \"C\" __global__ void " << code.gather << (w32 ? "_32" : "") << "(K k) { CELL_HEAD\n"
-              << "    if (FE_POW2(k)) d_" << code.gather << "<DirectT<" << w << ", true>>(k, x, y, z);\n"
-              << "    else d_" << code.gather << "<DirectT<" << w << ", false>>(k, x, y, z);\n}\n";
-        }
-        out_ << g.str();
+        g << "    return true;\n}\n";
         std::map<int, int> reach;
         int cost = 0;
         const bool bounded = field_reach(p, reach, cost);
+        int off_y = 0, off_z = 0;
+        row_reach(p, off_y, off_z);
+        for (const bool w32 : {false, true}) {
+            const std::string w = w32 ? "true" : "false", fn = "d_" + code.gather + "<DirectT<" + w;
+            g << "extern \"C\" __global__ void " << code.gather << (w32 ? "_32" : "") << "(K k) { CELL_HEAD\n";
+            if (w32) {
+                // A row clear of the y and z edges (the whole wave's, so no lanes part) takes the inner forms: no clamps, no
+                // face conditions, shift_t one read. A law that reads along x alone is clear of them everywhere.
+                std::string clear;
+                for (const auto& [axis, off] : {std::pair<std::string, int>{"y", off_y}, {"z", off_z}}) {
+                    if (off > 0) {
+                        clear += axis + " >= " + std::to_string(off) + " && " + axis + " + " + std::to_string(off) + " < k.n" + axis + " && ";
+                    }
+                }
+                g << "    if (FE_POW2(k)) {\n        if (" << clear << fn << ", true, true>>(k, x, y, z)) return;\n"
+                  << "        " << fn << ", true>>(k, x, y, z);\n    }\n";
+            } else {
+                g << "    if (FE_POW2(k)) " << fn << ", true>>(k, x, y, z);\n";
+            }
+            g << "    else " << fn << ", false>>(k, x, y, z);\n}\n";
+        }
+        out_ << g.str();
         int radius = 0;
         std::vector<int> windowed;
         for (const auto& [f, r] : reach) {
@@ -2048,6 +2205,42 @@ private:
         return bounded;
     }
 
+    // How far along y and z from its cell the gather reads anything (fields, stored stages) through what it inlines.
+    void row_reach(const ir::Program& p, int& out_y, int& out_z) const
+    {
+        std::set<std::tuple<int, int, int>> seen;
+        std::function<void(int, int, int)> walk = [&](int id, int y, int z) {
+            if (!seen.insert({id, y, z}).second) {
+                return;
+            }
+            out_y = std::max(out_y, y);
+            out_z = std::max(out_z, z);
+            if (lay_.stages.count(id) != 0) {
+                return;
+            }
+            const ir::Inst& in = at(id);
+            int ry = in.radius, rz = in.radius;
+            if (in.op == Op::Shift || in.op == Op::ShiftT) {
+                ry = std::abs(in.offset[1]);
+                rz = std::abs(in.offset[2]);
+            } else if (in.op == Op::Gx || in.op == Op::GxT) {
+                ry = rz = 0;
+            } else if (in.op == Op::Gy || in.op == Op::GyT) {
+                rz = 0;
+            } else if (in.op == Op::Gz || in.op == Op::GzT) {
+                ry = 0;
+            }
+            out_y = std::max(out_y, y + ry);
+            out_z = std::max(out_z, z + rz);
+            for (const int a : in.args) {
+                walk(a, y + ry, z + rz);
+            }
+        };
+        for (const ir::Equation& eq : p.equations) {
+            walk(eq.value, 0, 0);
+        }
+    }
+
     // Window gathers: tiles of cells marching in z, the fields read off-cell (`wf`, reach <= R) from an LDS ring of
     // planes. The ring holds planes z-R..z+R and the one being filled (RS >= 2R + 2 slots, a slot a plane, slot of
     // plane p = (p + RS) % RS, in unsigned arithmetic: p >= -R, so p + RS > 0); each plane of each field is loaded once by its tile, rows and halo columns at clamped
@@ -2196,6 +2389,7 @@ private:
         // for planes z-R..z+R (`own`), as the LDS ring holds them. Every other read goes through the ring.
         const int NOWN = 2 * R + 1;
         s << "template <bool P2> struct " << W << " {\n    static constexpr bool kClamps = false;\n    static constexpr bool kExact = false;\n"
+          << "    static constexpr bool kInner = false;\n"
           << "    static constexpr bool kPow2 = P2;\n"
           << "    int x0; int y0; int xc; int yc; int zc; mutable bool bad; double u[" << std::max(1, lay_.uniforms) << "];\n"
           << "    float own[" << NW << "][" << NOWN << "][" << VX << "];\n"
