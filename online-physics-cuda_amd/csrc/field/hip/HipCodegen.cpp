@@ -1700,6 +1700,74 @@ private:
              << "    }\n"
              << "    k.A[(i64)to_in * k.cells + here] = bi; k.A[(i64)to_out * k.cells + here] = bo;\n"
              << "}\n";
+        // The first axis of a lattice whose x lines are at most 512 cells, a row a wave: which cells are in the set as one
+        // 64-bit mask a word, a cell's nearest ones by bit scans of its own word and the last and first ones of the words
+        // beside it. For both sets (the other's mask is the complement).
+        out_ << "extern \"C\" __global__ __launch_bounds__(256) void " << s.kernel << "_rows(K k, const unsigned* w, int to_in, int to_out) {\n"
+             << "    if (w[0] == 0u) return;\n"
+             << "    const i64 line = (i64)blockIdx.x * 4 + (threadIdx.x >> 6);\n"
+             << "    if (line >= (i64)k.ny * k.nz) return;\n"
+             << "    const int lane = (int)(threadIdx.x & 63u);\n"
+             << "    const float* held = k.A + (i64)" << set << " * k.cells + line * k.nx;\n"
+             << "    u64 in[8], valid[8];\n"
+             << "#pragma unroll\n"
+             << "    for (int b = 0; b < 8; ++b) {\n"
+             << "        const int x = 64 * b + lane;\n"
+             << "        in[b] = 0ull; valid[b] = 0ull;\n"
+             << "        if (64 * b < k.nx) { const float v = x < k.nx ? held[x] : 0.0f; in[b] = __ballot(v != 0.0f); valid[b] = __ballot(x < k.nx); }\n"
+             << "    }\n"
+             << "    const float inf = __builtin_inff();\n"
+             << "    for (int out = 0; out < 2; ++out) {\n"
+             << "        float* o = k.A + (i64)(out ? to_out : to_in) * k.cells + line * k.nx;\n"
+             << "        int next = 1 << 20;\n"
+             << "        int after[8];\n" // the first one past word b
+             << "#pragma unroll\n"
+             << "        for (int b = 7; b >= 0; --b) { after[b] = next; const u64 m = out ? valid[b] & ~in[b] : in[b]; if (m != 0ull) next = 64 * b + __ffsll((long long)m) - 1; }\n"
+             << "        int before = -(1 << 20);\n" // the last one ahead of word b
+             << "#pragma unroll\n"
+             << "        for (int b = 0; b < 8; ++b) {\n"
+             << "            if (64 * b >= k.nx) break;\n"
+             << "            const u64 m = out ? valid[b] & ~in[b] : in[b];\n"
+             << "            const int x = 64 * b + lane;\n"
+             << "            const u64 up = m >> lane, down = m << (63 - lane);\n"
+             << "            const int right = up != 0ull ? __ffsll((long long)up) - 1 : after[b] - x, left = down != 0ull ? __clzll((long long)down) : x - before;\n"
+             << "            const int d = right < left ? right : left;\n"
+             << "            if (x < k.nx) o[x] = d < (1 << 15) ? (float)(d * d) : inf;\n"
+             << "            if (m != 0ull) before = 64 * b + 63 - __clzll((long long)m);\n"
+             << "        }\n    }\n}\n";
+        // A y or z line's least f(j) + (q - j)^2 by trying every j: eight q a thread, a line a lane, so a cell of the line
+        // read once serves eight sums. f(j) + j^2 - 2qj, and q^2 added to the least: whole numbers below 2^24, exact. An
+        // eighth of a cell's read and 1.5 instructions a pair against an envelope's serial pushes; which of the two is
+        // faster is a matter of how many cells there are to fill the card with (the launch's rule).
+        out_ << "extern \"C\" __global__ __launch_bounds__(256) void " << s.kernel
+             << "_near(K k, const unsigned* w, int axis, int from_in, int from_out, int to_in, int to_out) {\n"
+             << "    if (w[0] == 0u) return;\n"
+             << "    const int n = axis == 1 ? k.ny : k.nz;\n"
+             << "    const i64 lines = k.cells / n, line = (i64)blockIdx.x * 256 + threadIdx.x;\n"
+             << "    if (line >= lines) return;\n"
+             << "    const i64 step = axis == 1 ? (i64)k.nx : k.nxy;\n"
+             << "    const i64 base = axis == 1 ? (line / k.nx) * k.nxy + line % k.nx : line;\n"
+             << "    const bool out = blockIdx.z != 0u;\n"
+             << "    const float* f = k.A + (i64)(out ? from_out : from_in) * k.cells + base;\n"
+             << "    const int q0 = (int)blockIdx.y * 8;\n"
+             << "    float c[8], best[8];\n"
+             << "#pragma unroll\n"
+             << "    for (int u = 0; u < 8; ++u) { c[u] = (float)(-2 * (q0 + u)); best[u] = __builtin_inff(); }\n"
+             << "    for (int j0 = 0; j0 < n; j0 += 8) {\n"
+             << "        float g[8];\n"
+             << "#pragma unroll\n"
+             << "        for (int v = 0; v < 8; ++v) { const int j = j0 + v < n ? j0 + v : n - 1; g[v] = f[j * step]; }\n"
+             << "#pragma unroll\n"
+             << "        for (int v = 0; v < 8; v += 2) {\n"
+             << "            const int ja = j0 + v < n ? j0 + v : n - 1, jb = j0 + v + 1 < n ? j0 + v + 1 : n - 1;\n"
+             << "            const float fa = (float)ja, fb = (float)jb, ga = g[v] + fa * fa, gb = g[v + 1] + fb * fb;\n"
+             << "#pragma unroll\n"
+             << "            for (int u = 0; u < 8; ++u) best[u] = __builtin_fminf(best[u], __builtin_fminf(__builtin_fmaf(c[u], fa, ga), __builtin_fmaf(c[u], fb, gb)));\n"
+             << "        }\n    }\n"
+             << "    float* o = k.A + (i64)(out ? to_out : to_in) * k.cells + base;\n"
+             << "#pragma unroll\n"
+             << "    for (int u = 0; u < 8; ++u) if (q0 + u < n) o[(q0 + u) * step] = best[u] + (float)((q0 + u) * (q0 + u));\n"
+             << "}\n";
         // The same axis a line a thread: the lower envelope of the parabolas f(j) + (q - j)^2 (Felzenszwalb and
         // Huttenlocher's 1-D transform) built once along the line, then read at every q, in O(n) a line instead of an
         // outward search from every cell (which walks whole lines where a set is far or absent). The comparisons are
@@ -1789,16 +1857,20 @@ private:
         out_ << "extern \"C\" __global__ void " << s.kernel << "_sweep(K k, const unsigned* w, int from, int to) {\n"
              << "    if (w[0] == 0u) return;\n    CELL_HEAD\n"
              << (s.scalar_source ? "    const Direct m(k);\n" : "")
-             << "    const float* phi = k.A + (i64)from * k.cells;\n"
-             << "    const i64 i = IDX(x, y, z);\n"
+             << "    const float* row = k.A + (i64)from * k.cells + ROW(y, z);\n"
+             // Every neighbour read at its clamped coordinate, unconditional (a branch a read would wait for each in
+             // turn); one outside the lattice counts 0, which changes no bit of a sum that starts at +0.
+             << "    const double xl = row[(unsigned)ex(k, x - 1)], xh = row[(unsigned)ex(k, x + 1)];\n"
+             << "    const double yl = (row - (y > 0 ? k.nx : 0))[(unsigned)x], yh = (row + (y + 1 < k.ny ? k.nx : 0))[(unsigned)x];\n"
+             << "    const double zl = (row - (z > 0 ? k.nxy : 0))[(unsigned)x], zh = (row + (z + 1 < k.nz ? k.nxy : 0))[(unsigned)x];\n"
              << "    double sum = 0.0;\n"
-             << "    if (k.nx > 1) { if (x > 0) sum += phi[i - 1]; if (x + 1 < k.nx) sum += phi[i + 1]; }\n"
-             << "    if (k.ny > 1) { if (y > 0) sum += phi[i - k.nx]; if (y + 1 < k.ny) sum += phi[i + k.nx]; }\n"
-             << "    if (k.nz > 1) { if (z > 0) sum += phi[i - k.nxy]; if (z + 1 < k.nz) sum += phi[i + k.nxy]; }\n"
+             << "    sum += x > 0 ? xl : 0.0; sum += x + 1 < k.nx ? xh : 0.0;\n"
+             << "    sum += y > 0 ? yl : 0.0; sum += y + 1 < k.ny ? yh : 0.0;\n"
+             << "    sum += z > 0 ? zl : 0.0; sum += z + 1 < k.nz ? zh : 0.0;\n"
              << "    const int axes = (k.nx > 1 ? 1 : 0) + (k.ny > 1 ? 1 : 0) + (k.nz > 1 ? 1 : 0);\n"
              << "    const double denom = 2.0 * (double)(axes > 1 ? axes : 1);\n"
              << "    const double s = " << (s.scalar_source ? d(src) : "(double)AT(" + std::to_string(slot + 2) + ", x, y, z)") << ";\n"
-             << "    k.A[(i64)to * k.cells + i] = fe_rf((sum - k.h * k.h * s) / denom);\n"
+             << "    AT(to, x, y, z) = fe_rf((sum - k.h * k.h * s) / denom);\n"
              << "}\n";
         out_ << "extern \"C\" __global__ void " << s.kernel << "_copy(K k, unsigned* w, int from) {\n"
              << "    if (w[0] == 0u) return;\n    CELL_HEAD\n"

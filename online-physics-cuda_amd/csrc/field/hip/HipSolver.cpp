@@ -70,6 +70,7 @@ constexpr int kReduceBlocks = 1024; // blocks of a reduction's first pass (its p
 constexpr int kTotals = 1024;      // doubles of conserved totals judged at once
 constexpr int kFillWaves = 2048;    // two waves a SIMD of MI355X: a generic window's launch shortens its z-chunks to reach it
 constexpr int kRanges = 1024;      // range checks judged at once (a record each: two counts and the first bad cell)
+constexpr std::size_t kNearCells = std::size_t{1} << 22; // cells up to which a distance line tries every pair
 constexpr int kMaxWindowRegisters = 168; // a lane's registers that still leave a window gather three waves a SIMD
 
 struct Impl final : HipBackend {
@@ -783,6 +784,25 @@ struct Impl final : HipBackend {
                 // a block's lines fit 64 KB and the squared distances stay below 2^24; the outward search from every
                 // cell otherwise.
                 const int n = axis == 0 ? shape.nx : (axis == 1 ? shape.ny : shape.nz);
+                const long long axis_lines = static_cast<long long>(shape.cells()) / n;
+                if (axis == 0 && n <= 512) {
+                    std::vector<std::uint64_t> k = args(dt);
+                    void* argv[] = {k.data(), &w, &ti, &to};
+                    check(fe_hip_launch(fn(s.kernel + "_rows"), static_cast<unsigned>((axis_lines + 3) / 4), 1, 1, 256, 1, 1, 0, argv),
+                        "distance rows launch");
+                    ++prof.launches;
+                    continue;
+                }
+                // Every pair of a line's cells, while the squared distances stay below 2^24 (three axes of 1024 cells) and
+                // the lattice is small enough that the envelopes' few threads would leave the card idle.
+                if (axis != 0 && n <= 1024 && std::max(shape.nx, shape.ny) <= 1024 && shape.cells() <= kNearCells) {
+                    std::vector<std::uint64_t> k = args(dt);
+                    void* argv[] = {k.data(), &w, &a, &fi, &fo, &ti, &to};
+                    check(fe_hip_launch(fn(s.kernel + "_near"), static_cast<unsigned>((axis_lines + 255) / 256), static_cast<unsigned>((n + 7) / 8), 2,
+                              256, 1, 1, 0, argv), "distance near launch");
+                    ++prof.launches;
+                    continue;
+                }
                 int lines_a_block = 64;
                 while (lines_a_block > 1 && 12LL * lines_a_block * n > 65536) {
                     lines_a_block /= 2;
@@ -790,8 +810,7 @@ struct Impl final : HipBackend {
                 if (n <= 2048 && 12LL * lines_a_block * n <= 65536) {
                     std::vector<std::uint64_t> k = args(dt);
                     void* argv[] = {k.data(), &w, &a, &fi, &fo, &ti, &to};
-                    const long long lines = static_cast<long long>(shape.cells()) / n;
-                    check(fe_hip_launch(fn(s.kernel + "_lines"), static_cast<unsigned>((lines + lines_a_block - 1) / lines_a_block), 1, 1,
+                    check(fe_hip_launch(fn(s.kernel + "_lines"), static_cast<unsigned>((axis_lines + lines_a_block - 1) / lines_a_block), 1, 1,
                               static_cast<unsigned>(2 * lines_a_block), 1, 1, static_cast<unsigned>(12 * lines_a_block * n), argv),
                         "distance lines launch");
                     ++prof.launches;
