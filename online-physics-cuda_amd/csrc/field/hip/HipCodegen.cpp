@@ -66,19 +66,33 @@ __device__ __forceinline__ int clampi(int v, int lo, int hi) { return max(lo, mi
 // a / h, a / h^2, a / (h * span): when the divisor is a power of two (flags, set by the host) the quotient is the exact
 // product with its reciprocal, so the multiply gives the division's bits without the division's cost.
 // M::kPow2: the caller has checked both flags (a kernel instantiated for that case), so no branch is left.
+// Otherwise (flag 4, the spacing within 2^+-200) the quotient comes by Markstein's division with the reciprocal the host
+// rounded: two corrections by the exact remainder give the correctly rounded quotient, five multiply-adds where the
+// hardware's division is eleven instructions with a quarter-rate reciprocal. A remainder that is zero or not finite
+// (an exact quotient, a signed zero, an infinity, NaN) leaves the first product, which is the quotient then.
+__device__ __forceinline__ double div_by(double a, double d, double inv)
+{
+    const double q = a * inv, r = __builtin_fma(-q, d, a);
+    const double p = __builtin_fma(r, inv, q), s = __builtin_fma(-p, d, a), o = __builtin_fma(s, inv, p);
+    return __builtin_amdgcn_class(r, 0x108) ? o : q;
+}
+// M::kAnyH: the spacing may lie outside that range (the launch takes such a kernel then), so the division is there too.
 template <class M> __device__ __forceinline__ double div_h(const K& k, double a)
 {
-    return (M::kPow2 || (k.flags & 1)) ? a * k.inv_h : a / k.h;
+    if (M::kPow2 || (M::kAnyH && (k.flags & 1))) return a * k.inv_h;
+    return !M::kAnyH || (k.flags & 4) ? div_by(a, k.h, k.inv_h) : a / k.h;
 }
 template <class M> __device__ __forceinline__ double div_hh(const K& k, double a)
 {
-    return (M::kPow2 || (k.flags & 2)) ? a * k.inv_hh : a / (k.h * k.h);
+    if (M::kPow2 || (M::kAnyH && (k.flags & 2))) return a * k.inv_hh;
+    return !M::kAnyH || (k.flags & 4) ? div_by(a, k.h * k.h, k.inv_hh) : a / (k.h * k.h);
 }
 // A span of no cells (an axis one cell long) divides a cell's difference with itself: NaN, as 0 / 0 or NaN * inf.
 template <class M> __device__ __forceinline__ double div_hs(const K& k, double a, int span)
 {
-    if (M::kPow2) return a * (span == 2 ? 0.5 * k.inv_h : (span == 1 ? k.inv_h : __builtin_inf()));
-    return (k.flags & 1) && span > 0 ? a * (span == 1 ? k.inv_h : 0.5 * k.inv_h) : a / (k.h * (double)span);
+    const double part = span == 2 ? 0.5 : (span == 1 ? 1.0 : __builtin_inf());
+    if (M::kPow2 || (M::kAnyH && (k.flags & 1))) return a * (part * k.inv_h);
+    return !M::kAnyH || (k.flags & 4) ? div_by(a, k.h, k.inv_h) * part : a / (k.h * (double)span);
 }
 // The same quotients of a float, rounded to float: by a power of two both the double product and the float one are exact
 // (or overflow, or flush, alike), so the float product serves. The host sets the flags only where the reciprocals are
@@ -463,6 +477,7 @@ public:
         // waited for, would drain the loads in flight).
         out_ << "struct Direct {\n    static constexpr bool kClamps = true;\n    static constexpr bool kExact = true;\n"
              << "    static constexpr bool kPow2 = false;\n    static constexpr bool kInner = false;\n    static constexpr bool bad = false;\n"
+             << "    static constexpr bool kAnyH = true;\n"
              << "    __device__ void flag(bool) const {}\n    double u[" << nu << "];\n"
              << "    __device__ explicit Direct(const K& k) { for (int q = 0; q < " << nu << "; ++q) u[q] = " << (lay_.uniforms > 0 ? "k.U[q]" : "0.0")
              << "; }\n"
@@ -475,7 +490,7 @@ public:
              // row away from the lattice's y and z edges (M::kInner), in the fast forms (a cell they flag is taken again
              // in the exact ones).
              << "template <bool W32, bool P2, bool IN = false> struct DirectT : Direct {\n    static constexpr bool kPow2 = P2;\n"
-             << "    static constexpr bool kInner = IN;\n    static constexpr bool kExact = !IN;\n    mutable bool bad = false;\n"
+             << "    static constexpr bool kInner = IN;\n    static constexpr bool kExact = !IN;\n    static constexpr bool kAnyH = !W32;\n    mutable bool bad = false;\n"
              << "    __device__ __forceinline__ void flag(bool b) const { if (IN) bad = bad || b; }\n"
              << "    __device__ explicit DirectT(const K& k) : Direct(k) {}\n"
              << "    template <int F> __device__ __forceinline__ float fld(const K& k, int x, int y, int z) const\n"
@@ -2005,6 +2020,7 @@ private:
             const int kk = conduction_form(p);
             if (kk >= 0 && code.window) {
                 flux_kernels(code, cellfn, p.equations[0].target, kk);
+                row_flux_kernels(code, p.equations[0].target, kk);
             }
         }
         return code;
@@ -2029,14 +2045,14 @@ private:
         return in.args[0];
     }
 
-    // The window of a conduction term, carrying its face fluxes. Tiles of 256 x TY cells march in z, a lane four
-    // consecutive cells of a row (float4 loads and stores; nx a multiple of 4); plane z's x and y neighbours from a
+    // The window of a conduction term, carrying its face fluxes, for rows of one tile. Tiles of 256 x TY cells march in z, a
+    // lane four consecutive cells of a row (16-byte loads and stores; nx a multiple of 4); plane z's x and y neighbours from a
     // double-buffered LDS tile (one barrier a plane), its z neighbours from a four-slot register ring loaded three
-    // planes ahead. Two ways to bring the tile's halo rows: form A (`_f4_`), two more waves that only load them (the
-    // compute waves' loads stay one row each: the better form once the lattice streams from HBM); form B (`_h4_`),
-    // the tile's first and last row waves load them beside their own row, the others their own row twice (no idle
-    // waves, so more compute waves a CU: the better form while the lattice sits in the last-level cache; measured on
-    // MI355X at 256^3: 27.2 us against 30.6, at 512^3: 265 against 243).
+    // planes ahead. The tile's first and last row waves load its halo rows beside their own row, the others their own row
+    // twice (two more waves that only load them measured slower: 256^3 29.4-36.4 us against 27.2). Its quads are vectors of
+    // the compiler's own: in structs of the HIP header's one of its releases kept a plane in private memory. The form for rows of
+    // whole quads that fill a tile while the lattice sits in the last-level cache: at 256^3 27.9 us against 28.2-28.9
+    // for row_flux_kernels' form, which wins past it (512 x 512 x 128: 49.9-52 us against 69).
     // The CPU's face sum, in its order (-x, +x, -y, +y, -z, +z; src/field/Law.cpp:986-1018), from fluxes computed once
     // where IEEE arithmetic makes the share exact: kf * (a - b) is -(kf * (b - a)) to the bit, so the flux a cell sends
     // through its +x face is the one its right neighbour receives, and the flux through its +z face is carried into
@@ -2052,194 +2068,326 @@ private:
     {
         const std::vector<int> targets{target};
         const std::string t = std::to_string(target);
-        struct Form {
-            bool rows; // form B: halo rows loaded by the edge row waves
-            int ty;
-            int zchunk;
-        };
-        for (const Form form : {Form{false, 4, 32}, Form{false, 6, 32}, Form{true, 8, 16}}) {
-            const int TY = form.ty;
-            const int WAVES = form.rows ? TY : TY + 2;
-            const std::string name = code.gather + (form.rows ? "_h4_" : "_f4_") + std::to_string(TY);
-            const std::string LDS = "L_" + name;
-            const std::string MK = "M_" + name;
-            std::ostringstream s;
-            s << "template <bool P2> struct " << MK << " { static constexpr bool kPow2 = P2; };\n"
-              << "__shared__ __attribute__((aligned(16))) float " << LDS << "[" << 2 * (TY + 2) * 264 << "];\n"
-              << "template <bool P2, bool XH, bool TOTAL> __device__ __forceinline__ void run_" << name
-              << "(const K& k, int zchunk, int tiles_x, int tiles_y, int tiles_z, const bool TRACK, const bool REMAP, const bool STREAM,\n"
-              << "    double* tsum, unsigned* rec, u64* first, double lo_r, double hi_r) {\n"
-              << "    const int tl = REMAP ? xcd_tile((int)blockIdx.x, tiles_x * tiles_y * tiles_z) : (int)blockIdx.x;\n"
-              << "    const int lane = (int)threadIdx.x; const int r = (int)threadIdx.y;\n"
-              << "    const int x = (tl % tiles_x) * 256 + 4 * lane;\n"
-              << "    const int y0 = ((tl / tiles_x) % tiles_y) * " << TY << ";\n";
-            if (form.rows) {
-                s << "    const int y = y0 + r; const int slot = r + 1;\n"
-                  << "    const bool live = x < k.nx && y < k.ny;\n";
-            } else {
-                s << "    const int y = y0 + r - 1; const int slot = r;\n"
-                  << "    const bool live = x < k.nx && r >= 1 && r <= " << TY << " && y < k.ny;\n";
+        const int TY = 8, WAVES = TY;
+        const std::string name = code.gather + "_h4_" + std::to_string(TY);
+        const std::string LDS = "L_" + name;
+        const std::string MK = "M_" + name;
+        std::ostringstream s;
+        s << "template <bool P2> struct " << MK << " { static constexpr bool kPow2 = P2; static constexpr bool kAnyH = false; };\n"
+          << "__shared__ __attribute__((aligned(16))) float " << LDS << "[" << 2 * (TY + 2) * 264 << "];\n"
+          << "template <bool P2, bool TOTAL> __device__ __forceinline__ void run_" << name
+          << "(const K& k, int zchunk, int tiles_x, int tiles_y, int tiles_z, const bool TRACK, const bool REMAP, const bool STREAM,\n"
+          << "    double* tsum, unsigned* rec, u64* first, double lo_r, double hi_r) {\n"
+          << "    const int tl = REMAP ? xcd_tile((int)blockIdx.x, tiles_x * tiles_y * tiles_z) : (int)blockIdx.x;\n"
+          << "    const int lane = (int)threadIdx.x; const int r = (int)threadIdx.y;\n"
+          << "    const int x = (tl % tiles_x) * 256 + 4 * lane;\n"
+          << "    const int y0 = ((tl / tiles_x) % tiles_y) * " << TY << ";\n";
+        s << "    const int y = y0 + r; const int slot = r + 1;\n"
+          << "    const bool live = x < k.nx && y < k.ny;\n";
+        s << "    const int z0 = (tl / (tiles_x * tiles_y)) * zchunk; const int z1 = z0 + zchunk < k.nz ? z0 + zchunk : k.nz;\n"
+          << "    const int xs = x < k.nx - 4 ? x : k.nx - 4;\n"
+          << "    const int ys = clampi(y, 0, k.ny - 1);\n"
+          << "    const float* base = k.now[" << t << "] + (i64)ys * k.nx + xs;\n"
+          << "    float* outp = k.nxt[" << t << "] + (i64)ys * k.nx + xs;\n";
+        // the row above the tile (wave 0) or below it (the last wave); the others their own row again
+        s << "    const int hy = r == 0 ? clampi(y0 - 1, 0, k.ny - 1) : (r == " << TY - 1 << " ? clampi(y0 + " << TY
+          << ", 0, k.ny - 1) : ys);\n"
+          << "    const int hslot = r == 0 ? 0 : (r == " << TY - 1 << " ? " << TY + 1 << " : -1);\n"
+          << "    const float* hbase = k.now[" << t << "] + (i64)hy * k.nx + xs;\n";
+        s << "    const int zlim = z1 < k.nz - 1 ? z1 : k.nz - 1;\n"
+          << "    const Direct md(k);\n"
+          << "    const double kv = s" << kk << "(k, md);\n"
+          << "    const double kf = (kv + kv) > 0.0 ? 2.0 * kv * kv / (kv + kv) : 0.0;\n"
+          << "    float* const tile = " << LDS << ";\n";
+        // Every load unconditional, from a clamped plane (past the top, the plane itself: the zero-flux edge).
+        s << "    struct Pl { f4v v; f4v h; };\n"
+          << "    auto load = [&](Pl& p, int zp) __attribute__((always_inline)) { const i64 o = (i64)(zp < zlim ? zp : zlim) * k.nxy;\n"
+          << "        const float* q = base + o; const float* qh = hbase + o;\n"
+          << "        p.v = *reinterpret_cast<const f4v*>(q); p.h = *reinterpret_cast<const f4v*>(qh); };\n";
+        s << "    Pl A, B, C, D;\n"
+          << "    load(A, z0); __builtin_amdgcn_sched_barrier(0); load(B, z0 + 1); __builtin_amdgcn_sched_barrier(0);\n"
+          << "    load(C, z0 + 2); __builtin_amdgcn_sched_barrier(0);\n"
+          << "    const f4v lo = *reinterpret_cast<const f4v*>(base + (i64)(z0 > 0 ? z0 - 1 : 0) * k.nxy);\n"
+          << "    double c0 = (double)A.v.x, c1 = (double)A.v.y, c2 = (double)A.v.z, c3 = (double)A.v.w;\n"
+          << "    double fzm0 = kf * ((double)lo.x - c0), fzm1 = kf * ((double)lo.y - c1), fzm2 = kf * ((double)lo.z - c2),\n"
+          << "           fzm3 = kf * ((double)lo.w - c3);\n"
+          << "    int buf = 0;\n"
+          << "    bool seen[1] = {false};\n"
+          << "    double ts = 0.0, tm = 0.0; unsigned nout = 0, nbad = 0; u64 firstbad = ~0ull;\n"
+          << "    auto step = [&](const int z, const Pl& cur, const Pl& nxt, Pl& far) __attribute__((always_inline)) {\n"
+          << "        load(far, z + 3);\n"
+          << "        const f4v c = cur.v;\n"
+          << "        float* const plane = tile + buf * " << (TY + 2) * 264 << ";\n"
+          << "        float* const row = plane + slot * 264;\n"
+          << "        *reinterpret_cast<f4v*>(row + 4 + 4 * lane) = c;\n"
+          << "        if (hslot >= 0) { float* const hrow = plane + hslot * 264; *reinterpret_cast<f4v*>(hrow + 4 + 4 * lane) = cur.h; }\n"
+          << "        __syncthreads();\n"
+          << "        const f4v hi = nxt.v;\n"
+          << "        const double d0 = (double)hi.x, d1 = (double)hi.y, d2 = (double)hi.z, d3 = (double)hi.w;\n"
+          << "        if (live) {\n"
+          // values first, then the edge selects (a select between an LDS lvalue and a register takes addresses)
+          << "            const f4v ym = *reinterpret_cast<const f4v*>(row - 264 + 4 + 4 * lane);\n"
+          << "            const f4v yp = *reinterpret_cast<const f4v*>(row + 264 + 4 + 4 * lane);\n"
+          << "            const float txm = row[3 + 4 * lane]; const float txp = row[8 + 4 * lane];\n"
+          << "            const float xme = x > 0 ? txm : c.x; const float xpe = x + 4 < k.nx ? txp : c.w;\n"
+          << "            const double fxm = kf * ((double)xme - c0), f01 = kf * (c1 - c0), f12 = kf * (c2 - c1), f23 = kf * (c3 - c2),\n"
+          << "                         fxp = kf * ((double)xpe - c3);\n"
+          << "            const double fzp0 = kf * (d0 - c0), fzp1 = kf * (d1 - c1), fzp2 = kf * (d2 - c2), fzp3 = kf * (d3 - c3);\n"
+          << "            double q0 = 0.0 + fxm; q0 += f01; q0 += kf * ((double)ym.x - c0); q0 += kf * ((double)yp.x - c0); q0 += fzm0; q0 += fzp0;\n"
+          << "            double q1 = 0.0 + (-f01); q1 += f12; q1 += kf * ((double)ym.y - c1); q1 += kf * ((double)yp.y - c1); q1 += fzm1; q1 += fzp1;\n"
+          << "            double q2 = 0.0 + (-f12); q2 += f23; q2 += kf * ((double)ym.z - c2); q2 += kf * ((double)yp.z - c2); q2 += fzm2; q2 += fzp2;\n"
+          << "            double q3 = 0.0 + (-f23); q3 += fxp; q3 += kf * ((double)ym.w - c3); q3 += kf * ((double)yp.w - c3); q3 += fzm3; q3 += fzp3;\n"
+          << "            if (q0 != q0 || q1 != q1 || q2 != q2 || q3 != q3) {\n"
+          // An infinity or NaN among the inputs: the faces the cells have, in the CPU's order, from the plane still
+          // in LDS (nothing extra kept in registers for this rare path but the incoming -z fluxes).
+          << "                const bool xl = x > 0, xr = x + 4 < k.nx, yl = y > 0, yr = y + 1 < k.ny, zl = z > 0, zr = z + 1 < k.nz;\n"
+          << "                const f4v ya = *reinterpret_cast<const f4v*>(row - 264 + 4 + 4 * lane);\n"
+          << "                const f4v yb = *reinterpret_cast<const f4v*>(row + 264 + 4 + 4 * lane);\n"
+          << "                const double gm = kf * ((double)row[3 + 4 * lane] - c0), gp = kf * ((double)row[8 + 4 * lane] - c3);\n"
+          << "                const double g01 = kf * (c1 - c0), g12 = kf * (c2 - c1), g23 = kf * (c3 - c2);\n"
+          << "                q0 = 0.0; if (xl) q0 += gm; q0 += g01; if (yl) q0 += kf * ((double)ya.x - c0); if (yr) q0 += kf * ((double)yb.x - c0);\n"
+          << "                if (zl) q0 += fzm0; if (zr) q0 += kf * (d0 - c0);\n"
+          << "                q1 = 0.0; q1 += -g01; q1 += g12; if (yl) q1 += kf * ((double)ya.y - c1); if (yr) q1 += kf * ((double)yb.y - c1);\n"
+          << "                if (zl) q1 += fzm1; if (zr) q1 += kf * (d1 - c1);\n"
+          << "                q2 = 0.0; q2 += -g12; q2 += g23; if (yl) q2 += kf * ((double)ya.z - c2); if (yr) q2 += kf * ((double)yb.z - c2);\n"
+          << "                if (zl) q2 += fzm2; if (zr) q2 += kf * (d2 - c2);\n"
+          << "                q3 = 0.0; q3 += -g23; if (xr) q3 += gp; if (yl) q3 += kf * ((double)ya.w - c3); if (yr) q3 += kf * ((double)yb.w - c3);\n"
+          << "                if (zl) q3 += fzm3; if (zr) q3 += kf * (d3 - c3);\n"
+          << "            }\n"
+          << "            q0 = div_hh<" << MK << "<P2>>(k, q0); q1 = div_hh<" << MK << "<P2>>(k, q1);\n"
+          << "            q2 = div_hh<" << MK << "<P2>>(k, q2); q3 = div_hh<" << MK << "<P2>>(k, q3);\n"
+          << "            const f4v nv = {fe_ftz(c.x + fe_rf((double)fe_rf(q0) * k.dt)), fe_ftz(c.y + fe_rf((double)fe_rf(q1) * k.dt)),\n"
+          << "                            fe_ftz(c.z + fe_rf((double)fe_rf(q2) * k.dt)), fe_ftz(c.w + fe_rf((double)fe_rf(q3) * k.dt))};\n"
+          << "            f4v* dst = reinterpret_cast<f4v*>(outp + (i64)z * k.nxy);\n"
+          << "            if (STREAM) { asm volatile(\"\"); __builtin_nontemporal_store(nv, dst); asm volatile(\"\"); } else *dst = nv;\n"
+          << "            if (TRACK) { asm volatile(\"\");\n"
+          << "                const bool ch = __float_as_uint(nv.x) != __float_as_uint(c.x) || __float_as_uint(nv.y) != __float_as_uint(c.y) ||\n"
+          << "                    __float_as_uint(nv.z) != __float_as_uint(c.z) || __float_as_uint(nv.w) != __float_as_uint(c.w);\n"
+          << "                seen[0] = seen[0] || ch; }\n"
+          << "            if (TOTAL) {\n"
+          << "                const double v0 = (double)nv.x, v1 = (double)nv.y, v2 = (double)nv.z, v3 = (double)nv.w;\n"
+          << "                ts += v0; tm += fabs(v0); ts += v1; tm += fabs(v1); ts += v2; tm += fabs(v2); ts += v3; tm += fabs(v3);\n"
+          // out of range or not finite (the rare path: counted, and the least index kept)
+          << "                const bool b0 = !(v0 >= lo_r && v0 <= hi_r), b1 = !(v1 >= lo_r && v1 <= hi_r), b2 = !(v2 >= lo_r && v2 <= hi_r),\n"
+          << "                           b3 = !(v3 >= lo_r && v3 <= hi_r);\n"
+          << "                if (b0 || b1 || b2 || b3) {\n"
+          << "                    const double vs[4] = {v0, v1, v2, v3};\n"
+          << "                    const bool bs[4] = {b0, b1, b2, b3};\n"
+          << "#pragma unroll\n"
+          << "                    for (int q = 0; q < 4; ++q) {\n"
+          << "                        if (!bs[q]) continue;\n"
+          << "                        if (finite_d(vs[q])) ++nout; else ++nbad;\n"
+          << "                        const u64 i = (u64)z * (u64)k.nxy + (u64)y * (u64)k.nx + (u64)(x + q); firstbad = i < firstbad ? i : firstbad; } } }\n"
+          << "            fzm0 = -fzp0; fzm1 = -fzp1; fzm2 = -fzp2; fzm3 = -fzp3;\n"
+          << "        }\n"
+          << "        buf ^= 1; c0 = d0; c1 = d1; c2 = d2; c3 = d3;\n"
+          << "    };\n"
+          // Whole groups of four planes, then the rest (a break inside the group would make the compiler wait for
+          // nearly every load in flight at the loop's head).
+          << "    int z = z0;\n"
+          << "    for (; z + 4 <= z1; z += 4) { step(z, A, B, D); step(z + 1, B, C, A); step(z + 2, C, D, B); step(z + 3, D, A, C); }\n"
+          << "    if (z < z1) { step(z, A, B, D); if (z + 1 < z1) { step(z + 1, B, C, A); if (z + 2 < z1) step(z + 2, C, D, B); } }\n"
+          << "    if (TRACK) mark(k, " << t << ", seen[0]);\n"
+          << "    if (TOTAL) {\n"
+          << "        if (nout) atomicAdd(rec, nout);\n"
+          << "        if (nbad) atomicAdd(rec + 1, nbad);\n"
+          << "        if (firstbad != ~0ull) atomicMin(first, firstbad);\n"
+          << "        __shared__ double wv[" << WAVES << "][4];\n"
+          << "        Sum ps = {ts, 0.0}, pm = {tm, 0.0};\n"
+          << "        wave_fold(ps); wave_fold(pm);\n"
+          << "        if (lane == 0) { wv[r][0] = ps.s; wv[r][1] = ps.c; wv[r][2] = pm.s; wv[r][3] = pm.c; }\n"
+          << "        __syncthreads();\n"
+          << "        if (lane == 0 && r == 0) {\n"
+          << "            Sum a = {wv[0][0], wv[0][1]}, b = {wv[0][2], wv[0][3]};\n"
+          << "            for (int q = 1; q < " << WAVES << "; ++q) { merge(a, Sum{wv[q][0], wv[q][1]}); merge(b, Sum{wv[q][2], wv[q][3]}); }\n"
+          << "            tsum[2 * tl] = a.s + a.c; tsum[2 * tl + 1] = b.s + b.c; } }\n"
+          << "}\n";
+        // The step, and the step that also takes the contract's totals (name + "_t").
+        for (const bool total : {false, true}) {
+            s << "extern \"C\" __global__ __launch_bounds__(" << 64 * WAVES << ")" << (total ? " __attribute__((amdgpu_waves_per_eu(4)))" : "") << " void " << name << (total ? "_t" : "")
+              << "(K k, int zchunk, int tiles_x, int tiles_y, int tiles_z, int mode, double* tsum, unsigned* rec, u64* first, double lo,\n"
+              << "    double hi) {\n"
+              << "    const bool tr = (mode & 1) != 0, rm = (mode & 2) != 0, st = (mode & 4) != 0;\n";
+            for (const bool p2 : {true, false}) {
+                s << "    " << (p2 ? "if ((k.flags & 3) == 3) " : "else ") << "run_" << name << "<" << (p2 ? "true" : "false") << ", "
+                  << (total ? "true" : "false") << ">(k, zchunk, tiles_x, tiles_y, tiles_z, tr, rm, st, tsum, rec, first, lo, hi);\n";
             }
-            s << "    const int z0 = (tl / (tiles_x * tiles_y)) * zchunk; const int z1 = z0 + zchunk < k.nz ? z0 + zchunk : k.nz;\n"
-              << "    const int xs = x < k.nx - 4 ? x : k.nx - 4;\n"
-              << "    const int ys = clampi(y, 0, k.ny - 1);\n"
-              << "    const float* base = k.now[" << t << "] + (i64)ys * k.nx + xs;\n"
-              << "    float* outp = k.nxt[" << t << "] + (i64)ys * k.nx + xs;\n";
-            if (form.rows) {
-                // the row above the tile (wave 0) or below it (the last wave); the others their own row again
-                s << "    const int hy = r == 0 ? clampi(y0 - 1, 0, k.ny - 1) : (r == " << TY - 1 << " ? clampi(y0 + " << TY
-                  << ", 0, k.ny - 1) : ys);\n"
-                  << "    const int hslot = r == 0 ? 0 : (r == " << TY - 1 << " ? " << TY + 1 << " : -1);\n"
-                  << "    const float* hbase = k.now[" << t << "] + (i64)hy * k.nx + xs;\n";
-            }
-            s << "    const int zlim = z1 < k.nz - 1 ? z1 : k.nz - 1;\n"
-              << "    const int lofs = XH && lane == 0 && xs > 0 ? -1 : 0;\n"
-              << "    const int rofs = XH && lane == 63 && xs + 4 < k.nx ? 4 : 0;\n"
-              << "    const Direct md(k);\n"
-              << "    const double kv = s" << kk << "(k, md);\n"
-              << "    const double kf = (kv + kv) > 0.0 ? 2.0 * kv * kv / (kv + kv) : 0.0;\n"
-              << "    float* const tile = " << LDS << ";\n";
-            // Every load unconditional, from a clamped plane (past the top, the plane itself: the zero-flux edge).
-            if (form.rows) {
-                s << "    struct Pl { float4 v; float4 h; float l; float rr; float hl; float hr; };\n"
-                  << "    auto load = [&](Pl& p, int zp) { const i64 o = (i64)(zp < zlim ? zp : zlim) * k.nxy;\n"
-                  << "        const float* q = base + o; const float* qh = hbase + o;\n"
-                  << "        p.v = *reinterpret_cast<const float4*>(q); p.h = *reinterpret_cast<const float4*>(qh);\n"
-                  << "        if (XH) { p.l = q[lofs]; p.rr = q[rofs]; p.hl = qh[lofs]; p.hr = qh[rofs]; } };\n";
-            } else {
-                s << "    struct Pl { float4 v; float l; float rr; };\n"
-                  << "    auto load = [&](Pl& p, int zp) { const float* q = base + (i64)(zp < zlim ? zp : zlim) * k.nxy;\n"
-                  << "        p.v = *reinterpret_cast<const float4*>(q); if (XH) { p.l = q[lofs]; p.rr = q[rofs]; } };\n";
-            }
-            s << "    Pl A, B, C, D;\n"
-              << "    load(A, z0); __builtin_amdgcn_sched_barrier(0); load(B, z0 + 1); __builtin_amdgcn_sched_barrier(0);\n"
-              << "    load(C, z0 + 2); __builtin_amdgcn_sched_barrier(0);\n"
-              << "    const float4 lo = *reinterpret_cast<const float4*>(base + (i64)(z0 > 0 ? z0 - 1 : 0) * k.nxy);\n"
-              << "    double c0 = (double)A.v.x, c1 = (double)A.v.y, c2 = (double)A.v.z, c3 = (double)A.v.w;\n"
-              << "    double fzm0 = kf * ((double)lo.x - c0), fzm1 = kf * ((double)lo.y - c1), fzm2 = kf * ((double)lo.z - c2),\n"
-              << "           fzm3 = kf * ((double)lo.w - c3);\n"
-              << "    int buf = 0;\n"
-              << "    bool seen[1] = {false};\n"
-              << "    double ts = 0.0, tm = 0.0; unsigned nout = 0, nbad = 0; u64 firstbad = ~0ull;\n"
-              << "    auto step = [&](const int z, const Pl& cur, const Pl& nxt, Pl& far) {\n"
-              << "        load(far, z + 3);\n"
-              << "        const float4 c = cur.v;\n"
-              << "        float* const plane = tile + buf * " << (TY + 2) * 264 << ";\n"
-              << "        float* const row = plane + slot * 264;\n"
-              << "        *reinterpret_cast<float4*>(row + 4 + 4 * lane) = c;\n"
-              << "        if (XH) { if (lane == 0) row[3] = cur.l; if (lane == 63) row[260] = cur.rr; }\n";
-            if (form.rows) {
-                s << "        if (hslot >= 0) { float* const hrow = plane + hslot * 264; *reinterpret_cast<float4*>(hrow + 4 + 4 * lane) = cur.h;\n"
-                  << "            if (XH) { if (lane == 0) hrow[3] = cur.hl; if (lane == 63) hrow[260] = cur.hr; } }\n";
-            }
-            s << "        __syncthreads();\n"
-              << "        const float4 hi = nxt.v;\n"
-              << "        const double d0 = (double)hi.x, d1 = (double)hi.y, d2 = (double)hi.z, d3 = (double)hi.w;\n"
-              << "        if (live) {\n"
-              // values first, then the edge selects (a select between an LDS lvalue and a register takes addresses)
-              << "            const float4 ym = *reinterpret_cast<const float4*>(row - 264 + 4 + 4 * lane);\n"
-              << "            const float4 yp = *reinterpret_cast<const float4*>(row + 264 + 4 + 4 * lane);\n"
-              << "            const float txm = row[3 + 4 * lane]; const float txp = row[8 + 4 * lane];\n"
-              << "            const float xme = x > 0 ? txm : c.x; const float xpe = x + 4 < k.nx ? txp : c.w;\n"
-              << "            const double fxm = kf * ((double)xme - c0), f01 = kf * (c1 - c0), f12 = kf * (c2 - c1), f23 = kf * (c3 - c2),\n"
-              << "                         fxp = kf * ((double)xpe - c3);\n"
-              << "            const double fzp0 = kf * (d0 - c0), fzp1 = kf * (d1 - c1), fzp2 = kf * (d2 - c2), fzp3 = kf * (d3 - c3);\n"
-              << "            double q0 = 0.0 + fxm; q0 += f01; q0 += kf * ((double)ym.x - c0); q0 += kf * ((double)yp.x - c0); q0 += fzm0; q0 += fzp0;\n"
-              << "            double q1 = 0.0 + (-f01); q1 += f12; q1 += kf * ((double)ym.y - c1); q1 += kf * ((double)yp.y - c1); q1 += fzm1; q1 += fzp1;\n"
-              << "            double q2 = 0.0 + (-f12); q2 += f23; q2 += kf * ((double)ym.z - c2); q2 += kf * ((double)yp.z - c2); q2 += fzm2; q2 += fzp2;\n"
-              << "            double q3 = 0.0 + (-f23); q3 += fxp; q3 += kf * ((double)ym.w - c3); q3 += kf * ((double)yp.w - c3); q3 += fzm3; q3 += fzp3;\n"
-              << "            if (q0 != q0 || q1 != q1 || q2 != q2 || q3 != q3) {\n"
-              // An infinity or NaN among the inputs: the faces the cells have, in the CPU's order, from the plane still
-              // in LDS (nothing extra kept in registers for this rare path but the incoming -z fluxes).
-              << "                const bool xl = x > 0, xr = x + 4 < k.nx, yl = y > 0, yr = y + 1 < k.ny, zl = z > 0, zr = z + 1 < k.nz;\n"
-              << "                const float4 ya = *reinterpret_cast<const float4*>(row - 264 + 4 + 4 * lane);\n"
-              << "                const float4 yb = *reinterpret_cast<const float4*>(row + 264 + 4 + 4 * lane);\n"
-              << "                const double gm = kf * ((double)row[3 + 4 * lane] - c0), gp = kf * ((double)row[8 + 4 * lane] - c3);\n"
-              << "                const double g01 = kf * (c1 - c0), g12 = kf * (c2 - c1), g23 = kf * (c3 - c2);\n"
-              << "                q0 = 0.0; if (xl) q0 += gm; q0 += g01; if (yl) q0 += kf * ((double)ya.x - c0); if (yr) q0 += kf * ((double)yb.x - c0);\n"
-              << "                if (zl) q0 += fzm0; if (zr) q0 += kf * (d0 - c0);\n"
-              << "                q1 = 0.0; q1 += -g01; q1 += g12; if (yl) q1 += kf * ((double)ya.y - c1); if (yr) q1 += kf * ((double)yb.y - c1);\n"
-              << "                if (zl) q1 += fzm1; if (zr) q1 += kf * (d1 - c1);\n"
-              << "                q2 = 0.0; q2 += -g12; q2 += g23; if (yl) q2 += kf * ((double)ya.z - c2); if (yr) q2 += kf * ((double)yb.z - c2);\n"
-              << "                if (zl) q2 += fzm2; if (zr) q2 += kf * (d2 - c2);\n"
-              << "                q3 = 0.0; q3 += -g23; if (xr) q3 += gp; if (yl) q3 += kf * ((double)ya.w - c3); if (yr) q3 += kf * ((double)yb.w - c3);\n"
-              << "                if (zl) q3 += fzm3; if (zr) q3 += kf * (d3 - c3);\n"
-              << "            }\n"
-              << "            q0 = div_hh<" << MK << "<P2>>(k, q0); q1 = div_hh<" << MK << "<P2>>(k, q1);\n"
-              << "            q2 = div_hh<" << MK << "<P2>>(k, q2); q3 = div_hh<" << MK << "<P2>>(k, q3);\n"
-              << "            const f4v nv = {fe_ftz(c.x + fe_rf((double)fe_rf(q0) * k.dt)), fe_ftz(c.y + fe_rf((double)fe_rf(q1) * k.dt)),\n"
-              << "                            fe_ftz(c.z + fe_rf((double)fe_rf(q2) * k.dt)), fe_ftz(c.w + fe_rf((double)fe_rf(q3) * k.dt))};\n"
-              << "            f4v* dst = reinterpret_cast<f4v*>(outp + (i64)z * k.nxy);\n"
-              << "            if (STREAM) { asm volatile(\"\"); __builtin_nontemporal_store(nv, dst); asm volatile(\"\"); } else *dst = nv;\n"
-              << "            if (TRACK) { asm volatile(\"\");\n"
-              << "                const bool ch = __float_as_uint(nv.x) != __float_as_uint(c.x) || __float_as_uint(nv.y) != __float_as_uint(c.y) ||\n"
-              << "                    __float_as_uint(nv.z) != __float_as_uint(c.z) || __float_as_uint(nv.w) != __float_as_uint(c.w);\n"
-              << "                seen[0] = seen[0] || ch; }\n"
-              << "            if (TOTAL) {\n"
-              << "                const double v0 = (double)nv.x, v1 = (double)nv.y, v2 = (double)nv.z, v3 = (double)nv.w;\n"
-              << "                ts += v0; tm += fabs(v0); ts += v1; tm += fabs(v1); ts += v2; tm += fabs(v2); ts += v3; tm += fabs(v3);\n"
-              // out of range or not finite (the rare path: counted, and the least index kept)
-              << "                const bool b0 = !(v0 >= lo_r && v0 <= hi_r), b1 = !(v1 >= lo_r && v1 <= hi_r), b2 = !(v2 >= lo_r && v2 <= hi_r),\n"
-              << "                           b3 = !(v3 >= lo_r && v3 <= hi_r);\n"
-              << "                if (b0 || b1 || b2 || b3) {\n"
-              << "                    const double vs[4] = {v0, v1, v2, v3};\n"
-              << "                    const bool bs[4] = {b0, b1, b2, b3};\n"
-              << "#pragma unroll\n"
-              << "                    for (int q = 0; q < 4; ++q) {\n"
-              << "                        if (!bs[q]) continue;\n"
-              << "                        if (finite_d(vs[q])) ++nout; else ++nbad;\n"
-              << "                        const u64 i = (u64)z * (u64)k.nxy + (u64)y * (u64)k.nx + (u64)(x + q); firstbad = i < firstbad ? i : firstbad; } } }\n"
-              << "            fzm0 = -fzp0; fzm1 = -fzp1; fzm2 = -fzp2; fzm3 = -fzp3;\n"
-              << "        }\n"
-              << "        buf ^= 1; c0 = d0; c1 = d1; c2 = d2; c3 = d3;\n"
-              << "    };\n"
-              // Whole groups of four planes, then the rest (a break inside the group would make the compiler wait for
-              // nearly every load in flight at the loop's head).
-              << "    int z = z0;\n"
-              << "    for (; z + 4 <= z1; z += 4) { step(z, A, B, D); step(z + 1, B, C, A); step(z + 2, C, D, B); step(z + 3, D, A, C); }\n"
-              << "    if (z < z1) { step(z, A, B, D); if (z + 1 < z1) { step(z + 1, B, C, A); if (z + 2 < z1) step(z + 2, C, D, B); } }\n"
-              << "    if (TRACK) mark(k, " << t << ", seen[0]);\n"
-              << "    if (TOTAL) {\n"
-              << "        if (nout) atomicAdd(rec, nout);\n"
-              << "        if (nbad) atomicAdd(rec + 1, nbad);\n"
-              << "        if (firstbad != ~0ull) atomicMin(first, firstbad);\n"
-              << "        __shared__ double wv[" << WAVES << "][4];\n"
-              << "        Sum ps = {ts, 0.0}, pm = {tm, 0.0};\n"
-              << "        wave_fold(ps); wave_fold(pm);\n"
-              << "        if (lane == 0) { wv[r][0] = ps.s; wv[r][1] = ps.c; wv[r][2] = pm.s; wv[r][3] = pm.c; }\n"
-              << "        __syncthreads();\n"
-              << "        if (lane == 0 && r == 0) {\n"
-              << "            Sum a = {wv[0][0], wv[0][1]}, b = {wv[0][2], wv[0][3]};\n"
-              << "            for (int q = 1; q < " << WAVES << "; ++q) { merge(a, Sum{wv[q][0], wv[q][1]}); merge(b, Sum{wv[q][2], wv[q][3]}); }\n"
-              << "            tsum[2 * tl] = a.s + a.c; tsum[2 * tl + 1] = b.s + b.c; } }\n"
-              << "}\n";
-            // Four kernels: rows within one tile or spanning several (the second loads halo columns, which costs
-            // registers the first should not pay for: name + "x"), each as the step and as the step that also takes
-            // the contract's totals (name + "_t").
-            for (const bool xh : {false, true}) {
-                for (const bool total : {false, true}) {
-                    s << "extern \"C\" __global__ __launch_bounds__(" << 64 * WAVES << ")" << (total ? " __attribute__((amdgpu_waves_per_eu(4)))" : "") << " void " << name << (xh ? "x" : "") << (total ? "_t" : "")
-                      << "(K k, int zchunk, int tiles_x, int tiles_y, int tiles_z, int mode, double* tsum, unsigned* rec, u64* first, double lo,\n"
-                      << "    double hi) {\n"
-                      << "    const bool tr = (mode & 1) != 0, rm = (mode & 2) != 0, st = (mode & 4) != 0;\n";
-                    for (const bool p2 : {true, false}) {
-                        s << "    " << (p2 ? "if ((k.flags & 3) == 3) " : "else ") << "run_" << name << "<" << (p2 ? "true" : "false") << ", "
-                          << (xh ? "true" : "false") << ", " << (total ? "true" : "false")
-                          << ">(k, zchunk, tiles_x, tiles_y, tiles_z, tr, rm, st, tsum, rec, first, lo, hi);\n";
-                    }
-                    s << "}\n";
-                }
-            }
-            out_ << s.str();
-            WindowKernel w;
-            w.name = name;
-            w.vx = 4;
-            w.ty = TY;
-            w.block_y = WAVES;
-            w.flux = form.rows ? 2 : 1;
-            w.zchunk = form.zchunk;
-            code.windows.push_back(w);
+            s << "}\n";
         }
+        out_ << s.str();
+        WindowKernel w;
+        w.name = name;
+        w.vx = 4;
+        w.ty = TY;
+        w.block_y = WAVES;
+        w.flux = 2;
+        w.zchunk = 16;
+        code.windows.push_back(w);
+    }
+
+    // The conduction window for rows that are not whole quads of cells or fill 256-wide tiles badly, for lattices past the
+    // last-level cache and for few tiles (`_r_`). The fluxes, their sharing and their order are flux_kernels'; what differs is how a wave
+    // covers rows. Its 64 lanes are W lanes a row (8, 16, 32 or 64, the launch's choice: mode >> 8 is its logarithm) on
+    // 64 / W consecutive rows, four cells a lane, so a tile is 4W cells by 8 * 64 / W rows and the launch picks the W
+    // whose tiles the rows fill best. Row starts are not 16-byte aligned (the quads are loaded as such; the card takes a
+    // 4-byte aligned quad), and a row's last quad is read from the row's last four cells and moved up, the last cell
+    // repeated behind it: its face to the cells that are not there then has a flux of +0, as a closed face's.
+    void row_flux_kernels(ProgramCode& code, int target, int kk)
+    {
+        const std::string t = std::to_string(target);
+        const int TY = 8;
+        const std::string name = code.gather + "_r_" + std::to_string(TY);
+        const std::string MK = "M_" + name, LDS = "L_" + name;
+        // rows of 4W + 8 floats: W 64: 10 x 264; 32: 18 x 136; 16: 34 x 72; 8: 66 x 40
+        const int plane = 2640;
+        std::ostringstream s;
+        s << "typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));\n"
+          << "template <bool P2> struct " << MK << " { static constexpr bool kPow2 = P2; static constexpr bool kAnyH = false; };\n"
+          << "__shared__ __attribute__((aligned(16))) float " << LDS << "[" << 2 * plane << "];\n"
+          << "template <bool P2, bool TOTAL> __device__ __forceinline__ void run_" << name
+          << "(const K& k, int zchunk, int tiles_x, int tiles_y, int tiles_z, const int mode, double* tsum, unsigned* rec, u64* first,\n"
+          << "    double lo_r, double hi_r) {\n"
+          << "    const bool TRACK = (mode & 1) != 0, REMAP = (mode & 2) != 0, STREAM = (mode & 4) != 0;\n"
+          << "    const int lw = mode >> 8, W = 1 << lw, S = 4 * W + 8, R = " << TY << " * (64 >> lw);\n"
+          << "    const int tl = REMAP ? xcd_tile((int)blockIdx.x, tiles_x * tiles_y * tiles_z) : (int)blockIdx.x;\n"
+          << "    const int lane = (int)threadIdx.x, wave = (int)threadIdx.y, l = lane & (W - 1), r = wave * (64 >> lw) + (lane >> lw);\n"
+          << "    const int x = (tl % tiles_x) * 4 * W + 4 * l, y0 = ((tl / tiles_x) % tiles_y) * R, y = y0 + r;\n"
+          << "    const bool live = x < k.nx && y < k.ny;\n"
+          << "    const int z0 = (tl / (tiles_x * tiles_y)) * zchunk; const int z1 = z0 + zchunk < k.nz ? z0 + zchunk : k.nz;\n"
+          << "    const int xs = x < k.nx - 4 ? x : k.nx - 4, up = x - xs < 3 ? x - xs : 3, m = k.nx - x;\n"
+          << "    const int ys = clampi(y, 0, k.ny - 1);\n"
+          << "    const float* base = k.now[" << t << "] + (i64)ys * k.nx + xs;\n"
+          << "    float* outp = k.nxt[" << t << "] + (i64)ys * k.nx + x;\n"
+          << "    const int hy = r == 0 ? clampi(y0 - 1, 0, k.ny - 1) : (r == R - 1 ? clampi(y0 + R, 0, k.ny - 1) : ys);\n"
+          << "    const int hslot = r == 0 ? 0 : (r == R - 1 ? R + 1 : -1);\n"
+          << "    const float* hbase = k.now[" << t << "] + (i64)hy * k.nx + xs;\n"
+          << "    const int zlim = z1 < k.nz - 1 ? z1 : k.nz - 1;\n"
+          << "    const int ends = l == 0 ? (x > 0 ? up - 1 : 0) : (xs + 4 < k.nx ? 4 : 3);\n" // the cell beside the tile's row, or the row's own end
+          << "    const Direct md(k);\n"
+          << "    const double kv = s" << kk << "(k, md);\n"
+          << "    const double kf = (kv + kv) > 0.0 ? 2.0 * kv * kv / (kv + kv) : 0.0;\n"
+          // the row's last quad moved up so that its first cell is x, the row's last cell behind it
+          << "    auto moved = [&](f4v q) __attribute__((always_inline)) { if (up & 1) q = f4v{q.y, q.z, q.w, q.w}; if (up & 2) q = f4v{q.z, q.w, q.w, q.w}; return q; };\n"
+          << "    struct Pl { f4v v; f4v h; float e; };\n"
+          << "    auto load = [&](Pl& p, int zp) __attribute__((always_inline)) { const i64 o = (i64)(zp < zlim ? zp : zlim) * k.nxy;\n"
+          << "        p.v = *reinterpret_cast<const f4u*>(base + o); p.e = (base + o)[ends];\n"
+          << "        if (!TOTAL) p.h = *reinterpret_cast<const f4u*>(hbase + o); };\n"
+          // a contract step's registers hold its totals: its halo rows come one plane ahead, not three
+          << "    auto halo = [&](int zp) __attribute__((always_inline)) { return *reinterpret_cast<const f4u*>(hbase + (i64)(zp < zlim ? zp : zlim) * k.nxy); };\n"
+          // three planes in flight: a plane's slot takes the load three planes on as soon as LDS and the doubles hold it
+          << "    Pl A, B, C; f4v H = {0.0f, 0.0f, 0.0f, 0.0f};\n"
+          << "    if (TOTAL) H = halo(z0);\n"
+          << "    load(A, z0); __builtin_amdgcn_sched_barrier(0); load(B, z0 + 1); __builtin_amdgcn_sched_barrier(0);\n"
+          << "    load(C, z0 + 2); __builtin_amdgcn_sched_barrier(0);\n"
+          << "    const f4v lo = moved(*reinterpret_cast<const f4u*>(base + (i64)(z0 > 0 ? z0 - 1 : 0) * k.nxy));\n"
+          << "    A.v = moved(A.v);\n"
+          << "    double c0 = (double)A.v.x, c1 = (double)A.v.y, c2 = (double)A.v.z, c3 = (double)A.v.w;\n"
+          << "    double fzm0 = kf * ((double)lo.x - c0), fzm1 = kf * ((double)lo.y - c1), fzm2 = kf * ((double)lo.z - c2),\n"
+          << "           fzm3 = kf * ((double)lo.w - c3);\n"
+          << "    int buf = 0; bool seen = false;\n"
+          // the range counts in LDS: only a broken cell touches them
+          << "    double ts = 0.0, tm = 0.0; __shared__ unsigned counts[2]; __shared__ u64 firstbad;\n"
+          << "    if (TOTAL && wave == 0 && lane == 0) { counts[0] = 0u; counts[1] = 0u; firstbad = ~0ull; }\n"
+          << "    auto step = [&](const int z, Pl& cur, Pl& nxt) __attribute__((always_inline)) {\n"
+          << "        float* const plane = " << LDS << " + buf * " << plane << ";\n"
+          << "        float* const row = plane + (r + 1) * S + 4 * l;\n" // this lane's cells are row[4..7]
+          << "        *reinterpret_cast<f4v*>(row + 4) = cur.v;\n"
+          << "        if (l == 0) row[3] = cur.e;\n        if (l == W - 1) row[8] = cur.e;\n"
+          << "        if (hslot >= 0) *reinterpret_cast<f4v*>(plane + hslot * S + 4 * l + 4) = moved(TOTAL ? H : cur.h);\n        load(cur, z + 3); if (TOTAL) H = halo(z + 1);\n"
+          << "        __syncthreads();\n"
+          << "        nxt.v = moved(nxt.v);\n"
+          << "        const f4v hi = nxt.v;\n"
+          << "        const double d0 = (double)hi.x, d1 = (double)hi.y, d2 = (double)hi.z, d3 = (double)hi.w;\n"
+          << "        if (live) {\n"
+          << "            const f4v ym = *reinterpret_cast<const f4v*>(row - S + 4), yp = *reinterpret_cast<const f4v*>(row + S + 4);\n"
+          // past a row's ends LDS holds its own last cells (a lane past the end holds the last cell four times)
+          << "            const double fxm = kf * ((double)row[3] - c0), f01 = kf * (c1 - c0), f12 = kf * (c2 - c1), f23 = kf * (c3 - c2),\n"
+          << "                         fxp = kf * ((double)row[8] - c3);\n"
+          << "            const double fzp0 = kf * (d0 - c0), fzp1 = kf * (d1 - c1), fzp2 = kf * (d2 - c2), fzp3 = kf * (d3 - c3);\n"
+          << "            double q0 = 0.0 + fxm; q0 += f01; q0 += kf * ((double)ym.x - c0); q0 += kf * ((double)yp.x - c0); q0 += fzm0; q0 += fzp0;\n"
+          << "            double q1 = 0.0 + (-f01); q1 += f12; q1 += kf * ((double)ym.y - c1); q1 += kf * ((double)yp.y - c1); q1 += fzm1; q1 += fzp1;\n"
+          << "            double q2 = 0.0 + (-f12); q2 += f23; q2 += kf * ((double)ym.z - c2); q2 += kf * ((double)yp.z - c2); q2 += fzm2; q2 += fzp2;\n"
+          << "            double q3 = 0.0 + (-f23); q3 += fxp; q3 += kf * ((double)ym.w - c3); q3 += kf * ((double)yp.w - c3); q3 += fzm3; q3 += fzp3;\n"
+          << "            if (q0 != q0 || q1 != q1 || q2 != q2 || q3 != q3) {\n"
+          // An infinity or NaN among the inputs: the faces the cells have, in the CPU's order (a cell whose quad ends
+          // with it has none to the right).
+          << "                const bool xl = x > 0, yl = y > 0, yr = y + 1 < k.ny, zl = z > 0, zr = z + 1 < k.nz;\n"
+          << "                q0 = 0.0; if (xl) q0 += fxm; if (m > 1) q0 += f01; if (yl) q0 += kf * ((double)ym.x - c0); if (yr) q0 += kf * ((double)yp.x - c0);\n"
+          << "                if (zl) q0 += fzm0; if (zr) q0 += fzp0;\n"
+          << "                q1 = 0.0; q1 += -f01; if (m > 2) q1 += f12; if (yl) q1 += kf * ((double)ym.y - c1); if (yr) q1 += kf * ((double)yp.y - c1);\n"
+          << "                if (zl) q1 += fzm1; if (zr) q1 += fzp1;\n"
+          << "                q2 = 0.0; q2 += -f12; if (m > 3) q2 += f23; if (yl) q2 += kf * ((double)ym.z - c2); if (yr) q2 += kf * ((double)yp.z - c2);\n"
+          << "                if (zl) q2 += fzm2; if (zr) q2 += fzp2;\n"
+          << "                q3 = 0.0; q3 += -f23; if (m > 4) q3 += fxp; if (yl) q3 += kf * ((double)ym.w - c3); if (yr) q3 += kf * ((double)yp.w - c3);\n"
+          << "                if (zl) q3 += fzm3; if (zr) q3 += fzp3;\n"
+          << "            }\n"
+          << "            q0 = div_hh<" << MK << "<P2>>(k, q0); q1 = div_hh<" << MK << "<P2>>(k, q1);\n"
+          << "            q2 = div_hh<" << MK << "<P2>>(k, q2); q3 = div_hh<" << MK << "<P2>>(k, q3);\n"
+          << "            const f4v c = {(float)c0, (float)c1, (float)c2, (float)c3};\n"
+          << "            const f4v nv = {fe_ftz(c.x + fe_rf((double)fe_rf(q0) * k.dt)), fe_ftz(c.y + fe_rf((double)fe_rf(q1) * k.dt)),\n"
+          << "                            fe_ftz(c.z + fe_rf((double)fe_rf(q2) * k.dt)), fe_ftz(c.w + fe_rf((double)fe_rf(q3) * k.dt))};\n"
+          << "            float* const dst = outp + (i64)z * k.nxy;\n"
+          << "            if (m >= 4) { if (STREAM) __builtin_nontemporal_store(nv, reinterpret_cast<f4u*>(dst)); else *reinterpret_cast<f4u*>(dst) = nv; }\n"
+          << "            else { dst[0] = nv.x; if (m > 1) dst[1] = nv.y; if (m > 2) dst[2] = nv.z; }\n"
+          << "            if (TRACK) {\n"
+          << "                const bool ch = __float_as_uint(nv.x) != __float_as_uint(c.x) || (m > 1 && __float_as_uint(nv.y) != __float_as_uint(c.y)) ||\n"
+          << "                    (m > 2 && __float_as_uint(nv.z) != __float_as_uint(c.z)) || (m > 3 && __float_as_uint(nv.w) != __float_as_uint(c.w));\n"
+          << "                seen = seen || ch; }\n"
+          << "            if (TOTAL) {\n"
+          << "                const double v0 = (double)nv.x, v1 = m > 1 ? (double)nv.y : 0.0, v2 = m > 2 ? (double)nv.z : 0.0, v3 = m > 3 ? (double)nv.w : 0.0;\n"
+          << "                ts += v0; tm += fabs(v0); ts += v1; tm += fabs(v1); ts += v2; tm += fabs(v2); ts += v3; tm += fabs(v3);\n"
+          // out of range or not finite (the rare path: counted, and the least index kept)
+          << "                const bool b0 = !(v0 >= lo_r && v0 <= hi_r), b1 = m > 1 && !(v1 >= lo_r && v1 <= hi_r),\n"
+          << "                           b2 = m > 2 && !(v2 >= lo_r && v2 <= hi_r), b3 = m > 3 && !(v3 >= lo_r && v3 <= hi_r);\n"
+          << "                if (b0 || b1 || b2 || b3) {\n"
+          << "                    const double vs[4] = {v0, v1, v2, v3};\n"
+          << "                    const bool bs[4] = {b0, b1, b2, b3};\n"
+          << "#pragma unroll\n"
+          << "                    for (int q = 0; q < 4; ++q) {\n"
+          << "                        if (!bs[q]) continue;\n"
+          << "                        atomicAdd(&counts[finite_d(vs[q]) ? 0 : 1], 1u);\n"
+          << "                        atomicMin(&firstbad, (u64)z * (u64)k.nxy + (u64)y * (u64)k.nx + (u64)(x + q)); } } }\n"
+          << "            fzm0 = -fzp0; fzm1 = -fzp1; fzm2 = -fzp2; fzm3 = -fzp3;\n"
+          << "        }\n"
+          << "        buf ^= 1; c0 = d0; c1 = d1; c2 = d2; c3 = d3;\n"
+          << "    };\n"
+          << "    int z = z0;\n"
+          << "    for (; z + 3 <= z1; z += 3) { step(z, A, B); step(z + 1, B, C); step(z + 2, C, A); }\n"
+          << "    if (z < z1) { step(z, A, B); if (z + 1 < z1) step(z + 1, B, C); }\n"
+          << "    if (TRACK) mark(k, " << t << ", seen);\n"
+          << "    if (TOTAL) {\n"
+          << "        __shared__ double wv[" << TY << "][4];\n"
+          << "        Sum ps = {ts, 0.0}, pm = {tm, 0.0};\n"
+          << "        wave_fold(ps); wave_fold(pm);\n"
+          << "        if (lane == 0) { wv[wave][0] = ps.s; wv[wave][1] = ps.c; wv[wave][2] = pm.s; wv[wave][3] = pm.c; }\n"
+          << "        __syncthreads();\n"
+          << "        if (lane == 0 && wave == 0) {\n"
+          << "            if (counts[0] != 0u) atomicAdd(rec, counts[0]);\n"
+          << "            if (counts[1] != 0u) atomicAdd(rec + 1, counts[1]);\n"
+          << "            if (firstbad != ~0ull) atomicMin(first, firstbad);\n"
+          << "            Sum a = {wv[0][0], wv[0][1]}, b = {wv[0][2], wv[0][3]};\n"
+          << "            for (int q = 1; q < " << TY << "; ++q) { merge(a, Sum{wv[q][0], wv[q][1]}); merge(b, Sum{wv[q][2], wv[q][3]}); }\n"
+          << "            tsum[2 * tl] = a.s + a.c; tsum[2 * tl + 1] = b.s + b.c; } }\n"
+          << "}\n";
+        for (const bool total : {false, true}) {
+            s << "extern \"C\" __global__ __launch_bounds__(" << 64 * TY << ") __attribute__((amdgpu_waves_per_eu(" << 4 << "))) void " << name << (total ? "_t" : "")
+              << "(K k, int zchunk, int tiles_x, int tiles_y, int tiles_z, int mode, double* tsum, unsigned* rec, u64* first, double lo,\n"
+              << "    double hi) {\n";
+            for (const bool p2 : {true, false}) {
+                s << "    " << (p2 ? "if ((k.flags & 3) == 3) " : "else ") << "run_" << name << "<" << (p2 ? "true" : "false") << ", "
+                  << (total ? "true" : "false") << ">(k, zchunk, tiles_x, tiles_y, tiles_z, mode, tsum, rec, first, lo, hi);\n";
+            }
+            s << "}\n";
+        }
+        out_ << s.str();
+        WindowKernel w;
+        w.name = name;
+        w.vx = 4;
+        w.ty = TY;
+        w.block_y = TY;
+        w.flux = 3;
+        w.zchunk = 16;
+        code.windows.push_back(w);
     }
 
     // How far from its cell the gather reads each field through what it inlines (stages are read where they lie).
@@ -2461,7 +2609,7 @@ private:
         // for planes z-R..z+R (`own`), as the LDS ring holds them. Every other read goes through the ring.
         const int NOWN = 2 * R + 1;
         s << "template <bool P2> struct " << W << " {\n    static constexpr bool kClamps = false;\n    static constexpr bool kExact = false;\n"
-          << "    static constexpr bool kInner = false;\n"
+          << "    static constexpr bool kInner = false;\n    static constexpr bool kAnyH = false;\n"
           << "    static constexpr bool kPow2 = P2;\n"
           << "    int x0; int y0; int xc; int yc; int zc; mutable bool bad; double u[" << std::max(1, lay_.uniforms) << "];\n"
           << "    float own[" << NW << "][" << NOWN << "][" << VX << "];\n"

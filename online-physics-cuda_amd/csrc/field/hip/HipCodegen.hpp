@@ -75,8 +75,8 @@ struct WindowKernel {
     int vx = 1;
     int ty = 0;
     int block_y = 0;
-    // A conduction term's flux-carrying window (vx = 4; preferred where nx is a multiple of 4): 1 with waves that only
-    // load the halo rows, 2 with the halo rows loaded by the tile's edge rows; 0 the generic window.
+    // A conduction term's flux-carrying window (vx = 4): 2 for rows of whole quads, 3 for any row length of four cells or
+    // more (the launch's mode >> 8 the logarithm of its lanes a row); 0 the generic window.
     int flux = 0;
     int zchunk = 0; // planes a tile; 0: the program's
 };

@@ -71,6 +71,9 @@ constexpr int kTotals = 1024;      // doubles of conserved totals judged at once
 constexpr int kFillWaves = 2048;    // two waves a SIMD of MI355X: a generic window's launch shortens its z-chunks to reach it
 constexpr int kRanges = 1024;      // range checks judged at once (a record each: two counts and the first bad cell)
 constexpr std::size_t kNearCells = std::size_t{1} << 22; // cells up to which a distance line tries every pair
+// Cells from which a conduction window beats the direct gather (a step of few tiles is as long as a tile's
+// march: 64^3 6.4 us against 3.0, 96^3 7.0 against 7.0, 100^3 7.2 against 8.3, 128^3 7.8 against 9.7).
+constexpr std::size_t kRowCells = 900000;
 constexpr int kMaxWindowRegisters = 168; // a lane's registers that still leave a window gather three waves a SIMD
 
 struct Impl final : HipBackend {
@@ -102,7 +105,7 @@ struct Impl final : HipBackend {
     // other): FIELD_HIP_TILE="<cells a lane>x<rows>", FIELD_HIP_ZCHUNK=<planes a tile>, FIELD_HIP_DIRECT=1,
     // FIELD_HIP_REMAP=0|1 (tiles in XCD runs), FIELD_HIP_STREAM=0|1 (streaming stores).
     int tile_vx = 0, tile_ty = 0, zchunk_override = 0, remap_override = -1, stream_override = -1;
-    int tile_flux = 0; // FIELD_HIP_TILE named a flux-carrying window: 1 "f4x..", 2 "h4x.."
+    int tile_flux = 0; // FIELD_HIP_TILE named a flux-carrying window: 2 "h4x8", 3 "r4x8"
     bool force_direct = false;
     std::string last_gather;
     std::vector<void*> own; // per field bound to a caller's buffer: its own array (else null)
@@ -178,6 +181,18 @@ struct Impl final : HipBackend {
         return f;
     }
 
+    // 1 / h and 1 / h^2 in the kernels' arguments: where h (h^2) is a power of two a product with them is the quotient's
+    // bits (flags 1, 2; and, as normal floats, a float's); elsewhere they start a correctly rounded division (flag 4: no step
+    // of it over- or underflows). Past both, the kernels that divide.
+    int spacing_flags() const
+    {
+        int e = 0;
+        auto power_of_two = [&](double q) { return std::frexp(q, &e) == 0.5 && e > -125 && e < 126; };
+        auto moderate = [&](double q) { return std::isnormal(q) && (std::frexp(q, &e), e > -200 && e < 200); };
+        const double hh = shape.cell * shape.cell;
+        return (power_of_two(shape.cell) ? 1 : 0) | (power_of_two(hh) ? 2 : 0) | (moderate(shape.cell) && moderate(hh) ? 4 : 0);
+    }
+
     // The generated module's argument struct, by value (HipCodegen.cpp: struct K).
     std::vector<std::uint64_t> args(double dt) const
     {
@@ -203,18 +218,11 @@ struct Impl final : HipBackend {
         std::memcpy(&k[w++], &cells, 8);
         std::memcpy(&k[w++], &shape.cell, 8);
         std::memcpy(&k[w++], &dt, 8);
-        // 1 / h and 1 / h^2, used only where h (h^2) is a power of two: then a product with them is the quotient's bits
-        int e = 0;
-        // (and, as normal floats, a float's: past that range the kernels divide).
-        auto power_of_two = [&](double q) { return std::frexp(q, &e) == 0.5 && e > -125 && e < 126; };
-        const bool h_pow2 = power_of_two(shape.cell);
-        const double hh = shape.cell * shape.cell;
-        const bool hh_pow2 = power_of_two(hh);
-        const double inv_h = h_pow2 ? 1.0 / shape.cell : 0.0;
-        const double inv_hh = hh_pow2 ? 1.0 / hh : 0.0;
+        const double hh = shape.cell * shape.cell, inv_h = 1.0 / shape.cell, inv_hh = 1.0 / hh;
+        const int flags = spacing_flags();
         std::memcpy(&k[w++], &inv_h, 8);
         std::memcpy(&k[w++], &inv_hh, 8);
-        const int ints[4] = {shape.nx, shape.ny, shape.nz, (h_pow2 ? 1 : 0) | (hh_pow2 ? 2 : 0)};
+        const int ints[4] = {shape.nx, shape.ny, shape.nz, flags};
         std::memcpy(&k[w], ints, 16);
         w += 2;
         for (std::size_t p = 0; p < law->param_values.size(); ++p) {
@@ -272,8 +280,8 @@ struct Impl final : HipBackend {
     {
         const hip::WindowKernel* w = window_for(code);
         if (w == nullptr) {
-            // the direct gather, with 32-bit reads while the lattice allows them
-            last_gather = shape.cells() < (std::size_t{1} << 30) ? code.gather + "_32" : code.gather;
+            // the direct gather, with 32-bit reads while the lattice (and its spacing) allows them
+            last_gather = shape.cells() < (std::size_t{1} << 30) && spacing_flags() >= 3 ? code.gather + "_32" : code.gather;
             launch_cells(last_gather, dt);
             return;
         }
@@ -281,6 +289,12 @@ struct Impl final : HipBackend {
         int zchunk = zchunk_override > 0 ? zchunk_override : (w->zchunk > 0 ? w->zchunk : code.zchunk);
         int tx = (shape.nx + 64 * w->vx - 1) / (64 * w->vx);
         int ty = (shape.ny + w->ty - 1) / w->ty;
+        const Tiling rows = w->flux == 3 ? row_tiling() : Tiling{};
+        if (w->flux == 3) {
+            zchunk = zchunk_override > 0 ? zchunk_override : rows.zchunk;
+            tx = rows.tx;
+            ty = rows.ty;
+        }
         if (w->flux == 0 && zchunk_override <= 0) {
             // A flat lattice (a few rows of tiles, e.g. ny = 1) leaves few tiles: shorter z-chunks, until the card has
             // two waves a SIMD (or the chunks are 4 planes).
@@ -294,10 +308,10 @@ struct Impl final : HipBackend {
             throw std::runtime_error("lattice too large for one launch");
         }
         std::vector<std::uint64_t> k = args(dt);
-        const bool fits = fits_llc();
+        const bool fits = w->flux != 0 ? flux_cached() : fits_llc();
         const bool remap = remap_override >= 0 ? remap_override != 0 : fits;
         const bool stream = stream_override >= 0 ? stream_override != 0 : !fits;
-        int mode = (tracking ? 1 : 0) | (remap ? 2 : 0) | (stream ? 4 : 0);
+        int mode = (tracking ? 1 : 0) | (remap ? 2 : 0) | (stream ? 4 : 0) | (rows.lanes_log2 << 8);
         if (w->flux == 0) {
             void* argv[] = {k.data(), &zchunk, &tx, &ty, &tz, &mode};
             check(fe_hip_launch(fn(w->name), static_cast<unsigned>(total), 1, 1, 64, static_cast<unsigned>(w->block_y), 1, 0, argv),
@@ -305,8 +319,7 @@ struct Impl final : HipBackend {
             ++prof.launches;
             return;
         }
-        // Flux windows: rows spanning several tiles take the kernel that loads halo columns; a contract step's may take
-        // the totals.
+        // Flux windows: a contract step's may take the totals.
         double* tsum = nullptr;
         unsigned* rec = nullptr;
         unsigned long long* first = nullptr;
@@ -323,7 +336,7 @@ struct Impl final : HipBackend {
             hi = d.hi;
             fused->tiles = total;
         }
-        const std::string name = w->name + (tx > 1 ? "x" : "") + (fused != nullptr ? "_t" : "");
+        const std::string name = w->name + (fused != nullptr ? "_t" : "");
         void* argv[] = {k.data(), &zchunk, &tx, &ty, &tz, &mode, &tsum, &rec, &first, &lo, &hi};
         check(fe_hip_launch(fn(name), static_cast<unsigned>(total), 1, 1, 64, static_cast<unsigned>(w->block_y), 1, 0, argv),
             ("launch " + name).c_str());
@@ -340,25 +353,70 @@ struct Impl final : HipBackend {
         return 8.0 * static_cast<double>(shape.nx) * shape.ny * shape.nz * layout.fields <= 256.0 * 1024 * 1024;
     }
 
-    // The window gather for this lattice. Where rows are whole float4s: a conduction term's flux-carrying window (the
-    // form with halo rows loaded by the edge rows while the fields fit the last-level cache, the form with halo waves
-    // past it), else four cells a lane; else a cell a lane. Among windows of one kind, the tallest tile that still
-    // leaves at least 512 tiles (two per CU) to spread (measured on MI355X, the generic window at z-chunks of 32: 256^3
-    // 29.1 us with 256x4 tiles against 31.2 with 256x2 and 39.9 with 256x6; 512^3 219 us with 256x6 against 251 and
-    // 253). FIELD_HIP_TILE (e.g. "4x2", "1x6", "f4x4" or "h4x8" for the two flux-carrying forms) picks one. None: the
-    // direct gather.
+    // Whether a conduction window's two copies of its field sit in the last-level cache with room to spare: measured on
+    // MI355X, 128 MB (256^3) and 64 MB run faster in 16-plane chunks, 256 MB (512^2 x 128) and 250 MB (320^3) in 32.
+    bool flux_cached() const { return 8.0 * static_cast<double>(shape.cells()) <= 160.0 * 1024 * 1024; }
+
+    // How the conduction window for any row length (flux 3) covers this lattice: 2^lanes_log2 lanes a row, four cells a lane, eight
+    // waves a block. The lanes whose tiles the lattice fills best, more lanes a row where they are as good (fewer halo
+    // rows); then chunks of planes while the launch has two tiles a CU, shorter down to 4 planes.
+    struct Tiling {
+        int lanes_log2 = 0, tx = 0, ty = 0, zchunk = 0;
+        long long tiles = 0;
+    };
+    Tiling row_tiling() const
+    {
+        Tiling best;
+        double best_fill = 0.0;
+        for (int lw = 6; lw >= 3; --lw) {
+            const int width = 4 << lw, rows = 512 >> lw;
+            const int tx = (shape.nx + width - 1) / width, ty = (shape.ny + rows - 1) / rows;
+            const double fill = static_cast<double>(shape.nx) * shape.ny / (1.0 * tx * width * ty * rows);
+            if (fill > best_fill * 1.03) {
+                best_fill = fill;
+                best.lanes_log2 = lw;
+                best.tx = tx;
+                best.ty = ty;
+            }
+        }
+        best.zchunk = flux_cached() ? 16 : 32;
+        auto tiles = [&] { return 1LL * best.tx * best.ty * ((shape.nz + best.zchunk - 1) / best.zchunk); };
+        while (best.zchunk > 4 && tiles() < 512) {
+            best.zchunk /= 2;
+        }
+        best.tiles = tiles();
+        return best;
+    }
+
+    // The window gather for this lattice. A conduction term: the flux-carrying window for rows of whole quads that fill
+    // one 256-wide tile while the lattice sits in the last-level cache and the launch has two tiles a CU; for any other
+    // row, size or number of tiles the one that takes every row (its chunks of planes shorten). Measured on MI355X a step,
+    // that form against what ran before: 100^3 6.6 us against 8.3, 128^3 7.4 against 12.3, 200^3 21.5 against 32.0,
+    // 256 x 128^2 10.9 against 15.4, 333 x 301 x 200 39 against 66, 501 x 333 x 290 89 against 117, 512 x 512 x 128 50
+    // against 69, 512^3 208 against 214, 1024 x 512 x 256 203 against 214. Any other term: four cells a lane where
+    // rows are whole float4s, else a cell a lane. Among windows of one kind, the tallest tile that still leaves at least
+    // 512 tiles (two per CU) to spread (measured on MI355X, the generic window at z-chunks of 32: 256^3 29.1 us with 256x4
+    // tiles against 31.2 with 256x2 and 39.9 with 256x6; 512^3 219 us with 256x6 against 251 and 253). FIELD_HIP_TILE
+    // (e.g. "4x2", "1x6", "h4x8" and "r4x8" for the two flux-carrying forms) picks one. None: the direct gather.
     const hip::WindowKernel* window_for(const hip::ProgramCode& code) const
     {
         // A lattice one row high leaves a window's other rows (and its halo-row waves) idle: the direct gather (measured
         // on MI355X, Black-Scholes 4096 x 1 x 512: 16.8 us a pass against 23.8 through 256x2 tiles).
-        if (!code.window || code.windows.empty() || force_direct || (shape.ny == 1 && tile_vx == 0)) {
+        if (!code.window || code.windows.empty() || force_direct || spacing_flags() < 3 || (shape.ny == 1 && tile_vx == 0)) {
+            return nullptr;
+        }
+        // A conduction term on a lattice of few cells: a step is as long as one tile's march (see kRowCells).
+        const bool conduction = std::any_of(code.windows.begin(), code.windows.end(), [](const hip::WindowKernel& w) { return w.flux == 3; });
+        if (conduction && tile_vx == 0 && shape.cells() < kRowCells) {
             return nullptr;
         }
         const hip::WindowKernel* best = nullptr;
-        const bool cached = fits_llc();
         auto rank = [&](const hip::WindowKernel& w) {
+            if (w.flux == 3) {
+                return 2;
+            }
             if (w.flux != 0) {
-                return (w.flux == 2) == cached ? 3 : 2;
+                return 3;
             }
             return w.vx == 4 ? 1 : 0;
         };
@@ -367,11 +425,14 @@ struct Impl final : HipBackend {
         // (the valley law on 144 x 144 x 48: 0.66 ms a step against 0.82 through 256x2 and 64x6 tiles), so a window is
         // taken only when the row fills at least 90% of its tiles' width.
         auto fills = [&](const hip::WindowKernel& w) {
+            if (w.flux == 3) {
+                return shape.nx >= 4;
+            }
             const long long width = 64LL * w.vx, tiles_x = (shape.nx + width - 1) / width;
             return 10LL * shape.nx >= 9LL * width * tiles_x;
         };
         for (const hip::WindowKernel& w : code.windows) {
-            if (w.vx == 4 && shape.nx % 4 != 0) {
+            if (w.vx == 4 && (w.flux == 3 ? shape.nx < 4 : shape.nx % 4 != 0 || (w.flux == 2 && shape.nx > 256))) {
                 continue;
             }
             if (tile_vx > 0) {
@@ -380,12 +441,15 @@ struct Impl final : HipBackend {
                 }
                 continue;
             }
-            if (heavy.count(w.name) != 0 || !fills(w)) {
+            if ((w.flux == 0 && heavy.count(w.name) != 0) || !fills(w)) {
                 continue;
             }
             const int zc = zchunk_override > 0 ? zchunk_override : (w.zchunk > 0 ? w.zchunk : code.zchunk);
             const long long tz = (shape.nz + zc - 1) / zc;
             const long long tiles = 1LL * ((shape.nx + 64 * w.vx - 1) / (64 * w.vx)) * ((shape.ny + w.ty - 1) / w.ty) * tz;
+            if (w.flux == 2 && (tiles < 512 || !flux_cached())) {
+                continue; // its chunks do not shorten: the other form's do (256 x 128^2: 11 us against 15)
+            }
             if (best == nullptr || rank(w) > rank(*best) || (rank(w) == rank(*best) && w.ty > best->ty && tiles >= 512)) {
                 best = &w;
             }
@@ -396,7 +460,7 @@ struct Impl final : HipBackend {
     void read_overrides()
     {
         if (const char* t = std::getenv("FIELD_HIP_TILE")) {
-            tile_flux = t[0] == 'f' ? 1 : (t[0] == 'h' ? 2 : 0);
+            tile_flux = t[0] == 'f' ? 1 : (t[0] == 'h' ? 2 : (t[0] == 'r' ? 3 : 0));
             if (std::sscanf(t + (tile_flux != 0 ? 1 : 0), "%dx%d", &tile_vx, &tile_ty) != 2) {
                 tile_vx = tile_ty = 0;
                 tile_flux = 0;
@@ -446,7 +510,7 @@ struct Impl final : HipBackend {
         allocate();
     }
 
-    // Window gathers that would run badly: private (scratch) memory, or more registers a lane than leave three waves a
+    // Generic window gathers that would run badly: private (scratch) memory, or more registers a lane than leave three waves a
     // SIMD (four cells a lane of a law with many fields). The automatic choice passes them over.
     std::set<std::string> heavy;
     void weigh_windows()
