@@ -576,6 +576,7 @@ private:
                 stages.insert(p.limit_stages.begin(), p.limit_stages.end());
             }
         }
+        fold_coefficients(stages);
         for (const int id : stages) {
             const ir::Inst& in = at(id);
             StageCode s;
@@ -620,6 +621,75 @@ private:
             }
             lay_.stages.emplace(id, s);
         }
+    }
+
+    // A stored coefficient of y and z tridiagonal lines that is a few cheap operations on fields at its own cell is not
+    // stored: the solve reads the fields and computes it (four bytes written and read a cell less, and no pass of its own).
+    // Divisions other than by the spacing stay in a pass that fills the card: in a solve, one wave a SIMD, they cost more
+    // than they save. Implicit y then z with a field's coefficients on 256^3: four stored passes (149 us) and 4 of 44 bytes
+    // a cell a solve gone, 509 -> 350 us a step.
+    std::set<int> folded_;
+    static constexpr int kFoldOps = 12;
+    bool fold_cost(int id, int& ops, std::set<int>& fields) const
+    {
+        const ir::Inst& in = at(id);
+        if (scalar(id)) {
+            return in.op != Op::Mlp;
+        }
+        switch (in.op) {
+        case Op::Field: fields.insert(in.index); return true;
+        case Op::Add: case Op::Sub: case Op::Mul: case Op::Neg: case Op::Abs: case Op::Min: case Op::Max: case Op::Pos: case Op::Step: break;
+        case Op::Div:
+            if (!by_h(in) && !by_hh(in)) {
+                return false;
+            }
+            break;
+        default: return false;
+        }
+        if (++ops > kFoldOps) {
+            return false;
+        }
+        return std::all_of(in.args.begin(), in.args.end(), [&](int a) { return fold_cost(a, ops, fields); });
+    }
+    void fold_coefficients(std::set<int>& stages)
+    {
+        std::vector<char> lines(m_.insts.size(), 0), other(m_.insts.size(), 0);
+        for (std::size_t id = 0; id < m_.insts.size(); ++id) {
+            if (!used(static_cast<int>(id))) {
+                continue;
+            }
+            const ir::Inst& in = m_.insts[id];
+            for (std::size_t q = 0; q < in.args.size(); ++q) {
+                (in.op == Op::Tridiag && in.index != 0 && q < 3 ? lines : other)[static_cast<std::size_t>(in.args[q])] = 1;
+            }
+        }
+        for (const auto* progs : {&m_.terms, &m_.learned, &m_.derives}) {
+            for (const ir::Program& p : *progs) {
+                for (const ir::Equation& e : p.equations) {
+                    other[static_cast<std::size_t>(e.value)] = 1;
+                }
+            }
+        }
+        for (auto it = stages.begin(); it != stages.end();) {
+            const int id = *it;
+            int ops = 0;
+            std::set<int> fields;
+            const bool fold = at(id).op != Op::Tridiag && lines[static_cast<std::size_t>(id)] && !other[static_cast<std::size_t>(id)] &&
+                !scalar(id) && fold_cost(id, ops, fields) && fields.size() <= 2;
+            if (fold) {
+                folded_.insert(id);
+                it = stages.erase(it);
+            } else {
+                ++it;
+            }
+        }
+    }
+    // A program's stages without the folded ones.
+    std::vector<int> kept(const std::vector<int>& ids) const
+    {
+        std::vector<int> out;
+        std::copy_if(ids.begin(), ids.end(), std::back_inserter(out), [&](int id) { return folded_.count(id) == 0; });
+        return out;
     }
 
     // A neighbour's coordinate along axis a (0 x, 1 y, 2 z) for reading argument `arg` at `v`: clamped into the lattice,
@@ -1318,6 +1388,7 @@ private:
     //    of its 64 rows with lanes along x (coalesced; floats: the CPU widens each cell's float), then each thread walks
     //    its own row from LDS; d' (and c') go to S interleaved by line (S[i * lines + line]: contiguous across the
     //    threads), and a chunk's answers leave through LDS the same way.
+    //  - A coefficient folded into the solve (fold_coefficients) is computed from the fields the sweep reads.
     //  - a, b and u one number each (uniform): c' is the same for every line, so thread 0's is kept in LDS for the
     //    backward sweep and only d' goes through S. That kernel is for lines up to kTridiagLdsLine cells (the launch
     //    gives the LDS); <kernel>_s, the general form, takes longer ones.
@@ -1334,56 +1405,92 @@ private:
     void tridiag_kernel(const StageCode& s, const ir::Inst& in, int slot, bool u)
     {
         const char* names[4] = {"a", "b", "u", "r"};
-        std::vector<int> cell; // the cell-shaped coefficients (by position)
+        // What a line's sweep reads a cell: the cell-shaped coefficients, the fields of those folded.
+        struct Read {
+            std::string name;
+            int id; // the coefficient's instruction, or -1: field `index`
+            int index;
+        };
+        std::vector<Read> cell;
+        std::set<int> leaves;
         std::ostringstream fetch;
         for (int q = 0; q < 4; ++q) {
             const int arg = in.args[static_cast<std::size_t>(q)];
             if (scalar(arg)) {
                 fetch << "    const double s_" << names[q] << " = " << d(arg) << ";\n";
+            } else if (folded_.count(arg) != 0) {
+                int ops = 0;
+                fold_cost(arg, ops, leaves);
             } else {
-                cell.push_back(q);
+                cell.push_back({names[q], arg, -1});
             }
         }
-        auto val = [&](int q, const std::string& at) {
-            return scalar(in.args[static_cast<std::size_t>(q)]) ? "s_" + std::string(names[q]) : "(double)" + at;
+        for (const int f : leaves) {
+            cell.push_back({"w" + std::to_string(f), -1, f});
+        }
+        const std::string regs = "F_" + s.kernel;
+        if (!leaves.empty()) {
+            // the folded coefficients' view: their fields as the sweep holds them
+            out_ << "template <bool P2, bool ANY> struct " << regs << " : Direct {\n    static constexpr bool kPow2 = P2;\n"
+                 << "    static constexpr bool kAnyH = ANY;\n    __device__ explicit " << regs << "(const Direct& d) : Direct(d) {}\n   ";
+            for (const int f : leaves) {
+                out_ << " float w" << f << ";";
+            }
+            out_ << "\n    template <int F> __device__ __forceinline__ float fld(const K&, int, int, int) const\n    {\n";
+            for (const int f : leaves) {
+                out_ << "        if constexpr (F == " << f << ") return w" << f << ";\n";
+            }
+            out_ << "        return 0.0f;\n    }\n"
+                 << "    template <int F> __device__ __forceinline__ float fld_any(const K& k, int x, int y, int z) const { return fld<F>(k, x, y, z); }\n};\n";
+        }
+        auto val = [&](int q, const std::function<std::string(const std::string&)>& at) {
+            const int arg = in.args[static_cast<std::size_t>(q)];
+            if (scalar(arg)) {
+                return "s_" + std::string(names[q]);
+            }
+            return folded_.count(arg) != 0 ? "(double)v" + std::to_string(arg) + "(k, held, 0, 0, 0)" : "(double)" + at(names[q]);
         };
         // One forward step at i, the cell-shaped coefficients read through `at`; c' to LDS (thread 0) or S[cq].
-        auto forward = [&](const std::function<std::string(int)>& at, const std::string& cq, const std::string& pad) {
+        auto forward = [&](const std::function<std::string(const std::string&)>& at, const std::string& cq, const std::string& pad) {
             std::ostringstream f;
-            f << pad << "const double a = " << val(0, at(0)) << "; const double uu = " << val(2, at(2)) << ";\n"
-              << pad << "const double b = " << val(1, at(1)) << " + (i == 0 ? a : 0.0) + (i + 1 == n ? uu : 0.0);\n"
+            for (const int w : leaves) {
+                f << pad << "held.w" << w << " = " << at("w" + std::to_string(w)) << ";\n";
+            }
+            f << pad << "const double a = " << val(0, at) << "; const double uu = " << val(2, at) << ";\n"
+              << pad << "const double b = " << val(1, at) << " + (i == 0 ? a : 0.0) + (i + 1 == n ? uu : 0.0);\n"
               << pad << "const double piv = i == 0 ? b : b - a * cp;\n"
               << pad << "cp = i + 1 == n ? 0.0 : uu / piv;\n"
-              << pad << "dp = (" << val(3, at(3)) << " - (i == 0 ? 0.0 : a * dp)) / piv;\n"
+              << pad << "dp = (" << val(3, at) << " - (i == 0 ? 0.0 : a * dp)) / piv;\n"
               << pad << (u ? std::string("if (t == 0) t_cp[i] = cp;") : "k.S[" + cq + "] = cp;") << " k.S[k.cells + " << cq << "] = dp;\n";
             return f.str();
         };
         // Register arrays: `prefix`<name>[len] for each cell-shaped coefficient / for d' (and c' unless uniform).
         auto coef_arrays = [&](const std::string& prefix, const std::string& len) {
             std::string r;
-            for (int q : cell) {
-                r += "float " + prefix + names[q] + "[" + len + "]; ";
+            for (const Read& q : cell) {
+                r += "float " + prefix + q.name + "[" + len + "]; ";
             }
             return r;
         };
         auto coef_load = [&](const std::string& prefix, const std::string& x, const std::string& y, const std::string& z) {
             std::string r;
-            for (int q : cell) {
-                r += " " + prefix + names[q] + "[j] = " + v(in.args[static_cast<std::size_t>(q)], x, y, z) + ";";
+            for (const Read& q : cell) {
+                r += " " + prefix + q.name + "[j] = " +
+                    (q.id >= 0 ? v(q.id, x, y, z) : "m.template fld<" + std::to_string(q.index) + ">(k, " + x + ", " + y + ", " + z + ")") + ";";
             }
             return r;
         };
         auto coef_zero = [&](const std::string& prefix) {
             std::string r;
-            for (int q : cell) {
-                r += " " + prefix + names[q] + "[j] = 0.0f;";
+            for (const Read& q : cell) {
+                r += " " + prefix + q.name + "[j] = 0.0f;";
             }
             return r;
         };
         auto coef_move = [&](const std::string& to, const std::string& from) {
             std::string r;
-            for (int q : cell) {
-                r += " " + to + names[q] + "[j] = " + from + names[q] + "[j];";
+            for (const Read& q : cell) {
+                r += " " + to + q.name + "[j] = " + from + q.name + "[j];";
             }
             return r;
         };
@@ -1401,8 +1508,13 @@ private:
         };
         auto cp_of = [&](const std::string& prefix) { return u ? std::string("t_cp[i]") : prefix + "c[j]"; };
 
-        out_ << "extern \"C\" __global__ __launch_bounds__(64) void " << s.kernel << (s.uniform && !u ? "_s" : "")
-             << "(K k) {\n    const Direct m(k);\n";
+        const std::string kernel = s.kernel + (s.uniform && !u ? "_s" : "");
+        if (leaves.empty()) {
+            out_ << "extern \"C\" __global__ __launch_bounds__(64) void " << kernel << "(K k) {\n    const Direct m(k);\n";
+        } else { // a body each for a spacing that is a power of two, one that is not, and one out of that division's range
+            out_ << "template <bool P2, bool ANY> __device__ __forceinline__ void run_" << kernel << "(const K& k) {\n    const Direct m(k);\n"
+                 << "    " << regs << "<P2, ANY> held(m);\n";
+        }
         if (u) {
             out_ << "    extern __shared__ double t_cp[];\n";
         }
@@ -1427,7 +1539,7 @@ private:
                  << coef_load("n_", "x", yi, zi) << " } else {" << coef_zero("n_") << " } }\n"
                  << "#pragma unroll\n"
                  << "            for (int j = 0; j < " << R << "; ++j) { const int i = i0 + j; if (i < n) { const i64 q = " << at << ";\n"
-                 << forward([&](int q) { return "f_" + std::string(names[q]) + "[j]"; }, "q", "                ")
+                 << forward([&](const std::string& w) { return "f_" + w + "[j]"; }, "q", "                ")
                  << "            } }\n"
                  << "#pragma unroll\n"
                  << "            for (int j = 0; j < " << R << "; ++j) {" << coef_move("f_", "n_") << " }\n"
@@ -1453,12 +1565,17 @@ private:
                  << "            for (int j = 0; j < " << R << "; ++j) { " << sweep_move("g_", "h_") << " }\n"
                  << "        }\n"
                  << "    }\n}\n";
+            if (!leaves.empty()) {
+                out_ << "extern \"C\" __global__ __launch_bounds__(64) void " << kernel << "(K k) {\n"
+                     << "    if (FE_POW2(k)) run_" << kernel << "<true, false>(k);\n"
+                     << "    else if ((k.flags & 4) != 0) run_" << kernel << "<false, false>(k);\n    else run_" << kernel << "<false, true>(k);\n}\n";
+            }
             return;
         }
         // Lines along x. A thread reads for the staging the cells (x0 + (t & 31), row (t >> 5) + 2 r), r < 32, clamped
         // into the chunk and the block's rows so every read is in bounds (what falls outside is not stored).
-        for (int q : cell) {
-            out_ << "    __shared__ float t_" << names[q] << "[64][33];\n";
+        for (const Read& q : cell) {
+            out_ << "    __shared__ float t_" << q.name << "[64][33];\n";
         }
         auto stage_load = [&](const std::string& x0, const std::string& w) {
             return "            { const int l = min((t >> 5) + 2 * j, rows - 1); const int c = " + x0 + " + min(t & 31, " + w + " - 1);" +
@@ -1481,8 +1598,8 @@ private:
              << "        __syncthreads();\n";
         if (!cell.empty()) {
             std::string st;
-            for (int q : cell) {
-                st += " t_" + std::string(names[q]) + "[l][c] = g_" + names[q] + "[j];";
+            for (const Read& q : cell) {
+                st += " t_" + q.name + "[l][c] = g_" + q.name + "[j];";
             }
             out_ << "#pragma unroll\n"
                  << "        for (int j = 0; j < 32; ++j) { const int l = (t >> 5) + 2 * j, c = t & 31; if (l < rows && c < w) {" << st << " } }\n"
@@ -1496,7 +1613,7 @@ private:
         out_ << "        if (live) {\n"
              << "            for (int j = 0; j < w; ++j) {\n"
              << "                const int i = x0 + j; const i64 q = (i64)i * lines + line;\n"
-             << forward([&](int q) { return "t_" + std::string(names[q]) + "[t][j]"; }, "q", "                ")
+             << forward([&](const std::string& w) { return "t_" + w + "[t][j]"; }, "q", "                ")
              << "            }\n"
              << "        }\n"
              << "    }\n"
@@ -1897,8 +2014,8 @@ private:
     ProgramCode program(const ir::Program& p, const std::string& tag, bool derive)
     {
         ProgramCode code;
-        code.stages = p.stages;
-        code.limit_stages = p.limit_stages;
+        code.stages = kept(p.stages);
+        code.limit_stages = kept(p.limit_stages);
         code.max_dt = p.max_dt;
         if (p.equations.empty()) {
             return code;
