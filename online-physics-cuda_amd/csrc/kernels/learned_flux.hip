@@ -77,17 +77,16 @@ constexpr float kGeluB = -2.0f * 0.7978845608028654f * 0.044715f * 1.44269504088
 
 __device__ __forceinline__ float gelu_logistic(float z)
 {
-    const float e = __builtin_amdgcn_exp2f(z * (kGeluA + kGeluB * (z * z)));
+    const float e = __builtin_amdgcn_exp2f(z * __builtin_fmaf(kGeluB, z * z, kGeluA));
     return __builtin_amdgcn_rcpf(1.0f + e);
 }
 
 __device__ __forceinline__ float gelu(float z) { return z * gelu_logistic(z); }
 
-// d/dz z s(z) = s + z s (1 - s) 2 u'(z), u' = sqrt(2 / pi) (1 + 3 0.044715 z^2).
-__device__ __forceinline__ float gelu_grad(float z)
+// d/dz z s(z) = s + z s (1 - s) 2 u'(z), u' = sqrt(2 / pi) (1 + 3 0.044715 z^2), sg the s the forward pass took.
+__device__ __forceinline__ float gelu_grad(float z, float sg)
 {
     const float k0 = 0.7978845608028654f;
-    const float sg = gelu_logistic(z);
     return sg + z * sg * (1.0f - sg) * (2.0f * k0) * (1.0f + 3.0f * 0.044715f * (z * z));
 }
 
@@ -143,113 +142,223 @@ __device__ __forceinline__ void cell_of(long long i, int nx, int ny, long long& 
     x = (int)(c - yy * (unsigned)nx);
 }
 
-// Input k of evaluation row `row` (a face evaluation: (lattice, cell, direction) * 2 + side) at feature in (< 18).
-__device__ __forceinline__ float patch_value(const float* __restrict__ u, const float* __restrict__ v, const Lattice& L, long long fe,
-    int side, int in)
+// Where a lane finds the inputs of the evaluation row it holds in layer 1's B operand. Row n of a 16-row tile is face
+// n >> 1 of the tile's eight (cell n >> 2, direction (n >> 1) & 1), side n & 1 (1: the cell across the face, read
+// mirrored), whatever the tile; so a lane's inputs F(0, g, e) lie at the same offsets from its cell in every tile. Elements
+// 0..3 are inputs for every lane group, 4 and 5 for group 0 alone (18 inputs), 6 and 7 for none.
+constexpr int kReads = 6;
+struct Patch {
+    const float *u, *v;
+    int at[kReads]; // dy nx + dx: where nothing is clamped
+};
+
+// Element e's input of the lane: its field (false: u) and its cell's offset from the row's.
+__device__ __forceinline__ bool patch_input(int e, int& dx, int& dy)
 {
-    const long long cells = (long long)L.nx * L.ny;
-    const int dir = (int)(fe & 1);
-    long long lat;
-    int x, y;
-    cell_of(fe >> 1, L.nx, L.ny, lat, x, y);
-    const int field = in / 9, a = (in % 9) / 3 - 1, b = in % 3 - 1;
-    // the anchor: the cell itself (side 0) or the one across the face, read mirrored (a -> -a)
-    int da = a, db = b;
-    if (side) {
-        if (dir == 0) {
-            x += 1;
-        } else {
-            y += 1;
-        }
-        da = -a;
-    }
-    int xx = dir == 0 ? x + da : x + db;
-    int yy = dir == 0 ? y + db : y + da;
-    xx = min(max(xx, 0), L.nx - 1);
-    yy = min(max(yy, 0), L.ny - 1);
-    const float* f = field == 0 ? u : v;
-    return f[lat * cells + (long long)yy * L.nx + xx];
+    const int l = (int)(threadIdx.x & 63u), g = l >> 4, n = l & 15, dir = (n >> 1) & 1, side = n & 1;
+    const int in = min(kfeat(0, g, e), kIn - 1), a = (in % 9) / 3 - 1, b = in % 3 - 1, along = side ? 1 - a : a;
+    dx = dir == 0 ? along : b;
+    dy = dir == 0 ? b : along;
+    return in >= 9;
 }
 
-// The forward pass of 16 evaluation rows (8 faces, direct and mirror) held by one wave. Returns, in lane n < 16 of
-// group 0, outputs 0 and 1 of row n (o0, o1); keeps what the backward pass needs when asked.
+__device__ __forceinline__ Patch patch_of(const float* __restrict__ u, const float* __restrict__ v, int nx)
+{
+    Patch p;
+    p.u = u;
+    p.v = v;
+#pragma unroll
+    for (int e = 0; e < kReads; ++e) {
+        int dx, dy;
+        (void)patch_input(e, dx, dy);
+        p.at[e] = dy * nx + dx;
+    }
+    return p;
+}
+
+// The cell (its linear index, x and y) of this lane's row in the tile whose first cell is c0 at (x0, y0): at most seven
+// cells on (a cell past the last one is read as the last: its row's outputs go nowhere).
+__device__ __forceinline__ void cell_on(int step, unsigned c0, int x0, int y0, const Lattice& L, unsigned cells, unsigned& c, int& x, int& y)
+{
+    c = c0 + (unsigned)step;
+    x = x0 + step;
+    y = y0;
+    while (x >= L.nx) {
+        x -= L.nx;
+        y = y + 1 < L.ny ? y + 1 : 0;
+    }
+    if (c >= cells) {
+        c = cells - 1u;
+        x = L.nx - 1;
+        y = L.ny - 1;
+    }
+}
+
+__device__ __forceinline__ bf16x8 patch_rows(const Patch& p, const Lattice& L, unsigned c, int x, int y)
+{
+    float in[kReads];
+    const bool inside = x >= 1 && x + 2 < L.nx && y >= 1 && y + 2 < L.ny;
+    if (__all(inside)) { // nothing to clamp for any row of the tile
+#pragma unroll
+        for (int e = 0; e < kReads; ++e) {
+            const int in_e = kfeat(0, (int)(threadIdx.x & 63u) >> 4, e);
+            in[e] = (in_e >= 9 ? p.v : p.u)[(long long)((int)c + p.at[e])];
+        }
+    } else {
+        const int row0 = (int)c - y * L.nx - x;
+#pragma unroll
+        for (int e = 0; e < kReads; ++e) {
+            int dx, dy;
+            const bool second = patch_input(e, dx, dy);
+            const int xx = min(max(x + dx, 0), L.nx - 1), yy = min(max(y + dy, 0), L.ny - 1);
+            in[e] = (second ? p.v : p.u)[(long long)(row0 + yy * L.nx + xx)];
+        }
+    }
+    const bool first = (threadIdx.x & 48u) == 0u;
+    bf16x8 out;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        out[e] = bf(e < 4 ? in[e] : (e < kReads && first ? in[e < kReads ? e : 0] : 0.0f));
+    }
+    return out;
+}
+
+// The biases a lane group's accumulators start from, into LDS: two hidden layers of four blocks, then the outputs (rows 0
+// and 1). Held in registers they would take 36 a lane.
+__device__ __forceinline__ void biases_into(floatx4 (&B)[9][4], const float* __restrict__ params)
+{
+    if (threadIdx.x < 36u) {
+        const int b = (int)threadIdx.x >> 2, q = (int)threadIdx.x & 3, from = b < 4 ? kB1 + 16 * b : kB2 + 16 * (b - 4);
+        for (int r = 0; r < 4; ++r) {
+            B[b][q][r] = b < 8 ? params[from + 4 * q + r] : (r < kOut ? params[kB3 + r] : 0.0f);
+        }
+    }
+}
+
+// Face fluxes of every face evaluation: F[fe][field] = s (g_direct - g_mirror) / 2 (0 across the lattice's edge). A wave
+// takes 32 rows (16 faces of 8 cells) at a time, two tiles through each weight fragment read; the fragments and
+// the biases (the accumulators' starts) sit in LDS, and what a lane reads a row from is worked out once. Bound by the GELUs
+// (64 a lane a pair of tiles, 52 cycles each with their two quarter-rate instructions); the gather's index arithmetic,
+// the bias adds and the weights' reads were more than half of a tile's time before. Sixteen 128x128 lattices: 117 -> 59 us, four:
+// 28 -> 18 us. Four waves a SIMD: the compiler otherwise hoists the LDS reads and spills (41 us).
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_faces(
+    const bf16x8* __restrict__ frags, const float* __restrict__ params, const float* __restrict__ u, const float* __restrict__ v, Lattice L, float scale, long long faces, float* __restrict__ F, unsigned* __restrict__ clear)
+{
+    __shared__ bf16x8 W[kFragB3 * 64];
+    __shared__ floatx4 B[9][4];
+    for (int i = (int)threadIdx.x; i < kFragB3 * 64; i += 256) {
+        W[i] = frags[i];
+    }
+    biases_into(B, params);
+    if (clear != nullptr && blockIdx.x == 0 && threadIdx.x == 0) {
+        *clear = 0u; // the breach counter of the step that follows
+    }
+    __syncthreads();
+    const int l = (int)(threadIdx.x & 63u);
+    const int n = l & 15, g = l >> 4;
+    const Patch patch = patch_of(u, v, L.nx);
+    const unsigned cells = (unsigned)(faces >> 1);
+    const unsigned wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4u + (threadIdx.x >> 6)));
+    const unsigned waves = gridDim.x * 4u, pairs = (cells + 7u) / 8u;
+    for (unsigned t = wave; t < pairs; t += waves) {
+        long long lat;
+        int x0, y0;
+        cell_of((long long)(t * 8u), L.nx, L.ny, lat, x0, y0);
+        bf16x8 in[2];
+        int x[2], y[2];
+        unsigned c[2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            cell_on(4 * q + (n >> 2), t * 8u, x0, y0, L, cells, c[q], x[q], y[q]);
+            in[q] = patch_rows(patch, L, c[q], x[q], y[q]);
+        }
+        bf16x8 h[2][2];
+        floatx4 z[2][4];
+        // the weights are read where they are used: held across trips or layers they would not fit the registers
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int ob = 0; ob < 4; ++ob) {
+            const bf16x8 w = W[(kFragF1 + ob) * 64 + l];
+            z[0][ob] = mfma(w, in[0], B[ob][g]);
+            z[1][ob] = mfma(w, in[1], B[ob][g]);
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                h[q][0][e] = bf(gelu(z[q][e >> 2][e & 3]));
+                h[q][1][e] = bf(gelu(z[q][2 + (e >> 2)][e & 3]));
+            }
+        }
+#pragma unroll
+        for (int ob = 0; ob < 4; ++ob) {
+            asm volatile("" ::: "memory");
+            const bf16x8 w0 = W[(kFragF2 + 2 * ob) * 64 + l], w1 = W[(kFragF2 + 2 * ob + 1) * 64 + l];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                z[q][ob] = mfma(w1, h[q][1], mfma(w0, h[q][0], B[4 + ob][g]));
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                h[q][0][e] = bf(gelu(z[q][e >> 2][e & 3]));
+                h[q][1][e] = bf(gelu(z[q][2 + (e >> 2)][e & 3]));
+            }
+        }
+        asm volatile("" ::: "memory");
+        const bf16x8 w0 = W[kFragF3 * 64 + l], w1 = W[(kFragF3 + 1) * 64 + l];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const floatx4 o = mfma(w1, h[q][1], mfma(w0, h[q][0], B[8][g]));
+            const float m0 = __shfl_down(o[0], 1, 64), m1 = __shfl_down(o[1], 1, 64);
+            const int dir = (n >> 1) & 1;
+            if (g == 0 && (n & 1) == 0 && t * 8u + 4u * q + (unsigned)(n >> 2) < cells) {
+                const bool open = dir == 0 ? x[q] + 1 < L.nx : y[q] + 1 < L.ny;
+                const float2 f = open ? make_float2(0.5f * scale * (o[0] - m0), 0.5f * scale * (o[1] - m1)) : make_float2(0.0f, 0.0f);
+                reinterpret_cast<float2*>(F)[2LL * c[q] + dir] = f;
+            }
+        }
+    }
+}
+
+// The forward pass of 16 evaluation rows (8 faces, direct and mirror) held by one wave, keeping what the backward pass
+// needs: the activations and each GELU's derivative (half the registers of what it is computed from, and one exponential
+// and reciprocal for both).
 struct Acts {
-    floatx4 z1[4], z2[4];
+    floatx4 d1[4], d2[4];
     bf16x8 x, h1[2], h2[2];
 };
 
-__device__ __forceinline__ void forward16(const bf16x8* __restrict__ frags, const float* __restrict__ params, const float* u,
-    const float* v, const Lattice& L, long long fe0, long long fe_end, Acts& s, float& o0, float& o1)
+__device__ __forceinline__ void activate(const floatx4 (&z)[4], floatx4 (&d)[4], bf16x8 (&h)[2])
 {
-    const int l = (int)(threadIdx.x & 63u);
-    const int g = l >> 4, n = l & 15;
-    const long long fe = fe0 + (n >> 1);
-    const int side = n & 1;
-    // B operand of layer 1: inputs F(0, g, e) of row n (0 past the batch's end or past 18)
-    for (int e = 0; e < 8; ++e) {
-        const int in = kfeat(0, g, e);
-        const float val = (in < kIn && fe < fe_end) ? patch_value(u, v, L, fe, side, in) : 0.0f;
-        s.x[e] = bf(val);
-    }
-    const floatx4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
     for (int ob = 0; ob < 4; ++ob) {
-        floatx4 z = mfma(frags[(kFragF1 + ob) * 64 + l], s.x, zero);
+#pragma unroll
         for (int r = 0; r < 4; ++r) {
-            z[r] += params[kB1 + 16 * ob + 4 * g + r];
-        }
-        s.z1[ob] = z;
-    }
-    for (int c = 0; c < 2; ++c) {
-        for (int e = 0; e < 4; ++e) {
-            s.h1[c][e] = bf(gelu(s.z1[2 * c][e]));
-            s.h1[c][e + 4] = bf(gelu(s.z1[2 * c + 1][e]));
+            const float sg = gelu_logistic(z[ob][r]);
+            h[ob >> 1][4 * (ob & 1) + r] = bf(z[ob][r] * sg);
+            d[ob][r] = gelu_grad(z[ob][r], sg);
         }
     }
-    for (int ob = 0; ob < 4; ++ob) {
-        floatx4 z = mfma(frags[(kFragF2 + 2 * ob) * 64 + l], s.h1[0], zero);
-        z = mfma(frags[(kFragF2 + 2 * ob + 1) * 64 + l], s.h1[1], z);
-        for (int r = 0; r < 4; ++r) {
-            z[r] += params[kB2 + 16 * ob + 4 * g + r];
-        }
-        s.z2[ob] = z;
-    }
-    for (int c = 0; c < 2; ++c) {
-        for (int e = 0; e < 4; ++e) {
-            s.h2[c][e] = bf(gelu(s.z2[2 * c][e]));
-            s.h2[c][e + 4] = bf(gelu(s.z2[2 * c + 1][e]));
-        }
-    }
-    floatx4 y = mfma(frags[(kFragF3 + 0) * 64 + l], s.h2[0], zero);
-    y = mfma(frags[(kFragF3 + 1) * 64 + l], s.h2[1], y);
-    o0 = y[0] + params[kB3 + 0];
-    o1 = y[1] + params[kB3 + 1];
 }
 
-// Face fluxes of every face evaluation: F[fe][field] = s (g_direct - g_mirror) / 2 (0 across the lattice's edge).
-// A wave takes 16 rows (8 faces) at a time.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_faces(const bf16x8* __restrict__ frags, const float* __restrict__ params, const float* __restrict__ u,
-    const float* __restrict__ v, Lattice L, float scale, long long faces, float* __restrict__ F)
+__device__ __forceinline__ void forward16(const bf16x8* __restrict__ frags, const floatx4 (&B)[9][4], Acts& s)
 {
-    const int l = (int)(threadIdx.x & 63u);
-    const int n = l & 15, g = l >> 4;
-    const long long wave = ((long long)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    const long long waves = ((long long)gridDim.x * blockDim.x) >> 6;
-    for (long long t = wave; t * 8 < faces; t += waves) {
-        Acts s;
-        float o0, o1;
-        forward16(frags, params, u, v, L, t * 8, faces, s, o0, o1);
-        const float m0 = __shfl_down(o0, 1, 64), m1 = __shfl_down(o1, 1, 64);
-        const long long fe = t * 8 + (n >> 1);
-        if (g == 0 && (n & 1) == 0 && fe < faces) {
-            const int dir = (int)(fe & 1);
-            long long lat;
-            int x, y;
-            cell_of(fe >> 1, L.nx, L.ny, lat, x, y);
-            const bool open = dir == 0 ? x + 1 < L.nx : y + 1 < L.ny;
-            F[2 * fe] = open ? 0.5f * scale * (o0 - m0) : 0.0f;
-            F[2 * fe + 1] = open ? 0.5f * scale * (o1 - m1) : 0.0f;
-        }
+    const int l = (int)(threadIdx.x & 63u), g = l >> 4;
+    floatx4 z[4];
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob) {
+        z[ob] = mfma(frags[(kFragF1 + ob) * 64 + l], s.x, B[ob][g]);
     }
+    activate(z, s.d1, s.h1);
+#pragma unroll
+    for (int ob = 0; ob < 4; ++ob) {
+        z[ob] = mfma(frags[(kFragF2 + 2 * ob) * 64 + l], s.h1[0], B[4 + ob][g]);
+        z[ob] = mfma(frags[(kFragF2 + 2 * ob + 1) * 64 + l], s.h1[1], z[ob]);
+    }
+    activate(z, s.d2, s.h2);
 }
 
 // A cell's correction from its faces' fluxes: (inflow - outflow) / h, field by field.
@@ -348,14 +457,6 @@ __global__ void k_fallback(const float* __restrict__ u, const float* __restrict_
     v2[i] = v[i] + dt * rv;
 }
 
-__global__ void k_clear(unsigned* p, int n)
-{
-    const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (i < n) {
-        p[i] = 0u;
-    }
-}
-
 // Training, 1: the loss L = mean over cells and fields of (correction - target)^2 with target = (s1 - s0) / dt -
 // plain(s0); e = dL/dcorrection into E (two a cell), and the loss's terms into loss_parts (one a cell, summed in order
 // by k_sum).
@@ -382,22 +483,19 @@ __global__ void k_residual(const float* __restrict__ u0, const float* __restrict
     loss_parts[i] = (du * du + dv * dv) * inv;
 }
 
-// Training, 2: dL/dg of every evaluation row from E (through the faces' divergence and the antisymmetric pair).
-__device__ __forceinline__ void row_grad(const float* __restrict__ E, const Lattice& L, float scale, long long fe, int side, float& d0, float& d1)
+// Training, 2: dL/dg of the evaluation row of cell c at (x, y) from E (through the faces' divergence and the antisymmetric
+// pair).
+__device__ __forceinline__ void row_grad(const float* __restrict__ E, const Lattice& L, float scale, unsigned c, int x, int y, int dir,
+    int side, float& d0, float& d1)
 {
-    const int dir = (int)(fe & 1);
-    const long long c = fe >> 1;
-    long long lat;
-    int x, y;
-    cell_of(c, L.nx, L.ny, lat, x, y);
     const bool open = dir == 0 ? x + 1 < L.nx : y + 1 < L.ny;
     if (!open) {
         d0 = d1 = 0.0f;
         return;
     }
-    const long long c2 = c + (dir == 0 ? 1 : L.nx);
+    const long long here = c, c2 = here + (dir == 0 ? 1 : L.nx);
     // F leaves c (-F/h) and enters c2 (+F/h); F = s (g_d - g_m) / 2
-    const float df0 = (E[2 * c2] - E[2 * c]) / L.h, df1 = (E[2 * c2 + 1] - E[2 * c + 1]) / L.h;
+    const float df0 = (E[2 * c2] - E[2 * here]) / L.h, df1 = (E[2 * c2 + 1] - E[2 * here + 1]) / L.h;
     const float k = side ? -0.5f * scale : 0.5f * scale;
     d0 = k * df0;
     d1 = k * df1;
@@ -409,9 +507,13 @@ __device__ __forceinline__ void row_grad(const float* __restrict__ E, const Latt
 // number of trips; with one wave a block that holds by construction.
 constexpr int kWavesTrain = 1;
 
-__global__ __launch_bounds__(64 * kWavesTrain) void k_backward(const bf16x8* __restrict__ frags, const float* __restrict__ params,
-    const float* __restrict__ u, const float* __restrict__ v, const float* __restrict__ E, Lattice L, float scale, long long faces,
-    float* __restrict__ G)
+// Bound by latency at one wave a SIMD: 132 accumulators and the weights' fragments (100) stay in registers over the trips, 408
+// in all, and the two halves of a trip run into each other. Sixteen 128x128 lattices: 404 -> 221 us with the patches' fixed
+// offsets, the biases' gradients on the matrix cores and the GELU's derivative taken where its logistic is at hand; at
+// two waves (256 registers) it spills and takes 300, with the halves one after the other at one wave 350.
+__global__ __launch_bounds__(64 * kWavesTrain) __attribute__((amdgpu_waves_per_eu(1))) void k_backward(
+    const bf16x8* __restrict__ frags, const float* __restrict__ params, const float* __restrict__ u, const float* __restrict__ v,
+    const float* __restrict__ E, Lattice L, float scale, long long faces, float* __restrict__ G)
 {
     // A wave's LDS: rows 0..31 of the pair, features transposed ([feature][row], bf16).
     struct Tiles {
@@ -439,21 +541,42 @@ __global__ __launch_bounds__(64 * kWavesTrain) void k_backward(const bf16x8* __r
         gw1[0][a] = zero;
         gw1[1][a] = zero;
     }
-    float gb1 = 0.0f, gb2 = 0.0f, gb3 = 0.0f; // lane l: feature l (b3: output l < 2)
+    // The biases' gradients are products too: a row of ones against the gradients (the first layer's its input 18, which the
+    // weights give nothing), where a lane's sum down the LDS columns was 32 reads each.
+    floatx4 gb2[4], gb3 = zero;
+    bf16x8 ones;
+    for (int a = 0; a < 4; ++a) {
+        gb2[a] = zero;
+    }
+    for (int e = 0; e < 8; ++e) {
+        ones[e] = bf(1.0f);
+    }
+    const Patch patch = patch_of(u, v, L.nx);
+    __shared__ floatx4 B[9][4];
+    biases_into(B, params);
+    __syncthreads();
+    const unsigned cells = (unsigned)(faces >> 1);
     for (long long t = wave; t * 16 < faces; t += waves) {
+        long long lat;
+        int x0, y0;
+        cell_of(t * 8, L.nx, L.ny, lat, x0, y0);
         // rows 32 of the pair: tiles 2t and 2t + 1 (a face is 2 rows: 8 faces a tile)
         for (int half = 0; half < 2; ++half) {
             const long long fe0 = (2 * t + half) * 8;
             Acts s;
-            float o0, o1;
-            forward16(frags, params, u, v, L, fe0, faces, s, o0, o1);
-            (void)o0;
-            (void)o1;
+            unsigned c;
+            int x, y;
+            cell_on(4 * half + (n >> 2), (unsigned)(t * 8), x0, y0, L, cells, c, x, y);
+            s.x = patch_rows(patch, L, c, x, y);
+            if (g == 0) {
+                s.x[6] = bf(1.0f);
+            }
+            forward16(frags, B, s);
             // output gradients of the 16 rows: B operand of dH2 = W3 dY (lane group 0, elements 0, 1)
             const long long fe = fe0 + (n >> 1);
             float d0 = 0.0f, d1 = 0.0f;
             if (fe < faces) {
-                row_grad(E, L, scale, fe, n & 1, d0, d1);
+                row_grad(E, L, scale, c, x, y, (n >> 1) & 1, n & 1, d0, d1);
             }
             bf16x8 dyb;
             for (int e = 0; e < 8; ++e) {
@@ -467,7 +590,7 @@ __global__ __launch_bounds__(64 * kWavesTrain) void k_backward(const bf16x8* __r
             for (int ib = 0; ib < 4; ++ib) {
                 const floatx4 dh = mfma(frags[(kFragB3 + ib) * 64 + l], dyb, zero);
                 for (int r = 0; r < 4; ++r) {
-                    dz2[ib][r] = dh[r] * gelu_grad(s.z2[ib][r]);
+                    dz2[ib][r] = dh[r] * s.d2[ib][r];
                 }
             }
             bf16x8 dz2b[2];
@@ -482,7 +605,7 @@ __global__ __launch_bounds__(64 * kWavesTrain) void k_backward(const bf16x8* __r
                 floatx4 dh = mfma(frags[(kFragB2 + 2 * ib) * 64 + l], dz2b[0], zero);
                 dh = mfma(frags[(kFragB2 + 2 * ib + 1) * 64 + l], dz2b[1], dh);
                 for (int r = 0; r < 4; ++r) {
-                    dz1[ib][r] = dh[r] * gelu_grad(s.z1[ib][r]);
+                    dz1[ib][r] = dh[r] * s.d1[ib][r];
                 }
             }
             // Transposed into LDS: row = 16 half + n; features of this lane: F(c, g, e) of the packed registers.
@@ -527,19 +650,13 @@ __global__ __launch_bounds__(64 * kWavesTrain) void k_backward(const bf16x8* __r
                 gw2[ib][ob] = mfma(a2, rows8(T.dz2[16 * ob + n]), gw2[ib][ob]);
             }
             gw3[ib] = mfma(a3, rows8(T.dy[n]), gw3[ib]);
+            gb2[ib] = mfma(ones, rows8(T.dz2[16 * ib + n]), gb2[ib]);
         }
+        gb3 = mfma(ones, rows8(T.dy[n]), gb3);
         for (int ib = 0; ib < 2; ++ib) {
             const bf16x8 a1 = rows8(T.x[16 * ib + n]);
             for (int ob = 0; ob < 4; ++ob) {
                 gw1[ib][ob] = mfma(a1, rows8(T.dz1[16 * ob + n]), gw1[ib][ob]);
-            }
-        }
-        // biases: lane l sums feature l over the 32 rows, in row order
-        for (int r = 0; r < 32; ++r) {
-            gb1 += unbf(T.dz1[l][r]);
-            gb2 += unbf(T.dz2[l][r]);
-            if (l < kOut) {
-                gb3 += unbf(T.dy[l][r]);
             }
         }
         __syncthreads();
@@ -564,14 +681,19 @@ __global__ __launch_bounds__(64 * kWavesTrain) void k_backward(const bf16x8* __r
                 const int in = 16 * ib + 4 * g + r;
                 if (in < kIn) {
                     out[kW1 + in * kHid + 16 * ob + n] = gw1[ib][ob][r];
+                } else if (in == kIn) { // the input of ones
+                    out[kB1 + 16 * ob + n] = gw1[ib][ob][r];
                 }
             }
         }
     }
-    out[kB1 + l] = gb1;
-    out[kB2 + l] = gb2;
-    if (l < kOut) {
-        out[kB3 + l] = gb3;
+    if (g == 0) { // every row of the products with ones is the sum
+        for (int ob = 0; ob < 4; ++ob) {
+            out[kB2 + 16 * ob + n] = gb2[ob][0];
+        }
+        if (n < kOut) {
+            out[kB3 + n] = gb3[0];
+        }
     }
 }
 
@@ -609,7 +731,7 @@ __global__ void k_sum(const float* __restrict__ parts, int rows, int width, floa
 }
 
 // Sums n floats in two fixed-order levels: block b its chunk (each lane a fixed stride, then a fixed tree) into
-// parts[b], then k_total_fold the blocks' parts in order (one block over all n waited on memory a lane at a time).
+// parts[b], then k_total_fold the blocks' parts (one block over all n waited on memory a lane at a time).
 constexpr int kTotalBlocks = 256;
 __global__ __launch_bounds__(256) void k_total(const float* __restrict__ v, long long n, double* __restrict__ parts)
 {
@@ -635,13 +757,17 @@ __global__ __launch_bounds__(256) void k_total(const float* __restrict__ v, long
     }
 }
 
-__global__ void k_total_fold(const double* __restrict__ parts, int count, float* __restrict__ out)
+// One wave: each lane a fixed stride, then a fixed tree (one lane over all the parts took 12 us, a double's add at a time).
+__global__ __launch_bounds__(64) void k_total_fold(const double* __restrict__ parts, int count, float* __restrict__ out)
 {
+    double a = 0.0;
+    for (int b = (int)threadIdx.x; b < count; b += 64) {
+        a += parts[b];
+    }
+    for (int w = 32; w > 0; w >>= 1) {
+        a += __shfl_down(a, w, 64);
+    }
     if (threadIdx.x == 0) {
-        double a = 0.0;
-        for (int b = 0; b < count; ++b) {
-            a += parts[b];
-        }
         *out = (float)a;
     }
 }
@@ -779,7 +905,7 @@ struct fe_lnet {
     std::string error;
     hipStream_t stream() const { return static_cast<hipStream_t>(fe_hip_stream()); }
     static constexpr int kFaceBlocks = 1024; // face kernels: waves in flight (a grid-stride loop over 16-row tiles)
-    static constexpr int kTrainBlocks = 1024; // one wave a SIMD: the training pass holds 512 registers a lane
+    static constexpr int kTrainBlocks = 1024; // one wave a SIMD: the training pass holds 408 registers a lane
 };
 
 namespace {
@@ -882,7 +1008,7 @@ int fe_lnet_faces(fe_lnet* n, const float* u, const float* v, int nx, int ny, in
             n->F.alloc(static_cast<std::size_t>(2 * faces));
             F = n->F.p;
         }
-        hipLaunchKernelGGL(k_faces, dim3(fe_lnet::kFaceBlocks), dim3(256), 0, n->stream(), n->frags.p, n->params.p, u, v, L, n->scale, faces, F);
+        hipLaunchKernelGGL(k_faces, dim3(fe_lnet::kFaceBlocks), dim3(256), 0, n->stream(), n->frags.p, n->params.p, u, v, L, n->scale, faces, F, nullptr);
         hcheck(hipGetLastError(), "faces");
         return 0;
     } catch (const std::exception& e) {
@@ -906,8 +1032,7 @@ int fe_lnet_step(fe_lnet* n, const float* u, const float* v, int nx, int ny, int
         const hipStream_t s = static_cast<hipStream_t>(fe_hip_stream());
         if (learned) {
             n->F.alloc(static_cast<std::size_t>(4 * cells));
-            hipLaunchKernelGGL(k_clear, dim3(1), dim3(64), 0, s, n->flags.p, 1);
-            hipLaunchKernelGGL(k_faces, dim3(fe_lnet::kFaceBlocks), dim3(256), 0, s, n->frags.p, n->params.p, u, v, L, n->scale, 2 * cells, n->F.p);
+            hipLaunchKernelGGL(k_faces, dim3(fe_lnet::kFaceBlocks), dim3(256), 0, s, n->frags.p, n->params.p, u, v, L, n->scale, 2 * cells, n->F.p, n->flags.p);
             hipLaunchKernelGGL(k_step, dim3(blocks_for(cells, 256)), dim3(256), 0, s, u, v, n->F.p, L, R, static_cast<float>(dt), 1,
                 static_cast<float>(bound), u2, v2, n->flags.p);
             hipLaunchKernelGGL(k_fallback, dim3(blocks_for(cells, 256)), dim3(256), 0, s, u, v, L, R, static_cast<float>(dt), n->flags.p, u2, v2,
@@ -944,9 +1069,8 @@ int fe_lnet_step_noalloc(fe_lnet* n, const float* u, const float* v, int nx, int
         const Reaction R{static_cast<float>(du), static_cast<float>(dv), static_cast<float>(k)};
         const hipStream_t s = static_cast<hipStream_t>(fe_hip_stream());
         // The kernels of fe_lnet_step's learned path, with the faces and the breach counter in the scratch: the counter
-        // is cleared by a kernel (no memset node), the fallback count stays the net's own.
-        hipLaunchKernelGGL(k_clear, dim3(1), dim3(64), 0, s, breach, 1);
-        hipLaunchKernelGGL(k_faces, dim3(fe_lnet::kFaceBlocks), dim3(256), 0, s, n->frags.p, n->params.p, u, v, L, n->scale, 2 * cells, faces);
+        // is cleared by the faces' kernel (no memset node), the fallback count stays the net's own.
+        hipLaunchKernelGGL(k_faces, dim3(fe_lnet::kFaceBlocks), dim3(256), 0, s, n->frags.p, n->params.p, u, v, L, n->scale, 2 * cells, faces, breach);
         hipLaunchKernelGGL(k_step, dim3(blocks_for(cells, 256)), dim3(256), 0, s, u, v, faces, L, R, static_cast<float>(dt), 1,
             static_cast<float>(bound), u2, v2, breach);
         hipLaunchKernelGGL(k_fallback, dim3(blocks_for(cells, 256)), dim3(256), 0, s, u, v, L, R, static_cast<float>(dt), breach, u2, v2,
@@ -985,7 +1109,7 @@ int fe_lnet_gradient(fe_lnet* n, const float* u0, const float* v0, const float* 
         n->loss_parts.alloc(static_cast<std::size_t>(cells));
         const int waves = fe_lnet::kTrainBlocks * kWavesTrain;
         n->partials.alloc(static_cast<std::size_t>(waves) * kParams);
-        hipLaunchKernelGGL(k_faces, dim3(fe_lnet::kFaceBlocks), dim3(256), 0, s, n->frags.p, n->params.p, u0, v0, L, n->scale, faces, n->F.p);
+        hipLaunchKernelGGL(k_faces, dim3(fe_lnet::kFaceBlocks), dim3(256), 0, s, n->frags.p, n->params.p, u0, v0, L, n->scale, faces, n->F.p, nullptr);
         hipLaunchKernelGGL(k_residual, dim3(blocks_for(cells, 256)), dim3(256), 0, s, u0, v0, u1, v1, n->F.p, L, R, static_cast<float>(dt),
             static_cast<float>(weight), n->E.p, n->loss_parts.p);
         hipLaunchKernelGGL(k_backward, dim3(fe_lnet::kTrainBlocks), dim3(64 * kWavesTrain), 0, s, n->frags.p, n->params.p, u0, v0, n->E.p, L,

@@ -45,6 +45,26 @@ def test_face_fluxes_match_the_oracle(device):
     assert err.max() < 5e-3 * top and err.mean() < 2e-4 * top, (err.max() / top, err.mean() / top)
 
 
+@pytest.mark.parametrize("nx,ny,count", [(2, 2, 1), (2, 9, 3), (3, 2, 5), (7, 5, 2), (9, 4, 1), (19, 18, 1)])
+def test_small_and_odd_lattices_match_the_oracle(device, nx, ny, count):
+    """A tile is eight cells of the flattened lattices: rows and lattices shorter than one, cells that no tile fills, and
+    tiles of which every read is clamped. Tolerances as above (the gradient's in norm: few rows average less)."""
+    import field_hip
+
+    p = L.init_params(15, last_scale=1.0)
+    rng = np.random.default_rng(nx * 100 + ny)
+    u0, v0, u1, v1 = (rng.standard_normal(nx * ny * count).astype(np.float32) for _ in range(4))
+    net = field_hip.LearnedNet(p, SCALE)
+    out = field_hip.DeviceArray(4 * nx * ny * count)
+    net.faces(dev(u0), dev(v0), nx, ny, count, H, out)
+    ref = L.faces(p, u0, v0, nx, ny, count, SCALE)
+    assert np.max(np.abs(out.download().reshape(-1, 2) - ref)) <= 5e-3 * np.max(np.abs(ref))
+    loss, g = net.gradient(dev(u0), dev(v0), dev(u1), dev(v1), nx, ny, count, H, DU, DV, K, DT)
+    ref_loss, ref_g = L.loss_and_grad(p, u0, v0, u1, v1, nx, ny, count, H, DU, DV, K, DT, SCALE)
+    assert abs(loss - ref_loss) <= 1e-4 * ref_loss
+    assert np.linalg.norm(g - ref_g) <= 1e-2 * np.linalg.norm(ref_g)
+
+
 def test_learned_and_plain_steps_match_the_oracle(device):
     import field_hip
 
