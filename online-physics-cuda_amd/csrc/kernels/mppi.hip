@@ -1,13 +1,13 @@
 // A world model's MPPI planner on gfx950: rollouts of a learned ODE on the matrix cores and the softmin plan update.
 //
 // The reference plans with one thread a future, the dynamics MLP evaluated in fp32 registers with the weights in shared
-// memory (src/field/mind/WorldModel.cpp:192-240). Here a wave carries 16 futures at a time through the whole horizon:
-// their states in LDS (fp32), each step's inputs (state and action, normalised) rounded to fp16 into an LDS tile, and
-// the three layers as chains of v_mfma_f32_16x16x16_f16 (A: 16 futures x 16 inputs from the tile, lane l future l % 16
-// and inputs 4 (l / 16)..+3; B: the fp16 weights W[out][in], output l % 16; D: lane l output l % 16, futures
-// 4 (l / 16)..+3), fp32 accumulation, tanh on D into the other tile. The last layer's rates move the states in fp32.
-// The update weighs every future by exp(-(J - J_min) / lambda), one thread an (step, axis), summing the futures in
-// order: the same inputs give the same plan, bit for bit.
+// memory (src/field/mind/WorldModel.cpp:192-240). Here a wave carries 16 or 32 futures through the whole horizon without
+// leaving its registers: a layer is W (A: 16 outputs x 32 inputs a fragment, fp16, from LDS) times the futures' inputs (B:
+// 32 inputs x 16 futures), fp32 accumulators that start from the bias, and a product's D (lane l: future l % 16, outputs
+// 4 (l / 16)..+3 of a block of 16) is, after tanh and rounding to fp16, the next layer's B with no exchange between lanes.
+// The states stay in D's layout in fp32; the last layer's rates move them there.
+// The update weighs every future by exp(-(J - J_min) / lambda) and sums in a fixed order: the same inputs give the same
+// plan, bit for bit.
 #include "fe_mppi.h"
 #include "fe_hip.h"
 
@@ -24,28 +24,22 @@
 
 namespace {
 
-typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 typedef unsigned long long u64;
 
-constexpr int kMaxWidth = 128;        // padded inputs and hidden width
-constexpr int kMaxState = 64;         // features, padded
+constexpr int kMaxWidth = 128; // hidden width
+constexpr int kMaxState = 64;  // inputs: features and the two actions
 
 struct Desc {
-    int F, in_pad, hid, f_pad, horizon, samples;
-    const _Float16* W1; // [hid][in_pad]
-    const _Float16* W2; // [hid][hid]
-    const _Float16* W3; // [f_pad][hid]
-    const float* b1;    // [hid]
-    const float* b2;    // [hid]
-    const float* b3;    // [f_pad]
-    const float* shift; // [in_pad]
-    const float* inscale; // [in_pad]
-    const float* scale;   // [F]
-    const float* target;  // [F]
-    const float* weight;  // [F]
+    int F, fb, horizon, samples; // fb: blocks of 16 features
+    const half8* frags;    // the weights' fragments: layer 1, 2, 3, each [output block][32 inputs][lane]
+    const float4v* tables; // b1, b2 [hidden], b3 [16 fb], shift, inscale [32 NC], scale, target, weight [16 fb]
     float action_weight;
 };
+
+// The input that element e of lane group g holds of the 32 of fragment c: two blocks of a product's D side by side.
+__host__ __device__ inline int kfeat(int c, int g, int e) { return 32 * c + 16 * (e >> 2) + 4 * g + (e & 3); }
 
 // The noise of (agent id, tick, future, step, axis): a standard normal by Box-Muller from two uniforms, each the top 24
 // bits of a 64-bit mix (splitmix64's finaliser, Steele, Lea and Flood 2014) of the key and of the key's mix.
@@ -83,154 +77,249 @@ __device__ __forceinline__ float fast_tanh(float u)
     return 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
-// The block's LDS, sized to the net (a block is one wave): two fp16 activation tiles of 16 rows at a stride of ts
-// halves (the wider of the padded inputs and the hidden width, plus 8 so the 16 rows a product reads start in
-// different banks), the 16 futures' states at a stride of ss floats (odd), and their actions for two steps.
-struct Lds {
-    int ts, ss;
-    __host__ __device__ static Lds of(const Desc& d)
-    {
-        return Lds{(d.in_pad > d.hid ? d.in_pad : d.hid) + 8, d.F | 1};
-    }
-    __host__ __device__ int bytes() const { return 2 * 16 * ts * 2 + 16 * ss * 4 + 2 * 16 * 2 * 4; }
-};
-
-// One layer for a wave's 16 futures: in (K halves a row) -> out (N outputs), tanh or (last) the rates into the states.
-__device__ __forceinline__ void layer(const Desc& d, const _Float16* in, _Float16* out, int ts, int K, int N, const _Float16* W,
-    const float* b, bool last, float* st, int ss, float dt, int lane)
+// A layer's tanh, rounded into the next layer's inputs (zero past the hidden units).
+template <int HB, int Q>
+__device__ __forceinline__ void activate(const float4v (&z)[Q][HB], half8 (&h)[Q][(HB + 1) / 2])
 {
-    const int r = lane & 15, g = lane >> 4;
-    for (int nb = 0; nb < N; nb += 16) {
-        float4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int kc = 0; kc < K; kc += 16) {
-            const half4 a = *reinterpret_cast<const half4*>(in + r * ts + kc + 4 * g);
-            const half4 w = *reinterpret_cast<const half4*>(W + (long long)(nb + r) * K + kc + 4 * g);
-            acc = __builtin_amdgcn_mfma_f32_16x16x16f16(a, w, acc, 0, 0, 0);
-        }
-        const int col = nb + r;
-        const float bias = b[col];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int row = 4 * g + j;
-            const float v = acc[j] + bias;
-            if (!last) {
-                out[row * ts + col] = (_Float16)fast_tanh(v);
-            } else if (col < d.F) {
-                st[row * ss + col] += dt * v * d.scale[col];
+    for (int q = 0; q < Q; ++q) {
+#pragma unroll
+        for (int c = 0; c < (HB + 1) / 2; ++c) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int ob = 2 * c + (e >> 2);
+                h[q][c][e] = ob < HB ? (_Float16)fast_tanh(z[q][ob < HB ? ob : 0][e & 3]) : (_Float16)0.0f;
             }
         }
     }
 }
 
-// A block (agent, part), a wave a tile of 16 futures at a time: part p takes tiles 16 p, then every 16 * parts futures
-// on. Actions into acts[agent][k][t][axis], each future's cost into cost[agent][k]. LDS: Lds::of(d).bytes(). The noise
-// of two steps is drawn at once (lane l: future l / 2 % 16, axis l % 2, step t + l / 32), so every lane draws.
-__global__ __launch_bounds__(64) void k_mppi_rollout(Desc d, const float* __restrict__ obs, const float* __restrict__ mean,
-    const unsigned* __restrict__ ids, float* __restrict__ acts, float* __restrict__ cost, u64 tick, float sigma, float dt)
+// Fragments and tables (float4) of a net with HB blocks of 16 hidden units, NC fragments of inputs and fb blocks of features.
+__host__ __device__ constexpr int frag_count(int HB, int NC, int fb) { return HB * NC + (HB + fb) * ((HB + 1) / 2); }
+__host__ __device__ constexpr int table_count(int HB, int NC, int fb) { return 4 * (2 * HB + 4 * NC + 4 * fb); }
+constexpr int lds_bytes(int HB, int NC, int fb) { return frag_count(HB, NC, fb) * 1024 + table_count(HB, NC, fb) * 16; }
+
+__device__ __forceinline__ float4v mfma(half8 w, half8 x, float4v acc) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, acc, 0, 0, 0); }
+
+// A wave takes 16 Q futures of an agent at a time; wave w of the grid the items w, w + waves, ... (agent-major). Actions into
+// acts[agent][t][k][axis], each future's cost into cost[agent][k]. The noise is drawn by every lane: with two tiles (Q = 2)
+// lane l the future l / 2, axis l % 2 of the step; with one, the lanes 32.. draw the step after. The weights and the tables
+// are read from LDS where they are used (two tiles to a read).
+// Bound by the hidden units' tanh, two quarter-rate instructions each: about 165 us of 256 agents x 512 futures x 32 steps with
+// 16 features and 64 hidden units, which take 232 (784 when each layer's activations went through LDS and its weights were
+// read from memory a tile at a time); the update 8 us (36 with a thread a step and axis over all futures).
+template <int HB, int NC, int Q>
+__global__ __launch_bounds__(256) void k_mppi_rollout(Desc d, const float* __restrict__ obs, const float* __restrict__ mean,
+    const unsigned* __restrict__ ids, float* __restrict__ acts, float* __restrict__ cost, u64 tick, float sigma, float dt, unsigned items,
+    unsigned per_agent)
 {
+    constexpr int HC = (HB + 1) / 2;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-    const Lds L = Lds::of(d);
-    const int ts = L.ts, ss = L.ss;
-    _Float16* tile0 = reinterpret_cast<_Float16*>(lds);
-    _Float16* tile1 = tile0 + 16 * ts;
-    float* st = reinterpret_cast<float*>(tile1 + 16 * ts);
-    float* act = st + 16 * ss; // [2 steps][16 futures][2 axes]
-    const int lane = (int)threadIdx.x, r16 = lane & 15, g4 = lane >> 4;
-    const int agent = (int)blockIdx.x;
+    half8* W1 = reinterpret_cast<half8*>(lds);
+    const half8* W2 = W1 + HB * NC * 64;
+    const half8* W3 = W2 + HB * HC * 64;
+    const int fb = d.fb, frags = frag_count(HB, NC, fb) * 64, tables = table_count(HB, NC, fb);
+    float4v* b1 = reinterpret_cast<float4v*>(W1 + frags);
+    const float4v *b2 = b1 + 4 * HB, *b3 = b2 + 4 * HB, *shift = b3 + 4 * fb, *inscale = shift + 8 * NC, *scale = inscale + 8 * NC,
+                  *target = scale + 4 * fb, *weight = target + 4 * fb;
+    for (int i = (int)threadIdx.x; i < frags; i += 256) {
+        W1[i] = d.frags[i];
+    }
+    for (int i = (int)threadIdx.x; i < tables; i += 256) {
+        b1[i] = d.tables[i];
+    }
+    __syncthreads();
+    const int l = (int)(threadIdx.x & 63u), n = l & 15, g = l >> 4;
     const int F = d.F, H = d.horizon, K = d.samples;
-    const u64 base = noise_base(ids[agent], tick);
-    for (int t0 = (int)blockIdx.y * 16; t0 < K; t0 += 16 * (int)gridDim.y) {
-        for (int q = lane; q < 16 * F; q += 64) {
-            st[(q / F) * ss + q % F] = obs[(long long)agent * F + q % F];
-        }
-        float J = 0.0f; // lanes 0..15: future t0 + lane
-        for (int t = 0; t < H; ++t) {
-            if ((t & 1) == 0) {
-                const int row = (lane >> 1) & 15, axis = lane & 1, step = t + (lane >> 5), k = t0 + row;
-                if (step < H) {
-                    const float e = k == 0 ? 0.0f : gauss(base ^ ((u64)k << 24) ^ ((u64)step << 8) ^ (u64)axis);
-                    const float a = fminf(fmaxf(mean[((long long)agent * H + step) * 2 + axis] + sigma * e, -1.0f), 1.0f);
-                    act[lane] = a;
-                    acts[(((long long)agent * K + k) * H + step) * 2 + axis] = a;
+    const unsigned wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4u + (threadIdx.x >> 6)));
+    for (unsigned item = wave; item < items; item += gridDim.x * 4u) {
+        const long long agent = (long long)(item / per_agent);
+        const int k0 = (int)(item % per_agent) * 16 * Q;
+        const u64 base = noise_base(ids[agent], tick);
+        float4v st[Q][2 * NC];
+#pragma unroll
+        for (int b = 0; b < 2 * NC; ++b) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int f = 16 * b + 4 * g + r;
+                const float x = f < F ? obs[agent * F + f] : 0.0f;
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    st[q][b][r] = x;
                 }
             }
-            __syncthreads();
-            const float* at = act + 32 * (t & 1);
-            // the inputs (state, then action), normalised, in fp16; zero past them: lane l row l % 16, features l / 16,
-            // l / 16 + 4, ...
-            for (int f = g4; f < d.in_pad; f += 4) {
-                const float x = f < F ? st[r16 * ss + f] : (f < F + 2 ? at[r16 * 2 + f - F] : 0.0f);
-                tile0[r16 * ts + f] = (_Float16)(f < F + 2 ? (x - d.shift[f]) * d.inscale[f] : 0.0f);
-            }
-            __syncthreads();
-            layer(d, tile0, tile1, ts, d.in_pad, d.hid, d.W1, d.b1, false, st, ss, dt, lane);
-            __syncthreads();
-            layer(d, tile1, tile0, ts, d.hid, d.hid, d.W2, d.b2, false, st, ss, dt, lane);
-            __syncthreads();
-            layer(d, tile0, tile1, ts, d.hid, d.f_pad, d.W3, d.b3, true, st, ss, dt, lane);
-            __syncthreads();
-            // the step's cost: lane l the features l / 16, l / 16 + 4, ... of future l % 16, then the four lane groups
-            // added in a fixed order
-            float c = 0.0f;
-            for (int f = g4; f < F; f += 4) {
-                const float e = st[r16 * ss + f] - d.target[f];
-                c += d.weight[f] * e * e;
-            }
-            c += __shfl_xor(c, 16);
-            c += __shfl_xor(c, 32);
-            if (lane < 16) {
-                const float ax = at[lane * 2], ay = at[lane * 2 + 1];
-                J += c + d.action_weight * (ax * ax + ay * ay);
-            }
-            __syncthreads();
         }
-        if (lane < 16) {
-            cost[(long long)agent * K + t0 + lane] = J;
+        float J[Q] = {}, drawn = 0.0f;
+        for (int t = 0; t < H; ++t) {
+            asm volatile("" ::: "memory"); // what LDS holds is read again each step: kept in registers it would spill
+            if (Q == 2 || (t & 1) == 0) {
+                const int row = Q == 2 ? l >> 1 : (l >> 1) & 15, axis = l & 1, step = Q == 2 ? t : t + (l >> 5), k = k0 + row;
+                if (step < H) {
+                    const float e = k == 0 ? 0.0f : gauss(base ^ ((u64)k << 24) ^ ((u64)step << 8) ^ (u64)axis);
+                    drawn = fminf(fmaxf(mean[(agent * H + step) * 2 + axis] + sigma * e, -1.0f), 1.0f);
+                    if (k < K) {
+                        acts[((agent * H + step) * K + k) * 2 + axis] = drawn;
+                    }
+                }
+            }
+            float ax[Q], ay[Q];
+            half8 in[Q][NC];
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const int from = 2 * (16 * q + n) + (Q == 2 ? 0 : 32 * (t & 1));
+                ax[q] = __shfl(drawn, from);
+                ay[q] = __shfl(drawn, from + 1);
+            }
+            // the inputs (state, then action), normalised, in fp16; zero past them
+#pragma unroll
+            for (int b = 0; b < 2 * NC; ++b) {
+                const float4v sh = shift[4 * b + g], sc = inscale[4 * b + g];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int f = 16 * b + 4 * g + r;
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) {
+                        const float x = f < F ? st[q][b][r] : (f == F ? ax[q] : (f == F + 1 ? ay[q] : 0.0f));
+                        in[q][b >> 1][4 * (b & 1) + r] = (_Float16)((x - sh[r]) * sc[r]);
+                    }
+                }
+            }
+            half8 h[Q][HC];
+            float4v z[Q][HB];
+#pragma unroll
+            for (int ob = 0; ob < HB; ++ob) {
+                const float4v bias = b1[4 * ob + g];
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    z[q][ob] = bias;
+                }
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    const half8 w = W1[(ob * NC + c) * 64 + l];
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) {
+                        z[q][ob] = mfma(w, in[q][c], z[q][ob]);
+                    }
+                }
+            }
+            activate<HB, Q>(z, h);
+            asm volatile("" ::: "memory");
+#pragma unroll
+            for (int ob = 0; ob < HB; ++ob) {
+                const float4v bias = b2[4 * ob + g];
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    z[q][ob] = bias;
+                }
+#pragma unroll
+                for (int c = 0; c < HC; ++c) {
+                    const half8 w = W2[(ob * HC + c) * 64 + l];
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) {
+                        z[q][ob] = mfma(w, h[q][c], z[q][ob]);
+                    }
+                }
+            }
+            activate<HB, Q>(z, h);
+            asm volatile("" ::: "memory");
+            // the rates, the states they move, and the states' part of the step's cost
+            float c[Q] = {};
+#pragma unroll
+            for (int b = 0; b < 2 * NC; ++b) {
+                if (b < fb) {
+                    const float4v bias = b3[4 * b + g], sc = scale[4 * b + g], to = target[4 * b + g], wt = weight[4 * b + g];
+                    float4v v[Q];
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) {
+                        v[q] = bias;
+                    }
+#pragma unroll
+                    for (int k = 0; k < HC; ++k) {
+                        const half8 w = W3[(b * HC + k) * 64 + l];
+#pragma unroll
+                        for (int q = 0; q < Q; ++q) {
+                            v[q] = mfma(w, h[q][k], v[q]);
+                        }
+                    }
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) {
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            st[q][b][r] += dt * v[q][r] * sc[r];
+                            const float e = st[q][b][r] - to[r];
+                            c[q] += wt[r] * e * e;
+                        }
+                    }
+                }
+            }
+            // the four lane groups' features added in a fixed order
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                c[q] += __shfl_xor(c[q], 16);
+                c[q] += __shfl_xor(c[q], 32);
+                J[q] += c[q] + d.action_weight * (ax[q] * ax[q] + ay[q] * ay[q]);
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int k = k0 + 16 * q + n;
+            if (g == 0 && k < K) {
+                cost[agent * K + k] = J[q];
+            }
         }
     }
 }
 
-// The new plan: a thread an (step, axis); the futures' actions weighted by exp(-(J - J_min) / lambda), lambda a quarter
-// of (mean cost - least cost), at least 1e-4, summed in the futures' order. The least cost, the sum of costs (in order)
-// and each future's weight are found once a block (in LDS) instead of by every thread.
+// The new plan: the futures' actions weighted by exp(-(J - J_min) / lambda), lambda a quarter of (mean cost - least cost), at
+// least 1e-4. A block an agent: the least cost, the costs' sum and each future's weight once (in LDS), then a wave a step:
+// lane l the axis l % 2 of the futures l / 2, l / 2 + 32, ..., and the lanes of an axis in a fixed tree.
 constexpr int kMaxSamples = 1024;
-__global__ void k_mppi_update(const float* __restrict__ cost, const float* __restrict__ acts, float* __restrict__ mean, int K, int H)
+constexpr int kUpdateWaves = 16;
+__global__ __launch_bounds__(64 * kUpdateWaves) void k_mppi_update(const float* __restrict__ cost, const float* __restrict__ acts,
+    float* __restrict__ mean, int K, int H)
 {
     __shared__ float cs[kMaxSamples];
-    __shared__ float lo_s, lam_s;
-    const int agent = (int)blockIdx.x, q = (int)threadIdx.x;
-    const float* c = cost + (long long)agent * K;
-    for (int k = q; k < K; k += (int)blockDim.x) {
-        cs[k] = c[k];
+    __shared__ float lows[kUpdateWaves], sums[kUpdateWaves];
+    const long long agent = (long long)blockIdx.x;
+    const int q = (int)threadIdx.x, l = q & 63, w = q >> 6;
+    static_assert(kMaxSamples == 64 * kUpdateWaves, "a thread a future");
+    const float c = cost[agent * K + (q < K ? q : 0)];
+    float lo = c, sum = q < K ? c : 0.0f;
+    for (int m = 32; m > 0; m >>= 1) {
+        lo = fminf(lo, __shfl_xor(lo, m));
+        sum += __shfl_xor(sum, m);
+    }
+    if (l == 0) {
+        lows[w] = lo;
+        sums[w] = sum;
     }
     __syncthreads();
-    if (q == 0) {
-        float lo = cs[0], sum = 0.0f;
-#pragma unroll 8
-        for (int k = 0; k < K; ++k) { // eight reads in flight, added in order
-            lo = fminf(lo, cs[k]);
-            sum += cs[k];
+    lo = lows[0];
+    sum = sums[0];
+    for (int i = 1; i < kUpdateWaves; ++i) {
+        lo = fminf(lo, lows[i]);
+        sum += sums[i];
+    }
+    const float lam = fmaxf(1e-4f, 0.25f * (sum / (float)K - lo));
+    cs[q] = q < K ? expf(-(c - lo) / lam) : 0.0f;
+    __syncthreads();
+    for (int t = w; t < H; t += kUpdateWaves) {
+        const float* a = acts + (agent * H + t) * 2 * K;
+        float wsum = 0.0f, acc = 0.0f;
+#pragma unroll 4
+        for (int i = l; i < 2 * K; i += 64) {
+            const float wk = cs[i >> 1];
+            wsum += wk;
+            acc += wk * a[i];
         }
-        lo_s = lo;
-        lam_s = fmaxf(1e-4f, 0.25f * (sum / (float)K - lo));
+        for (int m = 32; m > 1; m >>= 1) {
+            wsum += __shfl_xor(wsum, m);
+            acc += __shfl_xor(acc, m);
+        }
+        if (l < 2) {
+            mean[(agent * H + t) * 2 + l] = acc / wsum;
+        }
     }
-    __syncthreads();
-    const float lo = lo_s, lam = lam_s;
-    for (int k = q; k < K; k += (int)blockDim.x) {
-        cs[k] = expf(-(cs[k] - lo) / lam);
-    }
-    __syncthreads();
-    if (q >= 2 * H) {
-        return;
-    }
-    float wsum = 0.0f, acc = 0.0f;
-#pragma unroll 8
-    for (int k = 0; k < K; ++k) { // eight loads in flight, added in order
-        const float wk = cs[k];
-        wsum += wk;
-        acc += wk * acts[((long long)agent * K + k) * 2 * H + q];
-    }
-    mean[(long long)agent * 2 * H + q] = acc / wsum;
 }
 
 void hcheck(hipError_t e, const char* what)
@@ -272,35 +361,46 @@ struct Dev {
     }
 };
 
-int pad16(int v) { return (v + 15) / 16 * 16; }
+} // namespace
+
+using Rollout = void (*)(Desc, const float*, const float*, const unsigned*, float*, float*, u64, float, float, unsigned, unsigned);
+
+namespace {
+
+template <int NC, int Q>
+Rollout rollout_of(int HB)
+{
+    static constexpr Rollout by_hidden[] = {k_mppi_rollout<1, NC, Q>, k_mppi_rollout<2, NC, Q>, k_mppi_rollout<3, NC, Q>,
+        k_mppi_rollout<4, NC, Q>, k_mppi_rollout<5, NC, Q>, k_mppi_rollout<6, NC, Q>, k_mppi_rollout<7, NC, Q>, k_mppi_rollout<8, NC, Q>};
+    static_assert(sizeof by_hidden / sizeof *by_hidden == kMaxWidth / 16, "every hidden width");
+    return by_hidden[HB - 1];
+}
 
 } // namespace
 
 struct fe_mppi {
-    int F = 0, hid = 0, horizon = 0, samples = 0, in_pad = 0, f_pad = 0, cus = 0;
+    int F = 0, hid = 0, horizon = 0, samples = 0, HB = 0, NC = 0, fb = 0, lds = 0, cus = 1;
+    Rollout rollout[2] = {};  // one, two tiles a wave
+    int resident[2] = {1, 1}; // their waves the card holds at once
     bool dynamics = false, costed = false;
-    Dev<_Float16> W1, W2, W3;
-    Dev<float> b1, b2, b3, shift, inscale, scale, target, weight;
+    Dev<half8> frags;
+    Dev<float> tables;
+    std::vector<float> host_tables;
     float action_weight = 0.0f;
     Dev<float> obs, mean, acts, cost;
     Dev<unsigned> ids;
     std::string error;
+    // where the tables begin, in floats
+    int b2() const { return hid; }
+    int b3() const { return 2 * hid; }
+    int shift() const { return b3() + 16 * fb; }
+    int inscale() const { return shift() + 32 * NC; }
+    int scale() const { return inscale() + 32 * NC; }
+    int target() const { return scale() + 16 * fb; }
+    int weight() const { return target() + 16 * fb; }
 };
 
 namespace {
-
-// Blocks an agent's futures spread over: one tile of 16 a block while every tile's block fits the card at once; past
-// that each block walks a few tiles in turn, so the launch is one round (a second, part-filled round of one-tile
-// blocks took longer than the first: 824 against 777 us for 256 agents x 512 futures). A CU holds as many blocks as
-// its 160 KB of LDS allows, at most 28 (seven waves a SIMD at the rollout's registers).
-int rollout_parts(const fe_mppi& p, const Desc& d, int agents)
-{
-    const int tiles = p.samples / 16;
-    const int per_cu = std::min(160 * 1024 / Lds::of(d).bytes(), 28);
-    const long long fit = static_cast<long long>(std::max(p.cus, 1)) * per_cu;
-    const long long rounds = (static_cast<long long>(agents) * tiles + fit - 1) / fit;
-    return static_cast<int>((tiles + rounds - 1) / rounds);
-}
 
 int fail(fe_mppi* p, const std::string& what)
 {
@@ -310,23 +410,19 @@ int fail(fe_mppi* p, const std::string& what)
     return -1;
 }
 
-// W[out][in] (row-major, fp32) into a zero-padded fp16 [out_pad][in_pad].
-std::vector<_Float16> pack(const float* w, int out, int in, int out_pad, int in_pad)
+// W[out][in] (row-major, fp32) as fragments: blocks of 16 outputs by 32 inputs, zero past both.
+void pack(std::vector<_Float16>& to, const float* w, int out, int in, int blocks, int chunks)
 {
-    std::vector<_Float16> h(static_cast<std::size_t>(out_pad) * in_pad, static_cast<_Float16>(0.0f));
-    for (int o = 0; o < out; ++o) {
-        for (int i = 0; i < in; ++i) {
-            h[static_cast<std::size_t>(o) * in_pad + i] = static_cast<_Float16>(w[static_cast<std::size_t>(o) * in + i]);
+    for (int ob = 0; ob < blocks; ++ob) {
+        for (int c = 0; c < chunks; ++c) {
+            for (int l = 0; l < 64; ++l) {
+                for (int e = 0; e < 8; ++e) {
+                    const int o = 16 * ob + l % 16, i = kfeat(c, l / 16, e);
+                    to.push_back(static_cast<_Float16>(o < out && i < in ? w[static_cast<std::size_t>(o) * in + i] : 0.0f));
+                }
+            }
         }
     }
-    return h;
-}
-
-std::vector<float> padded(const float* v, int n, int to, float fill = 0.0f)
-{
-    std::vector<float> out(static_cast<std::size_t>(to), fill);
-    std::copy(v, v + n, out.begin());
-    return out;
 }
 
 } // namespace
@@ -351,13 +447,28 @@ fe_mppi* fe_mppi_create(int features, int hidden, int horizon, int samples, char
         return nullptr;
     }
     auto p = std::make_unique<fe_mppi>();
-    p->cus = info.compute_units;
+    p->cus = std::max(info.compute_units, 1);
     p->F = features;
     p->hid = hidden;
     p->horizon = horizon;
     p->samples = samples;
-    p->in_pad = pad16(features + 2);
-    p->f_pad = pad16(features);
+    p->HB = hidden / 16;
+    p->NC = (features + 2 + 31) / 32;
+    p->fb = (features + 15) / 16;
+    p->lds = lds_bytes(p->HB, p->NC, p->fb);
+    p->rollout[0] = p->NC == 1 ? rollout_of<1, 1>(p->HB) : rollout_of<2, 1>(p->HB);
+    p->rollout[1] = p->NC == 1 ? rollout_of<1, 2>(p->HB) : rollout_of<2, 2>(p->HB);
+    for (int q = 0; q < 2; ++q) {
+        int blocks = 0;
+        const void* k = reinterpret_cast<const void*>(p->rollout[q]);
+        if ((p->lds > 64 * 1024 && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, p->lds) != hipSuccess) ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, k, 256, static_cast<std::size_t>(p->lds)) != hipSuccess || blocks < 1) {
+            say("the rollout does not fit the card");
+            return nullptr;
+        }
+        p->resident[q] = 4 * blocks * p->cus;
+    }
+    p->host_tables.assign(static_cast<std::size_t>(4 * table_count(p->HB, p->NC, p->fb)), 0.0f);
     return p.release();
 }
 
@@ -377,17 +488,21 @@ int fe_mppi_set_dynamics(fe_mppi* p, const float* weights, const float* in_shift
         const float* b2 = w2 + static_cast<std::size_t>(Hd) * Hd;
         const float* w3 = b2 + Hd;
         const float* b3 = w3 + static_cast<std::size_t>(Hd) * F;
-        const std::vector<_Float16> h1 = pack(w1, Hd, I, Hd, p->in_pad), h2 = pack(w2, Hd, Hd, Hd, Hd), h3 = pack(w3, F, Hd, p->f_pad, Hd);
-        p->W1.put(h1.data(), h1.size());
-        p->W2.put(h2.data(), h2.size());
-        p->W3.put(h3.data(), h3.size());
-        const std::vector<float> pb3 = padded(b3, F, p->f_pad), sh = padded(in_shift, I, p->in_pad), sc = padded(in_scale, I, p->in_pad);
-        p->b1.put(b1, static_cast<std::size_t>(Hd));
-        p->b2.put(b2, static_cast<std::size_t>(Hd));
-        p->b3.put(pb3.data(), pb3.size());
-        p->shift.put(sh.data(), sh.size());
-        p->inscale.put(sc.data(), sc.size());
-        p->scale.put(scale, static_cast<std::size_t>(F));
+        std::vector<_Float16> packed;
+        packed.reserve(static_cast<std::size_t>(frag_count(p->HB, p->NC, p->fb)) * 512);
+        const int HC = (p->HB + 1) / 2;
+        pack(packed, w1, Hd, I, p->HB, p->NC);
+        pack(packed, w2, Hd, Hd, p->HB, HC);
+        pack(packed, w3, F, Hd, p->fb, HC);
+        p->frags.put(reinterpret_cast<const half8*>(packed.data()), packed.size() / 8);
+        float* to = p->host_tables.data();
+        std::copy(b1, b1 + Hd, to);
+        std::copy(b2, b2 + Hd, to + p->b2());
+        std::copy(b3, b3 + F, to + p->b3());
+        std::copy(in_shift, in_shift + I, to + p->shift());
+        std::copy(in_scale, in_scale + I, to + p->inscale());
+        std::copy(scale, scale + F, to + p->scale());
+        p->tables.put(to, p->host_tables.size());
         p->dynamics = true;
         return 0;
     } catch (const std::exception& e) {
@@ -401,8 +516,9 @@ int fe_mppi_set_cost(fe_mppi* p, const float* target, const float* weight, float
         return fail(p, "invalid arguments");
     }
     try {
-        p->target.put(target, static_cast<std::size_t>(p->F));
-        p->weight.put(weight, static_cast<std::size_t>(p->F));
+        std::copy(target, target + p->F, p->host_tables.data() + p->target());
+        std::copy(weight, weight + p->F, p->host_tables.data() + p->weight());
+        p->tables.put(p->host_tables.data(), p->host_tables.size());
         p->action_weight = action_weight;
         p->costed = true;
         return 0;
@@ -422,21 +538,29 @@ int fe_mppi_plan(fe_mppi* p, int agents, const float* obs, const uint32_t* ids, 
     }
     try {
         const int F = p->F, H = p->horizon, K = p->samples;
+        const long long tiles = static_cast<long long>(agents) * (K / 16);
+        // Two tiles a wave share the weights' reads and hide each other's latency, once there are three a SIMD: hidden 64,
+        // 128 and 16 take 208, 286, 125 us against one tile's 218, 315, 126 at four a SIMD, 328, 495, 166 against 341, 558,
+        // 176 at eight; at two they are even (151, 199, 104 against 151, 199, 100), and a lone agent takes 129 against 111.
+        const int two = tiles >= 12LL * p->cus && K > 16 ? 1 : 0;
+        const unsigned per_agent = static_cast<unsigned>((K / 16 + two) / (1 + two));
+        const long long items = static_cast<long long>(agents) * per_agent;
+        if (items >= 4294967296LL - 2097152) { // the kernel's index, and its stride past the end; their actions would be 550 GB
+            return fail(p, "too many agents for one plan");
+        }
+        // one round of blocks, each wave as many items as any other, where more of them would start a second round
+        const long long rounds = (items + p->resident[two] - 1) / p->resident[two];
+        const long long waves = (items + rounds - 1) / rounds;
         const hipStream_t s = static_cast<hipStream_t>(fe_hip_stream());
         p->obs.put(obs, static_cast<std::size_t>(agents) * F);
         p->ids.put(ids, static_cast<std::size_t>(agents));
         p->mean.put(mean, static_cast<std::size_t>(agents) * H * 2);
         p->acts.alloc(static_cast<std::size_t>(agents) * K * H * 2);
         p->cost.alloc(static_cast<std::size_t>(agents) * K);
-        Desc d{F, p->in_pad, p->hid, p->f_pad, H, K, p->W1.p, p->W2.p, p->W3.p, p->b1.p, p->b2.p, p->b3.p, p->shift.p, p->inscale.p,
-            p->scale.p, p->target.p, p->weight.p, p->action_weight};
-        // a block is one wave (its barriers wait for no other wave), an agent's futures spread over samples / 16 blocks
-        hipLaunchKernelGGL(k_mppi_rollout, dim3(static_cast<unsigned>(agents), static_cast<unsigned>(rollout_parts(*p, d, agents))), dim3(64),
-            static_cast<unsigned>(Lds::of(d).bytes()), s,
-            d, p->obs.p, p->mean.p, p->ids.p,
-            p->acts.p, p->cost.p, static_cast<unsigned long long>(tick), sigma, dt);
-        hipLaunchKernelGGL(k_mppi_update, dim3(static_cast<unsigned>(agents)), dim3(static_cast<unsigned>(pad16(2 * H))), 0, s, p->cost.p,
-            p->acts.p, p->mean.p, K, H);
+        const Desc d{F, p->fb, H, K, p->frags.p, reinterpret_cast<const float4v*>(p->tables.p), p->action_weight};
+        hipLaunchKernelGGL(p->rollout[two], dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), static_cast<unsigned>(p->lds), s, d, p->obs.p,
+            p->mean.p, p->ids.p, p->acts.p, p->cost.p, static_cast<unsigned long long>(tick), sigma, dt, static_cast<unsigned>(items), per_agent);
+        hipLaunchKernelGGL(k_mppi_update, dim3(static_cast<unsigned>(agents)), dim3(64 * kUpdateWaves), 0, s, p->cost.p, p->acts.p, p->mean.p, K, H);
         hcheck(hipGetLastError(), "mppi launch");
         hcheck(hipMemcpyAsync(mean, p->mean.p, sizeof(float) * static_cast<std::size_t>(agents) * H * 2, hipMemcpyDeviceToHost, s), "download");
         if (cost_out != nullptr) {

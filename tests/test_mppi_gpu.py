@@ -41,6 +41,30 @@ def test_plan_matches_the_oracle_and_repeats(device):
     assert not np.array_equal(got, other)  # another tick, other noise
 
 
+@pytest.mark.parametrize("features,hidden,samples,agents,horizon", [
+    (1, 16, 16, 1, 1), (14, 48, 48, 3, 5), (15, 64, 32, 2, 4), (30, 128, 48, 2, 3), (31, 112, 16, 2, 3), (62, 80, 64, 1, 2),
+    (62, 128, 48, 2731, 2), (16, 64, 48, 2731, 3)])
+def test_every_net_shape_matches_the_oracle(device, features, hidden, samples, agents, horizon):
+    """Blocks of 16 features and hidden units that the net fills in part, the actions in every place of a fragment of 32
+    inputs, an odd horizon (the noise of two steps drawn at once), and two tiles a wave with one past the last future."""
+    import field_hip
+
+    p = mppi.make_params(features, hidden, 21)
+    rng = np.random.default_rng(features * 1000 + hidden)
+    obs = rng.uniform(-1, 1, (agents, features)).astype(np.float32)
+    ids = np.arange(agents, dtype=np.uint32) * 7 + 3
+    mean = rng.uniform(-0.3, 0.3, (agents, horizon, 2)).astype(np.float32)
+    pl = field_hip.MppiPlanner(features, hidden, horizon, samples)
+    pl.set_dynamics(p["flat"], p["shift"], p["inscale"], p["scale"])
+    pl.set_cost(p["target"], p["weight"], p["action_weight"])
+    got, costs = pl.plan(obs, ids, mean, tick=12, sigma=0.3, dt=0.1, costs=True)
+    some = sorted({0, agents // 2, agents - 1})
+    want, wcost = mppi.plan(p, obs[some].astype(np.float64), ids[some], mean[some].astype(np.float64), 12, 0.3, 0.1, samples)
+    rel = np.abs(costs[some] - wcost) / np.maximum(np.abs(wcost), 1e-3)
+    assert rel.max() < 2e-3, rel.max()
+    assert np.max(np.abs(got[some] - want)) < 2e-3, np.max(np.abs(got[some] - want))
+
+
 def test_planning_lowers_the_plans_cost(device):
     """Planning repeatedly from where it left off: the plan's own cost (future 0) falls."""
     import field_hip
