@@ -34,6 +34,9 @@ constexpr int kChunk = 32;      // blocks' partials summed together in the first
 constexpr int kOneLevel = 64;   // up to this many blocks their partials are added in one level
 constexpr int kBlocks = 1024;   // the most blocks a pass (four blocks of four waves a CU)
 constexpr int kMaxLds = 65536;  // bytes of LDS a block may use
+// A product's steps of 4 whose loads are in flight together: a weight's read is the chain's longest wait. 4 of them: 1024 rows
+// take 69 us a step (with the copies), 16: 46.8 and spills, 8: 43 and the most rows that fill the card 405 against 422.
+constexpr int kDepth = 8;
 constexpr int kWaves = 4;       // waves a block: a tile's 16-column blocks spread over them
 
 struct Shape {
@@ -55,7 +58,7 @@ struct Shape {
 __host__ __device__ inline int pad16(int v) { return (v + 15) / 16 * 16; }
 
 // An input row's stride in LDS: padded to 16 (a product's depth goes 16 at a time, four steps of 4 whose loads are
-// issued together; the padding stays zero) plus 1, so the 16 rows a product reads at once fall in different banks.
+// taken or left together; the padding stays zero) plus 1, so the 16 rows a product reads at once fall in different banks.
 __host__ __device__ inline int a_ld(int n) { return pad16(n) + 1; }
 
 // The activations through the hardware base-2 exponential and reciprocal (v_exp_f32, v_rcp_f32, a few ulp of fp32;
@@ -107,7 +110,7 @@ __device__ __forceinline__ float act_d(int a, float x)
 // thread adds to the same elements for every tile, so the order is fixed). The four waves share a tile: each product's
 // 16-column blocks (or the weight gradient's 16 x 16 blocks) go round the waves. LDS: s.lds floats (the launch gives
 // them).
-__global__ __launch_bounds__(64 * kWaves) void k_nt_tile(Shape s, const float* __restrict__ w, const float* __restrict__ X,
+__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4))) void k_nt_tile(Shape s, const float* __restrict__ w, const float* __restrict__ X,
     const float* __restrict__ T, const float* __restrict__ M, int rows, float* __restrict__ partial)
 {
     extern __shared__ __attribute__((aligned(16))) float sh[];
@@ -130,6 +133,11 @@ __global__ __launch_bounds__(64 * kWaves) void k_nt_tile(Shape s, const float* _
             const int r = q / in, i = q % in, row = r0 + r;
             a0[r * ld0 + i] = row < rows ? (X[(long long)row * in + i] - w[i]) * w[in + i] : 0.0f;
         }
+        float* t0 = sh + s.d_at[1]; // the targets, until the deltas below the last layer take their place
+        for (int q = tid; q < kRows * out; q += 64 * kWaves) {
+            const int r = q / out, i = q % out, row = r0 + r;
+            t0[r * dl + i] = row < rows ? T[(long long)row * out + i] : 0.0f;
+        }
         __syncthreads();
         for (int k = 0; k < s.layers; ++k) {
             const int ni = s.sizes[k], no = s.sizes[k + 1], ni16 = pad16(ni), la = a_ld(ni), lo = a_ld(no);
@@ -140,16 +148,19 @@ __global__ __launch_bounds__(64 * kWaves) void k_nt_tile(Shape s, const float* _
             for (int nb = 16 * wave; nb < no; nb += 16 * kWaves) {
                 const int col = nb + c16;
                 float4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
-                for (int kc = 0; kc < ni16; kc += 16) {
-                    float av[4], bv[4];
+                for (int kc = 0; kc < ni16; kc += 4 * kDepth) {
+                    float av[kDepth], bv[kDepth];
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
+                    for (int u = 0; u < kDepth; ++u) {
                         const int kk = kc + 4 * u + g4;
-                        av[u] = A[c16 * la + kk];
+                        av[u] = kk < ni16 ? A[c16 * la + kk] : 0.0f;
                         bv[u] = col < no && kk < ni ? W[(long long)col * ni + kk] : 0.0f;
                     }
 #pragma unroll
-                    for (int u = 0; u < 4; ++u) {
+                    for (int u = 0; u < kDepth; ++u) {
+                        if (u % 4 == 0 && kc + 4 * u >= ni16) {
+                            break;
+                        }
                         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u], bv[u], acc, 0, 0, 0);
                     }
                 }
@@ -165,7 +176,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_nt_tile(Shape s, const float* _
                             float d = 0.0f;
                             if (row < rows) {
                                 const float m = M != nullptr ? M[row] : 1.0f;
-                                const float e = pre * scale - T[(long long)row * out + col];
+                                const float e = pre * scale - t0[r * dl + col];
                                 loss += 0.5f * m * e * e;
                                 d = m * e * scale;
                             }
@@ -221,16 +232,19 @@ __global__ __launch_bounds__(64 * kWaves) void k_nt_tile(Shape s, const float* _
                 for (int ib = 16 * wave; ib < ni; ib += 16 * kWaves) {
                     const int i = ib + c16;
                     float4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
-                    for (int oc = 0; oc < no16; oc += 16) {
-                        float av[4], bv[4];
+                    for (int oc = 0; oc < no16; oc += 4 * kDepth) {
+                        float av[kDepth], bv[kDepth];
 #pragma unroll
-                        for (int u = 0; u < 4; ++u) {
+                        for (int u = 0; u < kDepth; ++u) {
                             const int o = oc + 4 * u + g4;
                             av[u] = o < no ? D[c16 * dl + o] : 0.0f;
                             bv[u] = o < no && i < ni ? W[(long long)o * ni + i] : 0.0f;
                         }
 #pragma unroll
-                        for (int u = 0; u < 4; ++u) {
+                        for (int u = 0; u < kDepth; ++u) {
+                            if (u % 4 == 0 && oc + 4 * u >= no16) {
+                                break;
+                            }
                             acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[u], bv[u], acc, 0, 0, 0);
                         }
                     }
@@ -299,8 +313,9 @@ __device__ __forceinline__ void adam_at(const Adam& a, int p, float grad)
 }
 
 // Last level: `count` rows of partial sums (the blocks' own, or the chunks') added in order, divided by the rows (the
-// mean; the last column is the loss), and, when adam.n > 0, the Adam step on each weight and bias with its mean.
-__global__ void k_nt_fold(const float* __restrict__ sums, int count, int width, float rows_f, float* __restrict__ grad, Adam adam)
+// mean; the last column is the loss, which goes to the host's memory too), and, when adam.n > 0, the Adam step on each weight and bias with its mean.
+__global__ void k_nt_fold(const float* __restrict__ sums, int count, int width, float rows_f, float* __restrict__ grad, Adam adam,
+    float* __restrict__ loss)
 {
     const int c = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (c < width) {
@@ -311,6 +326,9 @@ __global__ void k_nt_fold(const float* __restrict__ sums, int count, int width, 
         }
         const float g = s / rows_f;
         grad[c] = g;
+        if (c == width - 1) {
+            *loss = g;
+        }
         if (c < adam.n) {
             adam_at(adam, c, g);
         }
@@ -356,6 +374,39 @@ struct Dev {
     }
 };
 
+// Host memory the card reads and writes in place.
+struct Pinned {
+    float* p = nullptr;
+    std::size_t n = 0;
+    Pinned() = default;
+    Pinned(const Pinned&) = delete;
+    Pinned& operator=(const Pinned&) = delete;
+    ~Pinned()
+    {
+        if (p != nullptr) {
+            (void)hipHostFree(p);
+        }
+    }
+    void alloc(std::size_t count)
+    {
+        if (count <= n) {
+            return;
+        }
+        if (p != nullptr) {
+            hcheck(hipHostFree(p), "free");
+            p = nullptr;
+            n = 0;
+        }
+        hcheck(hipHostMalloc(reinterpret_cast<void**>(&p), count * sizeof(float), hipHostMallocDefault), "pinned allocation");
+        n = count;
+    }
+};
+
+// Rows, targets and row weights of at most this many floats are read by the pass itself from pinned host memory (each once),
+// where two copies of pageable memory and the loss's way back cost a step 25 us beside its kernels' 27 (1024 rows of 18 + 16
+// floats; 69 -> 43 us a step, 2048 rows 72 -> 47); past that the copy's rate counts and the rows are uploaded as before.
+constexpr std::size_t kStaged = 131072;
+
 unsigned blocks_for(long long n, int per) { return static_cast<unsigned>((n + per - 1) / per); }
 
 } // namespace
@@ -363,22 +414,23 @@ unsigned blocks_for(long long n, int per) { return static_cast<unsigned>((n + pe
 struct fe_nettrain {
     Shape s;
     Dev<float> w, m1, m2, x, t, m, partial, chunks, grad;
+    Pinned staged, loss;         // every call waits for its pass before it returns, so the next may write them
+    const float *rx = nullptr, *rt = nullptr, *rm = nullptr; // the pass's rows, targets and row weights
     int adam_t = 0;
     std::string error;
     hipStream_t stream() const { return static_cast<hipStream_t>(fe_hip_stream()); }
-    const float* loss() const { return grad.p + s.trained; }
 
     // The gradient and loss for the rows already uploaded; leaves the mean gradient in grad[0, trained), the mean loss
     // in grad[trained], and takes the Adam step when adam.n > 0. Up to kOneLevel blocks their partials are added in one
     // level, past it in chunks of kChunk first.
-    void gradient(int rows, bool masked, const Adam& adam)
+    void gradient(int rows, const Adam& adam)
     {
         const hipStream_t st = stream();
         const int blocks = std::min((rows + kRows - 1) / kRows, kBlocks), width = s.trained + 1;
         partial.alloc(static_cast<std::size_t>(blocks) * width);
         grad.alloc(static_cast<std::size_t>(width));
-        hipLaunchKernelGGL(k_nt_tile, dim3(static_cast<unsigned>(blocks)), dim3(64 * kWaves), static_cast<unsigned>(s.lds) * 4u, st, s, w.p, x.p,
-            t.p, masked ? m.p : nullptr, rows, partial.p);
+        hipLaunchKernelGGL(k_nt_tile, dim3(static_cast<unsigned>(blocks)), dim3(64 * kWaves), static_cast<unsigned>(s.lds) * 4u, st, s, w.p, rx,
+            rt, rm, rows, partial.p);
         const float* sums = partial.p;
         int count = blocks;
         if (blocks > kOneLevel) {
@@ -388,18 +440,34 @@ struct fe_nettrain {
                 chunks.p);
             sums = chunks.p;
         }
-        hipLaunchKernelGGL(k_nt_fold, dim3(blocks_for(width, 256)), dim3(256), 0, st, sums, count, width, static_cast<float>(rows), grad.p, adam);
+        hipLaunchKernelGGL(k_nt_fold, dim3(blocks_for(width, 256)), dim3(256), 0, st, sums, count, width, static_cast<float>(rows), grad.p, adam,
+            loss.p);
         hcheck(hipGetLastError(), "gradient launch");
     }
 
     void upload(const float* xs, const float* ts, const float* ms, int rows)
     {
         const hipStream_t st = stream();
-        x.put(xs, static_cast<std::size_t>(rows) * s.sizes[0], st);
-        t.put(ts, static_cast<std::size_t>(rows) * s.sizes[s.layers], st);
-        if (ms != nullptr) {
-            m.put(ms, static_cast<std::size_t>(rows), st);
+        const std::size_t nr = static_cast<std::size_t>(rows), nx = nr * s.sizes[0], nt = nr * s.sizes[s.layers];
+        if (nx + nt + nr <= kStaged) {
+            std::memcpy(staged.p, xs, nx * sizeof(float));
+            std::memcpy(staged.p + nx, ts, nt * sizeof(float));
+            if (ms != nullptr) {
+                std::memcpy(staged.p + nx + nt, ms, nr * sizeof(float));
+            }
+            rx = staged.p;
+            rt = rx + nx;
+            rm = ms != nullptr ? rt + nt : nullptr;
+            return;
         }
+        x.put(xs, nx, st);
+        t.put(ts, nt, st);
+        if (ms != nullptr) {
+            m.put(ms, nr, st);
+        }
+        rx = x.p;
+        rt = t.p;
+        rm = ms != nullptr ? m.p : nullptr;
     }
 };
 
@@ -476,6 +544,8 @@ fe_nettrain* fe_nettrain_create(const int* sizes, int count, int act, char* why,
         }
         image[static_cast<std::size_t>(2 * sizes[0])] = 1.0f;
         t->w.put(image.data(), image.size(), t->stream());
+        t->staged.alloc(kStaged);
+        t->loss.alloc(1);
         std::vector<float> zeros(static_cast<std::size_t>(s.trained), 0.0f);
         t->m1.put(zeros.data(), zeros.size(), t->stream());
         t->m2.put(zeros.data(), zeros.size(), t->stream());
@@ -534,19 +604,18 @@ int fe_nettrain_gradient(fe_nettrain* t, const float* x, const float* target, co
     }
     try {
         t->upload(x, target, m, rows);
-        t->gradient(rows, m != nullptr, Adam{});
+        t->gradient(rows, Adam{});
         const hipStream_t st = t->stream();
         if (grad != nullptr) {
             hcheck(hipMemcpyAsync(grad, t->grad.p, sizeof(float) * static_cast<std::size_t>(t->s.trained), hipMemcpyDeviceToHost, st), "download");
         }
-        float l = 0.0f;
-        hcheck(hipMemcpyAsync(&l, t->loss(), sizeof(float), hipMemcpyDeviceToHost, st), "download");
         hcheck(hipStreamSynchronize(st), "sync");
         if (loss != nullptr) {
-            *loss = l;
+            *loss = *t->loss.p;
         }
         return 0;
     } catch (const std::exception& e) {
+        (void)hipStreamSynchronize(t->stream()); // what was launched reads the staged rows
         return fail(t, e.what());
     }
 }
@@ -562,17 +631,16 @@ int fe_nettrain_step(fe_nettrain* t, const float* x, const float* target, const 
         const int step = t->adam_t + 1;
         const float c1 = 1.0f - std::pow(b1, static_cast<float>(step));
         const float c2 = 1.0f - std::pow(b2, static_cast<float>(step));
-        t->gradient(rows, m != nullptr, Adam{t->w.p + t->s.base, t->m1.p, t->m2.p, t->s.trained, lr, b1, b2, c1, c2, clip});
+        t->gradient(rows, Adam{t->w.p + t->s.base, t->m1.p, t->m2.p, t->s.trained, lr, b1, b2, c1, c2, clip});
         t->adam_t = step;
         const hipStream_t st = t->stream();
-        float l = 0.0f;
-        hcheck(hipMemcpyAsync(&l, t->loss(), sizeof(float), hipMemcpyDeviceToHost, st), "download");
         hcheck(hipStreamSynchronize(st), "sync");
         if (loss != nullptr) {
-            *loss = l;
+            *loss = *t->loss.p;
         }
         return 0;
     } catch (const std::exception& e) {
+        (void)hipStreamSynchronize(t->stream()); // what was launched reads the staged rows
         return fail(t, e.what());
     }
 }

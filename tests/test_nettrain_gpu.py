@@ -169,3 +169,24 @@ def test_rows_weighted_zero_give_zero_and_adam_leaves_the_weights(device):
     assert loss == 0.0 and not np.any(g)
     tr.step(x, t, m)
     assert np.array_equal(tr.image().view(np.uint32), image.view(np.uint32))
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("rows", [1, 17, 3640, 3641, 3700])
+def test_staged_and_uploaded_rows_give_the_oracles_gradient(device, rows, masked):
+    """On both sides of the size up to which the rows are read from pinned host memory (20 + 15 + 1 floats a row), and two
+    calls in turn, the second's rows in the place of the first's. fp32 sums of 3700 rows: a few times 2^-24 sqrt(3700), 4e-6."""
+    import field_hip
+
+    sizes = [20, 37, 15]
+    image = nettrain.make_image(sizes, 5)
+    tr = field_hip.NetTrainer(sizes, "tanh")
+    tr.set_image(image.astype(np.float32))
+    for seed in (6, 7):
+        rng = np.random.default_rng(seed)
+        x, t = rng.standard_normal((rows, 20)).astype(np.float32), rng.standard_normal((rows, 15)).astype(np.float32)
+        m = rng.uniform(0, 2, rows).astype(np.float32) if masked else None
+        loss, g = tr.gradient(x, t, m)
+        want_loss, want = nettrain.gradient(sizes, "tanh", image.astype(np.float32), x, t, m)
+        assert abs(loss - want_loss) <= 1e-5 * want_loss
+        assert np.linalg.norm(g - want) <= 1e-5 * np.linalg.norm(want)
