@@ -712,7 +712,11 @@ struct fe_heston {
         bool col_lds = false;  // the column passes keep d' in LDS (k_cols_lds; 64 threads a block, ny_max <= 256)
         int col_part = 0;      // M > 0: the column passes partitioned, M rows a thread (k_cols_part; 64 x P threads)
         Dev<Task> row_tasks, col_tasks;
-        int n_row_tasks = 0, n_col_tasks = 0;
+        // Consecutive members stepped together, as ranges of the task tables.
+        struct Chunk {
+            int row0, row1, col0, col1;
+        };
+        std::vector<Chunk> chunks;
     };
     int n = 0;
     int steps = 0;
@@ -741,23 +745,40 @@ struct fe_heston {
 
     hipStream_t stream() const { return static_cast<hipStream_t>(fe_hip_stream()); }
 
+    // The members that take their steps together before the next ones begin. A pass reads what the one before wrote, three
+    // lattices of 4 bytes a cell: at 16M cells those are 192 MB, and part of each is still in the 256 MB last-level cache.
+    // 2048 options (three classes), 64 steps: 62.2 ms in one piece, 59.9 at 16M, 61 at 32M; at 8M and below the passes no
+    // longer fill the card (62.5 and more).
+    static constexpr long long kChunkCells = 1LL << 24;
+
     void build_tasks(Class& c)
     {
         std::vector<Task> rt, ct;
         const int rows_a_block = c.row_waves * (64 / c.lanes);
+        long long cells = 0, held = 0;
+        for (const int o : c.members) {
+            cells += 1LL * c.nx * host_opts[static_cast<std::size_t>(o)].ny;
+        }
+        const long long parts = (cells + kChunkCells - 1) / kChunkCells, most = parts > 0 ? (cells + parts - 1) / parts : 0;
+        c.chunks.clear();
         for (const int o : c.members) {
             const int ny = host_opts[static_cast<std::size_t>(o)].ny;
+            if (c.chunks.empty() || held >= most) {
+                c.chunks.push_back({static_cast<int>(rt.size()), 0, static_cast<int>(ct.size()), 0});
+                held = 0;
+            }
+            held += 1LL * c.nx * ny;
             for (int j = 0; j < ny; j += rows_a_block) {
                 rt.push_back({o, j});
             }
             for (int i = 0; i < c.nx; i += c.col_threads) {
                 ct.push_back({o, i});
             }
+            c.chunks.back().row1 = static_cast<int>(rt.size());
+            c.chunks.back().col1 = static_cast<int>(ct.size());
         }
         c.row_tasks.upload(rt);
         c.col_tasks.upload(ct);
-        c.n_row_tasks = static_cast<int>(rt.size());
-        c.n_col_tasks = static_cast<int>(ct.size());
     }
 
     static unsigned lds_bytes(const Class& c) { return static_cast<unsigned>(c.ny_max) * 64u * 4u; }
@@ -765,66 +786,68 @@ struct fe_heston {
     // The partitioned column passes: P = ceil(ny_max / M) waves a block (at most 16: 1024 threads).
     static int part_waves(const Class& c, int m) { return (c.ny_max + m - 1) / m; }
     static bool part_fits(const Class& c, int m) { return (m == 8 || m == 16) && c.ny_max >= 1 && part_waves(c, m) <= 16; }
-    void launch_cols_part(const Class& c, bool final_pass, hipStream_t s)
+    void launch_cols_part(const Class& c, const Class::Chunk& h, bool final_pass, hipStream_t s)
     {
         const int pw = part_waves(c, c.col_part);
         const dim3 block(64, static_cast<unsigned>(pw));
         const unsigned shm = 3u * static_cast<unsigned>(pw) * 64u * 4u;
-        const dim3 grid(static_cast<unsigned>(c.n_col_tasks));
+        const dim3 grid(static_cast<unsigned>(h.col1 - h.col0));
+        const Task* tasks = c.col_tasks.p + h.col0;
         if (c.col_part == 8) {
             if (final_pass) {
-                hipLaunchKernelGGL((k_cols_part<8, true>), grid, block, shm, s, opts.p, ptab.p, c.col_tasks.p, U.p, D2.p, T1.p);
+                hipLaunchKernelGGL((k_cols_part<8, true>), grid, block, shm, s, opts.p, ptab.p, tasks, U.p, D2.p, T1.p);
             } else {
-                hipLaunchKernelGGL((k_cols_part<8, false>), grid, block, shm, s, opts.p, ptab.p, c.col_tasks.p, U.p, D2.p, T1.p);
+                hipLaunchKernelGGL((k_cols_part<8, false>), grid, block, shm, s, opts.p, ptab.p, tasks, U.p, D2.p, T1.p);
             }
         } else if (final_pass) {
-            hipLaunchKernelGGL((k_cols_part<16, true>), grid, block, shm, s, opts.p, ptab.p, c.col_tasks.p, U.p, D2.p, T1.p);
+            hipLaunchKernelGGL((k_cols_part<16, true>), grid, block, shm, s, opts.p, ptab.p, tasks, U.p, D2.p, T1.p);
         } else {
-            hipLaunchKernelGGL((k_cols_part<16, false>), grid, block, shm, s, opts.p, ptab.p, c.col_tasks.p, U.p, D2.p, T1.p);
+            hipLaunchKernelGGL((k_cols_part<16, false>), grid, block, shm, s, opts.p, ptab.p, tasks, U.p, D2.p, T1.p);
         }
     }
 
-    void queue_step() { queue_step_of(-1); }
+    // `count` steps of every class, chunk by chunk.
+    void queue_steps(int count)
+    {
+        for (Class& c : classes) {
+            queue_class(c, count);
+        }
+    }
 
-    // One step of every class (cls < 0) or of one class only (the tuner's measurements).
-    void queue_step_of(int cls)
+    void queue_class(const Class& c, int count)
+    {
+        for (const Class::Chunk& h : c.chunks) {
+            for (int step = 0; step < count; ++step) {
+                queue_chunk(c, h);
+            }
+        }
+        hcheck(hipGetLastError(), "launch");
+    }
+
+    // One step of a chunk: the four passes.
+    void queue_chunk(const Class& c, const Class::Chunk& h)
     {
         const hipStream_t s = stream();
         const int second = scheme == 0 ? kCsSecond : kHvSecond;
         for (int pass = 0; pass < 4; ++pass) {
-            for (std::size_t ci = 0; ci < classes.size(); ++ci) {
-                if (cls >= 0 && static_cast<int>(ci) != cls) {
-                    continue;
-                }
-                Class& c = classes[ci];
-                if (pass == 0 || pass == 2) {
-                    RowKernel k = pick_row_kernel(c.nx / c.lanes, c.lanes, pass == 0 ? kFirst : second);
-                    // pass 3 reads D2 rows for the mixed term (CS) or U and D2 (HV)
-                    const float* src = pass == 2 && scheme == 0 ? D2.p : U.p;
-                    hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(c.n_row_tasks)), dim3(64 * c.row_waves), 0, s, opts.p, rows.p,
-                        c.row_tasks.p, src, D2.p, T1.p);
-                } else if (c.col_part > 0) {
-                    launch_cols_part(c, pass == 3, s);
-                } else if (pass == 1) {
-                    if (c.col_lds) {
-                        hipLaunchKernelGGL(k_cols_lds<false>, dim3(static_cast<unsigned>(c.n_col_tasks)), dim3(64), lds_bytes(c), s, opts.p,
-                            rows.p, c.col_tasks.p, U.p, D2.p, T1.p);
-                    } else {
-                        hipLaunchKernelGGL(k_cols<false>, dim3(static_cast<unsigned>(c.n_col_tasks)), dim3(c.col_threads), 0, s, opts.p,
-                            rows.p, c.col_tasks.p, U.p, D2.p, T1.p);
-                    }
-                } else {
-                    if (c.col_lds) {
-                        hipLaunchKernelGGL(k_cols_lds<true>, dim3(static_cast<unsigned>(c.n_col_tasks)), dim3(64), lds_bytes(c), s, opts.p,
-                            rows.p, c.col_tasks.p, U.p, D2.p, T1.p);
-                    } else {
-                        hipLaunchKernelGGL(k_cols<true>, dim3(static_cast<unsigned>(c.n_col_tasks)), dim3(c.col_threads), 0, s, opts.p,
-                            rows.p, c.col_tasks.p, U.p, D2.p, T1.p);
-                    }
-                }
+            const dim3 cols(static_cast<unsigned>(h.col1 - h.col0));
+            const Task* tasks = c.col_tasks.p + h.col0;
+            if (pass == 0 || pass == 2) {
+                RowKernel k = pick_row_kernel(c.nx / c.lanes, c.lanes, pass == 0 ? kFirst : second);
+                // pass 3 reads D2 rows for the mixed term (CS) or U and D2 (HV)
+                const float* src = pass == 2 && scheme == 0 ? D2.p : U.p;
+                hipLaunchKernelGGL(k, dim3(static_cast<unsigned>(h.row1 - h.row0)), dim3(64 * c.row_waves), 0, s, opts.p, rows.p,
+                    c.row_tasks.p + h.row0, src, D2.p, T1.p);
+            } else if (c.col_part > 0) {
+                launch_cols_part(c, h, pass == 3, s);
+            } else if (c.col_lds) {
+                hipLaunchKernelGGL(pass == 1 ? k_cols_lds<false> : k_cols_lds<true>, cols, dim3(64), lds_bytes(c), s, opts.p, rows.p,
+                    tasks, U.p, D2.p, T1.p);
+            } else {
+                hipLaunchKernelGGL(pass == 1 ? k_cols<false> : k_cols<true>, cols, dim3(c.col_threads), 0, s, opts.p, rows.p, tasks,
+                    U.p, D2.p, T1.p);
             }
         }
-        hcheck(hipGetLastError(), "launch");
     }
 
     // Card time (ms) of `reps` steps of one class with its current shape, after one untimed step.
@@ -833,11 +856,10 @@ struct fe_heston {
         hipEvent_t e0 = nullptr, e1 = nullptr;
         hcheck(hipEventCreate(&e0), "event");
         hcheck(hipEventCreate(&e1), "event");
-        queue_step_of(cls);
+        const Class& c = classes[static_cast<std::size_t>(cls)];
+        queue_class(c, 1);
         hcheck(hipEventRecord(e0, stream()), "event");
-        for (int r = 0; r < reps; ++r) {
-            queue_step_of(cls);
-        }
+        queue_class(c, reps);
         hcheck(hipEventRecord(e1, stream()), "event");
         hcheck(hipEventSynchronize(e1), "event");
         float ms = 0.0f;
@@ -1133,9 +1155,7 @@ int fe_heston_step(fe_heston* b, int count)
         return -1;
     }
     try {
-        for (int s = 0; s < count; ++s) {
-            b->queue_step();
-        }
+        b->queue_steps(count);
         return 0;
     } catch (const std::exception& e) {
         return fail(b, e.what());
@@ -1157,9 +1177,7 @@ int fe_heston_capture(fe_heston* b, int count)
             return fail(b, "graph capture did not start");
         }
         try {
-            for (int s = 0; s < count; ++s) {
-                b->queue_step();
-            }
+            b->queue_steps(count);
         } catch (...) {
             fe_hip_graph graph = nullptr;
             fe_hip_graph_end_capture(&graph);
