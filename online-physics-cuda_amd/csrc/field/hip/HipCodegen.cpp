@@ -120,9 +120,11 @@ __device__ __forceinline__ void run_to(int j, int d, int n, int& lo, int& hi)
     lo = j == 0 ? 0 : j - d; if (lo < 0) lo = 0;
     hi = j == n - 1 ? n - 1 : j - d; if (hi > n - 1) hi = n - 1;
 }
-// "Field t changed": one store a wave at most, by its first lane that saw a change.
+// "Field t changed": one store a wave at most, by its first lane that saw a change, and only in a step that reads the flags
+// back (flag 16): every wave's store goes to one word. Three fields' adjoint on 256^3: six targets, 374 us with, 325 without.
 __device__ __forceinline__ void mark(const K& k, int t, bool changed)
 {
+    if ((k.flags & 16) == 0) return;
     const u64 m = __ballot(changed);
     if (m != 0ull && (int)(threadIdx.x & 63u) == __ffsll((long long)m) - 1) k.C[t] = 1u;
 }

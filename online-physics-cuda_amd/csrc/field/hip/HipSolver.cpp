@@ -219,7 +219,7 @@ struct Impl final : HipBackend {
         std::memcpy(&k[w++], &shape.cell, 8);
         std::memcpy(&k[w++], &dt, 8);
         const double hh = shape.cell * shape.cell, inv_h = 1.0 / shape.cell, inv_hh = 1.0 / hh;
-        const int flags = spacing_flags();
+        const int flags = spacing_flags() | (tracking ? 16 : 0);
         std::memcpy(&k[w++], &inv_h, 8);
         std::memcpy(&k[w++], &inv_hh, 8);
         const int ints[4] = {shape.nx, shape.ny, shape.nz, flags};
@@ -1879,6 +1879,7 @@ struct Impl final : HipBackend {
         upload_params();
         upload(fields, edits);
         check(fe_hip_memset_d32_async(C.p, 0u, std::max<std::size_t>(1, law->fields.size())), "change flags reset");
+        tracking = true;
         std::vector<Judge> none;
         run_derives(false, none);
         std::vector<int> measured;

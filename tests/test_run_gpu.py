@@ -57,3 +57,29 @@ def test_run_ends_on_the_reference_bits(device, name):
     solver.run(meta["dt"], meta["steps"])
     for f, expected in final.items():
         assert golden_io.same(meta, solver.get_field(f), expected), f"{name}/{f}"
+
+
+@pytest.mark.parametrize("flat", [False, True])
+def test_a_derive_after_a_run_still_reports_its_change(device, flat):
+    """A run of steps that reads no change flags back writes none; what is derived next, and the next eager step, do."""
+    import field_hip
+
+    law = field_hip.Law("field a init 0 range -10 10\nfield w init 0 range -10 10\nparam q = 2\nderive w = q * a\n"
+                        "term decay\n  d a = -0.5 * a\n")
+    shape = (130, 1, 9) if flat else (20, 14, 9)
+    s = field_hip.Solver(law, shape, 1.0)
+    a = np.random.default_rng(4).uniform(-1, 1, int(np.prod(shape))).astype(np.float32)
+    s.set_field("a", a)
+    s.refresh_derived()
+    s.set_lazy_readback(True)
+    s.check_contracts_every(1 << 30)
+    s.run(0.125, 40)
+    w = s.get_field("w")  # the host's copy is the card's
+    s.set_param("q", 4.0)
+    s.refresh_derived()
+    assert s.last_changed()[1]
+    assert np.array_equal(bits(s.get_field("w")), bits(2.0 * w))  # a power of two: exact
+    s.set_lazy_readback(False)
+    s.step(0.125)
+    assert list(s.last_changed()) == [1, 1]
+    assert np.array_equal(bits(s.get_field("w")), bits(np.float32(4.0) * s.get_field("a")))
