@@ -400,7 +400,7 @@ struct Impl final : HipBackend {
     // (e.g. "4x2", "1x6", "h4x8" and "r4x8" for the two flux-carrying forms) picks one. None: the direct gather.
     const hip::WindowKernel* window_for(const hip::ProgramCode& code) const
     {
-        // A lattice one row high leaves a window's other rows (and its halo-row waves) idle: the direct gather (measured
+        // A lattice one row high leaves a window's other rows idle: the direct gather (measured
         // on MI355X, Black-Scholes 4096 x 1 x 512: 16.8 us a pass against 23.8 through 256x2 tiles, and 9.6 with four planes a thread).
         if (!code.window || code.windows.empty() || force_direct || spacing_flags() < 3 || (shape.ny == 1 && tile_vx == 0)) {
             return nullptr;
