@@ -301,21 +301,20 @@ extern "C" __global__ __launch_bounds__(256) void k_total(K k, int field, i64 ch
     if (t == 0) { out[2 * blockIdx.x] = s.s + s.c; out[2 * blockIdx.x + 1] = m.s + m.c; }
 }
 
-// Pass 2: one block folds `parts` pairs in order into dst[0], dst[1].
-extern "C" __global__ __launch_bounds__(256) void k_total_final(const double* parts, int count, double* dst)
+// Pass 2: one block folds `parts` pairs in order into dst[0], dst[1]; with acc not null the total is also added into acc[0],
+// acc[1] in double, in call order (no wait for the host, no launch of its own).
+extern "C" __global__ __launch_bounds__(256) void k_total_final(const double* parts, int count, double* dst, double* acc)
 {
     __shared__ double wv[4][4];
     const int t = (int)threadIdx.x;
     Sum s = {0.0, 0.0}; Sum m = {0.0, 0.0};
     for (int i = t; i < count; i += 256) { add(s, parts[2 * i]); add(m, parts[2 * i + 1]); }
     block_pairs(s, m, wv);
-    if (t == 0) { dst[0] = s.s + s.c; dst[1] = m.s + m.c; }
-}
-
-// acc[0..1] += src[0..1] in double (a field's total added on the card, in call order: no wait for the host).
-extern "C" __global__ void k_acc(const double* src, double* acc)
-{
-    if (threadIdx.x == 0) { acc[0] = acc[0] + src[0]; acc[1] = acc[1] + src[1]; }
+    if (t == 0) {
+        const double sum = s.s + s.c, mag = m.s + m.c;
+        dst[0] = sum; dst[1] = mag;
+        if (acc != nullptr) { acc[0] = acc[0] + sum; acc[1] = acc[1] + mag; }
+    }
 }
 
 // Words [0, zeros) to 0 and [zeros, zeros + ones) to all ones: the change flags, range counts and first bad cells of a

@@ -1002,8 +1002,8 @@ struct Impl final : HipBackend {
     }
 
     // The conserved total (sum, sum of magnitudes) of a field into totals[slot], [slot + 1]; with a range record
-    // (`record` >= 0) the same pass checks (and clamps) the field's range into it.
-    void total(int field, int slot, int record = -1)
+    // (`record` >= 0) the same pass checks (and clamps) the field's range into it; `acc`: two doubles it is added into.
+    void total(int field, int slot, int record = -1, double* acc = nullptr)
     {
         const bool ranged = record >= 0;
         const long long cells = static_cast<long long>(shape.cells());
@@ -1020,7 +1020,7 @@ struct Impl final : HipBackend {
         check(fe_hip_launch(fn("k_total"), static_cast<unsigned>(blocks), 1, 1, 256, 1, 1, 0, argv1), "total launch");
         double* dst = totals.as<double>() + slot;
         int count = blocks;
-        void* argv2[] = {&parts, &count, &dst};
+        void* argv2[] = {&parts, &count, &dst, &acc};
         check(fe_hip_launch(fn("k_total_final"), 1, 1, 1, 256, 1, 1, 0, argv2), "total final launch");
         prof.launches += 2;
         if (ranged && clamp) {
@@ -1164,7 +1164,8 @@ struct Impl final : HipBackend {
                         double* parts = tile_sums.as<double>();
                         int count = static_cast<int>(fused.tiles);
                         double* dst = totals.as<double>() + slot + 2 * m + 2 * q;
-                        void* fargs[] = {&parts, &count, &dst};
+                        double* no_acc = nullptr;
+                        void* fargs[] = {&parts, &count, &dst, &no_acc};
                         check(fe_hip_launch(fn("k_total_final"), 1, 1, 1, 256, 1, 1, 0, fargs), "total final launch");
                         ++prof.launches;
                         note_total(f, slot + 2 * m + 2 * q);
@@ -1959,11 +1960,8 @@ struct Impl final : HipBackend {
     void field_total_accumulate(int f, double* acc) override
     {
         const std::lock_guard<std::mutex> lock(device_mutex());
-        total(f, kTotals - 2);
+        total(f, kTotals - 2, -1, acc);
         note_total(f, kTotals - 2);
-        double* src = totals.as<double>() + (kTotals - 2);
-        void* argv[] = {&src, &acc};
-        check(fe_hip_launch(fn("k_acc"), 1, 1, 1, 64, 1, 1, 0, argv), "total accumulate");
     }
 
     void field_total(int f, double& sum, double& mag) override
