@@ -629,13 +629,18 @@ private:
     // Divisions other than by the spacing stay in a pass that fills the card: in a solve, one wave a SIMD, they cost more
     // than they save. Implicit y then z with a field's coefficients on 256^3: four stored passes (149 us) and 4 of 44 bytes
     // a cell a solve gone, 509 -> 350 us a step.
+    // A folded coefficient holds field reads alone: one built from a value that is itself stored (another coefficient,
+    // `1 - 2 * a` beside `a`) would read that value's lattice, which the solve does not hold, so it stays stored too.
     std::set<int> folded_;
     static constexpr int kFoldOps = 12;
-    bool fold_cost(int id, int& ops, std::set<int>& fields) const
+    bool fold_cost(int id, int& ops, std::set<int>& fields, const std::set<int>& stages, bool root = true) const
     {
         const ir::Inst& in = at(id);
         if (scalar(id)) {
             return in.op != Op::Mlp;
+        }
+        if (!root && stages.count(id) != 0) {
+            return false;
         }
         switch (in.op) {
         case Op::Field: fields.insert(in.index); return true;
@@ -650,10 +655,11 @@ private:
         if (++ops > kFoldOps) {
             return false;
         }
-        return std::all_of(in.args.begin(), in.args.end(), [&](int a) { return fold_cost(a, ops, fields); });
+        return std::all_of(in.args.begin(), in.args.end(), [&](int a) { return fold_cost(a, ops, fields, stages, false); });
     }
     void fold_coefficients(std::set<int>& stages)
     {
+        const std::set<int> all = stages;
         std::vector<char> lines(m_.insts.size(), 0), other(m_.insts.size(), 0);
         for (std::size_t id = 0; id < m_.insts.size(); ++id) {
             if (!used(static_cast<int>(id))) {
@@ -676,7 +682,7 @@ private:
             int ops = 0;
             std::set<int> fields;
             const bool fold = at(id).op != Op::Tridiag && lines[static_cast<std::size_t>(id)] && !other[static_cast<std::size_t>(id)] &&
-                !scalar(id) && fold_cost(id, ops, fields) && fields.size() <= 2;
+                !scalar(id) && fold_cost(id, ops, fields, all) && fields.size() <= 2;
             if (fold) {
                 folded_.insert(id);
                 it = stages.erase(it);
@@ -1421,7 +1427,7 @@ private:
                 fetch << "    const double s_" << names[q] << " = " << d(arg) << ";\n";
             } else if (folded_.count(arg) != 0) {
                 int ops = 0;
-                fold_cost(arg, ops, leaves);
+                fold_cost(arg, ops, leaves, {});
             } else {
                 cell.push_back({names[q], arg, -1});
             }
