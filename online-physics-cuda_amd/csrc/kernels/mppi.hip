@@ -2,12 +2,13 @@
 //
 // The reference plans with one thread a future, the dynamics MLP evaluated in fp32 registers with the weights in shared
 // memory (src/field/mind/WorldModel.cpp:192-240). Here a wave carries 16 or 32 futures through the whole horizon without
-// leaving its registers: a layer is W (A: 16 outputs x 32 inputs a fragment, fp16, from LDS) times the futures' inputs (B:
-// 32 inputs x 16 futures), fp32 accumulators that start from the bias, and a product's D (lane l: future l % 16, outputs
-// 4 (l / 16)..+3 of a block of 16) is, after tanh and rounding to fp16, the next layer's B with no exchange between lanes.
-// The states stay in D's layout in fp32; the last layer's rates move them there.
-// The update weighs every future by exp(-(J - J_min) / lambda) and sums in a fixed order: the same inputs give the same
-// plan, bit for bit.
+// leaving its registers: a layer is W (A: 16 outputs x 16 inputs a product, fp16, two products a fragment from LDS) times the
+// futures' inputs (B: 16 inputs x 16 futures) summed in fp32 from 0, a block of 16 inputs after the other, and the bias; a
+// product's D (lane l: future l % 16, outputs 4 (l / 16)..+3 of a block of 16) is, after tanh and rounding to fp16, the next
+// layer's B with no exchange between lanes. The states stay in D's layout in fp32; the last layer's rates move them there.
+// The update weighs every future by exp(-(J - J_min) / lambda) and sums the futures one by one. Every sum's order is fixed
+// (a layer's inputs in blocks of 16, a cost's features four apart, the futures in turn), whatever the number of agents,
+// futures and tiles a wave: the same inputs give the same plan, bit for bit, and tests/golden/mppi_plans.npz holds some.
 #include "fe_mppi.h"
 #include "fe_hip.h"
 
@@ -24,6 +25,7 @@
 
 namespace {
 
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 typedef unsigned long long u64;
@@ -70,17 +72,26 @@ __device__ inline float gauss(u64 key)
 
 // tanh u = 1 - 2 / (1 + e^(2u)) through the hardware exponential and reciprocal: a few ulp of fp32, below the fp16
 // rounding of the activation it becomes; the library tanhf's long polynomial sequence was most of a layer's issue slots.
-// Saturates to +-1 (e^(2u) overflowing to inf, or to 0).
+// Saturates to +-1 (e^(2u) overflowing to inf, or to 0). Not a fused multiply-add: with the rounding to fp16 behind it the
+// compiler takes one instruction that rounds once, and the activation's last bit changes.
 __device__ __forceinline__ float fast_tanh(float u)
 {
     const float e = __builtin_amdgcn_exp2f((2.0f * 1.4426950408889634f) * u); // e^(2u), 2 log2(e) folded
     return 1.0f - 2.0f * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
-// A layer's tanh, rounded into the next layer's inputs (zero past the hidden units).
+// A layer's bias and tanh, rounded into the next layer's inputs (zero past the hidden units).
 template <int HB, int Q>
-__device__ __forceinline__ void activate(const float4v (&z)[Q][HB], half8 (&h)[Q][(HB + 1) / 2])
+__device__ __forceinline__ void activate(float4v (&z)[HB][Q], const float4v* b, int g, half8 (&h)[Q][(HB + 1) / 2])
 {
+#pragma unroll
+    for (int ob = 0; ob < HB; ++ob) {
+        const float4v bias = b[4 * ob + g];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            z[ob][q] += bias;
+        }
+    }
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
 #pragma unroll
@@ -88,7 +99,7 @@ __device__ __forceinline__ void activate(const float4v (&z)[Q][HB], half8 (&h)[Q
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const int ob = 2 * c + (e >> 2);
-                h[q][c][e] = ob < HB ? (_Float16)fast_tanh(z[q][ob < HB ? ob : 0][e & 3]) : (_Float16)0.0f;
+                h[q][c][e] = ob < HB ? (_Float16)fast_tanh(z[ob < HB ? ob : 0][q][e & 3]) : (_Float16)0.0f;
             }
         }
     }
@@ -99,15 +110,54 @@ __host__ __device__ constexpr int frag_count(int HB, int NC, int fb) { return HB
 __host__ __device__ constexpr int table_count(int HB, int NC, int fb) { return 4 * (2 * HB + 4 * NC + 4 * fb); }
 constexpr int lds_bytes(int HB, int NC, int fb) { return frag_count(HB, NC, fb) * 1024 + table_count(HB, NC, fb) * 16; }
 
-__device__ __forceinline__ float4v mfma(half8 w, half8 x, float4v acc) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(w, x, acc, 0, 0, 0); }
+// A fragment's 32 inputs for all Q tiles as two products of 16, the first block and (`both`) the second: the one deep product
+// adds them in an order of its own, which moves activations across fp16 boundaries. A block of zeros changes nothing.
+template <int Q, typename In>
+__device__ __forceinline__ void mfma(half8 w, const In& in, float4v (&acc)[Q], bool both)
+{
+    const half4 w0 = __builtin_shufflevector(w, w, 0, 1, 2, 3), w1 = __builtin_shufflevector(w, w, 4, 5, 6, 7);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        acc[q] = __builtin_amdgcn_mfma_f32_16x16x16f16(w0, __builtin_shufflevector(in(q), in(q), 0, 1, 2, 3), acc[q], 0, 0, 0);
+    }
+    if (both) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            acc[q] = __builtin_amdgcn_mfma_f32_16x16x16f16(w1, __builtin_shufflevector(in(q), in(q), 4, 5, 6, 7), acc[q], 0, 0, 0);
+        }
+    }
+}
+
+// Lane group g's four values for features 4g..4g + 3 of a block to those of features g, g + 4, g + 8, g + 12 (a 4 x 4
+// transpose over the wave's four groups of 16 lanes): v_permlane32_swap exchanges a register's upper 32 lanes with another's
+// lower ones, v_permlane16_swap its odd rows of 16 with another's even ones.
+__device__ __forceinline__ void swap32(float& a, float& b)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void swap16(float& a, float& b)
+{
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+}
+__device__ __forceinline__ void by_fours(float (&v)[4])
+{
+    swap32(v[0], v[2]);
+    swap32(v[1], v[3]);
+    swap16(v[0], v[1]);
+    swap16(v[2], v[3]);
+}
 
 // A wave takes 16 Q futures of an agent at a time; wave w of the grid the items w, w + waves, ... (agent-major). Actions into
 // acts[agent][t][k][axis], each future's cost into cost[agent][k]. The noise is drawn by every lane: with two tiles (Q = 2)
 // lane l the future l / 2, axis l % 2 of the step; with one, the lanes 32.. draw the step after. The weights and the tables
 // are read from LDS where they are used (two tiles to a read).
 // Bound by the hidden units' tanh, two quarter-rate instructions each: about 165 us of 256 agents x 512 futures x 32 steps with
-// 16 features and 64 hidden units, which take 232 (784 when each layer's activations went through LDS and its weights were
-// read from memory a tile at a time); the update 8 us (36 with a thread a step and axis over all futures).
+// 16 features and 64 hidden units, which take 229 (784 when each layer's activations went through LDS and its weights were
+// read from memory a tile at a time). Products of 32 inputs that start from the bias would take 210, and give other bits.
 template <int HB, int NC, int Q>
 __global__ __launch_bounds__(256) void k_mppi_rollout(Desc d, const float* __restrict__ obs, const float* __restrict__ mean,
     const unsigned* __restrict__ ids, float* __restrict__ acts, float* __restrict__ cost, u64 tick, float sigma, float dt, unsigned items,
@@ -185,42 +235,32 @@ __global__ __launch_bounds__(256) void k_mppi_rollout(Desc d, const float* __res
                 }
             }
             half8 h[Q][HC];
-            float4v z[Q][HB];
+            float4v z[HB][Q];
 #pragma unroll
             for (int ob = 0; ob < HB; ++ob) {
-                const float4v bias = b1[4 * ob + g];
 #pragma unroll
                 for (int q = 0; q < Q; ++q) {
-                    z[q][ob] = bias;
+                    z[ob][q] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
                 }
 #pragma unroll
                 for (int c = 0; c < NC; ++c) {
-                    const half8 w = W1[(ob * NC + c) * 64 + l];
-#pragma unroll
-                    for (int q = 0; q < Q; ++q) {
-                        z[q][ob] = mfma(w, in[q][c], z[q][ob]);
-                    }
+                    mfma(W1[(ob * NC + c) * 64 + l], [&](int q) { return in[q][c]; }, z[ob], true);
                 }
             }
-            activate<HB, Q>(z, h);
+            activate<HB, Q>(z, b1, g, h);
             asm volatile("" ::: "memory");
 #pragma unroll
             for (int ob = 0; ob < HB; ++ob) {
-                const float4v bias = b2[4 * ob + g];
 #pragma unroll
                 for (int q = 0; q < Q; ++q) {
-                    z[q][ob] = bias;
+                    z[ob][q] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
                 }
 #pragma unroll
                 for (int c = 0; c < HC; ++c) {
-                    const half8 w = W2[(ob * HC + c) * 64 + l];
-#pragma unroll
-                    for (int q = 0; q < Q; ++q) {
-                        z[q][ob] = mfma(w, h[q][c], z[q][ob]);
-                    }
+                    mfma(W2[(ob * HC + c) * 64 + l], [&](int q) { return h[q][c]; }, z[ob], 2 * c + 1 < HB);
                 }
             }
-            activate<HB, Q>(z, h);
+            activate<HB, Q>(z, b2, g, h);
             asm volatile("" ::: "memory");
             // the rates, the states they move, and the states' part of the step's cost
             float c[Q] = {};
@@ -231,28 +271,31 @@ __global__ __launch_bounds__(256) void k_mppi_rollout(Desc d, const float* __res
                     float4v v[Q];
 #pragma unroll
                     for (int q = 0; q < Q; ++q) {
-                        v[q] = bias;
+                        v[q] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
                     }
 #pragma unroll
                     for (int k = 0; k < HC; ++k) {
-                        const half8 w = W3[(b * HC + k) * 64 + l];
-#pragma unroll
-                        for (int q = 0; q < Q; ++q) {
-                            v[q] = mfma(w, h[q][k], v[q]);
-                        }
+                        mfma(W3[(b * HC + k) * 64 + l], [&](int q) { return h[q][k]; }, v, 2 * k + 1 < HB);
                     }
 #pragma unroll
                     for (int q = 0; q < Q; ++q) {
+                        v[q] += bias;
+                        float term[4];
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
                             st[q][b][r] += dt * v[q][r] * sc[r];
                             const float e = st[q][b][r] - to[r];
-                            c[q] += wt[r] * e * e;
+                            term[r] = wt[r] * e * e;
+                        }
+                        by_fours(term);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            c[q] += term[r];
                         }
                     }
                 }
             }
-            // the four lane groups' features added in a fixed order
+            // the four lane groups' features (four apart each) added in a fixed order
 #pragma unroll
             for (int q = 0; q < Q; ++q) {
                 c[q] += __shfl_xor(c[q], 16);
@@ -271,54 +314,110 @@ __global__ __launch_bounds__(256) void k_mppi_rollout(Desc d, const float* __res
 }
 
 // The new plan: the futures' actions weighted by exp(-(J - J_min) / lambda), lambda a quarter of (mean cost - least cost), at
-// least 1e-4. A block an agent: the least cost, the costs' sum and each future's weight once (in LDS), then a wave a step:
-// lane l the axis l % 2 of the futures l / 2, l / 2 + 32, ..., and the lanes of an axis in a fixed tree.
+// least 1e-4. A block an agent: the least cost, the costs' sum and each future's weight once (in LDS), then a lane a (step,
+// axis) of the first waves, the futures added in their order: a chain of K adds, which reads LDS. All threads bring the next
+// run of futures there, its loads in flight beside the chain: 13 us for 256 agents x 512 futures x 32 steps, 4 x 32 futures
+// 4 us (18-25 where a lane reads its own actions from memory, eight or 256 of them in flight; 8 as a tree over the lanes, whose
+// sums are others).
 constexpr int kMaxSamples = 1024;
-constexpr int kUpdateWaves = 16;
-__global__ __launch_bounds__(64 * kUpdateWaves) void k_mppi_update(const float* __restrict__ cost, const float* __restrict__ acts,
+constexpr int kUpdateThreads = 512;
+constexpr int kRunFloats = 8192; // a run's actions: 128 futures up to 32 steps, 64 past them
+__global__ __launch_bounds__(kUpdateThreads) void k_mppi_update(const float* __restrict__ cost, const float* __restrict__ acts,
     float* __restrict__ mean, int K, int H)
 {
-    __shared__ float cs[kMaxSamples];
-    __shared__ float lows[kUpdateWaves], sums[kUpdateWaves];
+    constexpr int kPairs = kRunFloats / 2 / kUpdateThreads;
+    __shared__ __attribute__((aligned(16))) float cs[kMaxSamples];
+    __shared__ __attribute__((aligned(16))) float run[kRunFloats + 128]; // a step's futures a row, two floats of padding each
+    __shared__ float lo_s, lam_s;
     const long long agent = (long long)blockIdx.x;
-    const int q = (int)threadIdx.x, l = q & 63, w = q >> 6;
-    static_assert(kMaxSamples == 64 * kUpdateWaves, "a thread a future");
-    const float c = cost[agent * K + (q < K ? q : 0)];
-    float lo = c, sum = q < K ? c : 0.0f;
-    for (int m = 32; m > 0; m >>= 1) {
-        lo = fminf(lo, __shfl_xor(lo, m));
-        sum += __shfl_xor(sum, m);
+    const int q = (int)threadIdx.x;
+    const int lt = H > 32 ? 6 : 7, T = 1 << lt, pitch = 2 * T + 2; // futures a run
+    const float* a = acts + agent * H * 2 * K;
+    // pair i of a run: future i % T of step i / T, both axes
+    float2 held[kPairs];
+    auto fetch = [&](int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < kPairs; ++u) {
+            const int i = q + u * kUpdateThreads, t = i >> lt, k = k0 + (i & (T - 1));
+            held[u] = t < H && k < K ? *reinterpret_cast<const float2*>(a + (t * K + k) * 2) : make_float2(0.0f, 0.0f);
+        }
+    };
+    auto put = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < kPairs; ++u) {
+            const int i = q + u * kUpdateThreads;
+            *reinterpret_cast<float2*>(run + (i >> lt) * pitch + 2 * (i & (T - 1))) = held[u];
+        }
+    };
+    fetch(0);
+    for (int k = q; k < K; k += kUpdateThreads) {
+        cs[k] = cost[agent * K + k];
     }
-    if (l == 0) {
-        lows[w] = lo;
-        sums[w] = sum;
+    put();
+    __syncthreads();
+    fetch(T);
+    if (q < 64) {
+        float lo = cs[0], sum = 0.0f;
+        for (int k = q; k < K; k += 64) {
+            lo = fminf(lo, cs[k]);
+        }
+        for (int m = 32; m > 0; m >>= 1) {
+            lo = fminf(lo, __shfl_xor(lo, m));
+        }
+        for (int k = 0; k < K; k += 16) { // added in order, sixteen to a wait
+            float4v c[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                c[i] = *reinterpret_cast<const float4v*>(cs + k + 4 * i);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                sum += c[i >> 2][i & 3];
+            }
+        }
+        if (q == 0) {
+            lo_s = lo;
+            lam_s = fmaxf(1e-4f, 0.25f * (sum / (float)K - lo));
+        }
     }
     __syncthreads();
-    lo = lows[0];
-    sum = sums[0];
-    for (int i = 1; i < kUpdateWaves; ++i) {
-        lo = fminf(lo, lows[i]);
-        sum += sums[i];
+    const float lo = lo_s, lam = lam_s;
+    for (int k = q; k < K; k += kUpdateThreads) {
+        cs[k] = expf(-(cs[k] - lo) / lam);
     }
-    const float lam = fmaxf(1e-4f, 0.25f * (sum / (float)K - lo));
-    cs[q] = q < K ? expf(-(c - lo) / lam) : 0.0f;
     __syncthreads();
-    for (int t = w; t < H; t += kUpdateWaves) {
-        const float* a = acts + (agent * H + t) * 2 * K;
-        float wsum = 0.0f, acc = 0.0f;
-#pragma unroll 4
-        for (int i = l; i < 2 * K; i += 64) {
-            const float wk = cs[i >> 1];
-            wsum += wk;
-            acc += wk * a[i];
+    float wsum = 0.0f, acc = 0.0f;
+    const float* mine = run + (q >> 1) * pitch + (q & 1);
+    for (int k0 = 0; k0 < K; k0 += T) {
+        if (q < 2 * H) {
+            const int n = K - k0 < T ? K - k0 : T;
+            for (int k = 0; k < n; k += 16) {
+                float4v w[4];
+                float v[16];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    w[i] = *reinterpret_cast<const float4v*>(cs + k0 + k + 4 * i);
+                }
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    v[i] = mine[2 * (k + i)];
+                }
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    wsum += w[i >> 2][i & 3];
+                    acc += w[i >> 2][i & 3] * v[i];
+                }
+            }
         }
-        for (int m = 32; m > 1; m >>= 1) {
-            wsum += __shfl_xor(wsum, m);
-            acc += __shfl_xor(acc, m);
+        if (k0 + T < K) {
+            __syncthreads();
+            put();
+            __syncthreads();
+            fetch(k0 + 2 * T);
         }
-        if (l < 2) {
-            mean[(agent * H + t) * 2 + l] = acc / wsum;
-        }
+    }
+    if (q < 2 * H) {
+        mean[agent * 2 * H + q] = acc / wsum;
     }
 }
 
@@ -539,10 +638,11 @@ int fe_mppi_plan(fe_mppi* p, int agents, const float* obs, const uint32_t* ids, 
     try {
         const int F = p->F, H = p->horizon, K = p->samples;
         const long long tiles = static_cast<long long>(agents) * (K / 16);
-        // Two tiles a wave share the weights' reads and hide each other's latency, once there are three a SIMD: hidden 64,
-        // 128 and 16 take 208, 286, 125 us against one tile's 218, 315, 126 at four a SIMD, 328, 495, 166 against 341, 558,
-        // 176 at eight; at two they are even (151, 199, 104 against 151, 199, 100), and a lone agent takes 129 against 111.
-        const int two = tiles >= 12LL * p->cus && K > 16 ? 1 : 0;
+        // Two tiles a wave share the weights' reads and hide each other's latency, once there are four a SIMD: hidden 64,
+        // 128 and 16 take 205, 315, 137 us a plan against one tile's 200, 328, 136 at four a SIMD, 307, 546, 181 against 316,
+        // 588, 187 at eight; at three one tile is the faster (174, 258, 123 against 203, 310, 135), and for a lone agent (121
+        // against 146).
+        const int two = tiles >= 16LL * p->cus && K > 16 ? 1 : 0;
         const unsigned per_agent = static_cast<unsigned>((K / 16 + two) / (1 + two));
         const long long items = static_cast<long long>(agents) * per_agent;
         if (items >= 4294967296LL - 2097152) { // the kernel's index, and its stride past the end; their actions would be 550 GB
@@ -560,7 +660,7 @@ int fe_mppi_plan(fe_mppi* p, int agents, const float* obs, const uint32_t* ids, 
         const Desc d{F, p->fb, H, K, p->frags.p, reinterpret_cast<const float4v*>(p->tables.p), p->action_weight};
         hipLaunchKernelGGL(p->rollout[two], dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), static_cast<unsigned>(p->lds), s, d, p->obs.p,
             p->mean.p, p->ids.p, p->acts.p, p->cost.p, static_cast<unsigned long long>(tick), sigma, dt, static_cast<unsigned>(items), per_agent);
-        hipLaunchKernelGGL(k_mppi_update, dim3(static_cast<unsigned>(agents)), dim3(64 * kUpdateWaves), 0, s, p->cost.p, p->acts.p, p->mean.p, K, H);
+        hipLaunchKernelGGL(k_mppi_update, dim3(static_cast<unsigned>(agents)), dim3(kUpdateThreads), 0, s, p->cost.p, p->acts.p, p->mean.p, K, H);
         hcheck(hipGetLastError(), "mppi launch");
         hcheck(hipMemcpyAsync(mean, p->mean.p, sizeof(float) * static_cast<std::size_t>(agents) * H * 2, hipMemcpyDeviceToHost, s), "download");
         if (cost_out != nullptr) {

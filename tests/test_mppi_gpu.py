@@ -3,6 +3,9 @@
 The card runs the dynamics on fp16 MFMA with fp32 accumulation and its own transcendentals; the oracle rounds where
 the card rounds and sums in float64, so futures' costs agree to 2e-3 relative and the plans to 2e-3 absolute. Two runs
 give the same plan bit for bit."""
+import os
+
+import make_mppi_golden
 import numpy as np
 import pytest
 
@@ -63,6 +66,18 @@ def test_every_net_shape_matches_the_oracle(device, features, hidden, samples, a
     rel = np.abs(costs[some] - wcost) / np.maximum(np.abs(wcost), 1e-3)
     assert rel.max() < 2e-3, rel.max()
     assert np.max(np.abs(got[some] - want)) < 2e-3, np.max(np.abs(got[some] - want))
+
+
+@pytest.mark.parametrize("shape", make_mppi_golden.SHAPES, ids=make_mppi_golden.name)
+def test_plans_keep_their_bits(device, shape):
+    """The order of every sum is the planner's first form's, so its plans and costs are too (tests/golden/make_mppi_golden.py)."""
+    import field_hip
+
+    kept = np.load(os.path.join(os.path.dirname(__file__), "golden", "mppi_plans.npz"))
+    got, costs = make_mppi_golden.plan(field_hip, mppi, shape)
+    name = make_mppi_golden.name(shape)
+    assert np.array_equal(costs.view(np.uint32), kept["costs_" + name].view(np.uint32))
+    assert np.array_equal(got.view(np.uint32), kept["plan_" + name].view(np.uint32))
 
 
 def test_planning_lowers_the_plans_cost(device):
