@@ -8,7 +8,7 @@
 // layer's B with no exchange between lanes. The states stay in D's layout in fp32; the last layer's rates move them there.
 // The update weighs every future by exp(-(J - J_min) / lambda) and sums the futures one by one. Every sum's order is fixed
 // (a layer's inputs in blocks of 16, a cost's features four apart, the futures in turn), whatever the number of agents,
-// futures and tiles a wave: the same inputs give the same plan, bit for bit, and tests/golden/mppi_plans.npz holds some.
+// futures and tiles a wave: the same inputs give the same plan, bit for bit, and tests/golden/mppi/plans.npz holds some.
 #include "fe_mppi.h"
 #include "fe_hip.h"
 

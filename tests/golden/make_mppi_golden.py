@@ -1,4 +1,4 @@
-"""Writes mppi_plans.npz: plans and costs of the planner on the card, for the test that every later build gives their bits.
+"""Writes mppi/plans.npz: plans and costs of the planner on the card, for the test that every later build gives their bits.
 
     python tests/golden/make_mppi_golden.py PACKAGE_FOLDER OUT.npz      (on a gfx950 card)
 

@@ -73,7 +73,7 @@ def test_plans_keep_their_bits(device, shape):
     """The order of every sum is the planner's first form's, so its plans and costs are too (tests/golden/make_mppi_golden.py)."""
     import field_hip
 
-    kept = np.load(os.path.join(os.path.dirname(__file__), "golden", "mppi_plans.npz"))
+    kept = np.load(os.path.join(os.path.dirname(__file__), "golden", "mppi", "plans.npz"))
     got, costs = make_mppi_golden.plan(field_hip, mppi, shape)
     name = make_mppi_golden.name(shape)
     assert np.array_equal(costs.view(np.uint32), kept["costs_" + name].view(np.uint32))
