@@ -2144,7 +2144,8 @@ private:
             const int kk = conduction_form(p);
             if (kk >= 0 && code.window) {
                 flux_kernels(code, cellfn, p.equations[0].target, kk);
-                row_flux_kernels(code, p.equations[0].target, kk);
+                row_flux_kernels(code, p.equations[0].target, kk, 8);
+                row_flux_kernels(code, p.equations[0].target, kk, 4);
             }
         }
         return code;
@@ -2345,6 +2346,7 @@ private:
         w.ty = TY;
         w.block_y = WAVES;
         w.flux = 2;
+        w.totals = true;
         w.zchunk = 16;
         code.windows.push_back(w);
     }
@@ -2352,18 +2354,20 @@ private:
     // The conduction window for rows that are not whole quads of cells or fill 256-wide tiles badly, for lattices past the
     // last-level cache and for few tiles (`_r_`). The fluxes, their sharing and their order are flux_kernels'; what differs is how a wave
     // covers rows. Its 64 lanes are W lanes a row (8, 16, 32 or 64, the launch's choice: mode >> 8 is its logarithm) on
-    // 64 / W consecutive rows, four cells a lane, so a tile is 4W cells by 8 * 64 / W rows and the launch picks the W
-    // whose tiles the rows fill best. Row starts are not 16-byte aligned (the quads are loaded as such; the card takes a
+    // 64 / W consecutive rows, four cells a lane, so a tile of TY waves is 4W cells by TY * 64 / W rows and the launch picks the
+    // W whose tiles the rows fill best. Eight waves (fewer halo rows) hold four waves a SIMD in 128 registers, four of which
+    // spill outside the planes' loop's loads; four waves (more tiles where the lattice gives few) may take 256 and spill none,
+    // and alone take the totals, whose sums would cost the eight 24 spilled registers a plane: 512 x 512 x 128 judged 127 us a
+    // step against 133, 384^3 195 against 205, 256 x 256 x 160 78 against 82. Row starts are not 16-byte aligned (the quads are loaded as such; the card takes a
     // 4-byte aligned quad), and a row's last quad is read from the row's last four cells and moved up, the last cell
     // repeated behind it: its face to the cells that are not there then has a flux of +0, as a closed face's.
-    void row_flux_kernels(ProgramCode& code, int target, int kk)
+    void row_flux_kernels(ProgramCode& code, int target, int kk, int TY)
     {
         const std::string t = std::to_string(target);
-        const int TY = 8;
         const std::string name = code.gather + "_r_" + std::to_string(TY);
         const std::string MK = "M_" + name, LDS = "L_" + name;
-        // rows of 4W + 8 floats: W 64: 10 x 264; 32: 18 x 136; 16: 34 x 72; 8: 66 x 40
-        const int plane = 2640;
+        // rows of 4W + 8 floats, of 8 waves: W 64: 10 x 264; 32: 18 x 136; 16: 34 x 72; 8: 66 x 40; of 4: 6 x 264 the largest
+        const int plane = TY == 8 ? 2640 : 1584;
         std::ostringstream s;
         s << "typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));\n"
           << "template <bool P2> struct " << MK << " { static constexpr bool kPow2 = P2; static constexpr bool kAnyH = false; };\n"
@@ -2494,7 +2498,10 @@ private:
           << "            tsum[2 * tl] = a.s + a.c; tsum[2 * tl + 1] = b.s + b.c; } }\n"
           << "}\n";
         for (const bool total : {false, true}) {
-            s << "extern \"C\" __global__ __launch_bounds__(" << 64 * TY << ") __attribute__((amdgpu_waves_per_eu(" << 4 << "))) void " << name << (total ? "_t" : "")
+            if (total && TY != 4) {
+                continue;
+            }
+            s << "extern \"C\" __global__ __launch_bounds__(" << 64 * TY << ") __attribute__((amdgpu_waves_per_eu(" << (TY == 8 ? 4 : 2) << "))) void " << name << (total ? "_t" : "")
               << "(K k, int zchunk, int tiles_x, int tiles_y, int tiles_z, int mode, double* tsum, unsigned* rec, u64* first, double lo,\n"
               << "    double hi) {\n";
             for (const bool p2 : {true, false}) {
@@ -2510,6 +2517,7 @@ private:
         w.ty = TY;
         w.block_y = TY;
         w.flux = 3;
+        w.totals = TY == 4;
         w.zchunk = 16;
         code.windows.push_back(w);
     }

@@ -78,6 +78,7 @@ struct WindowKernel {
     // A conduction term's flux-carrying window (vx = 4): 2 for rows of whole quads, 3 for any row length of four cells or
     // more (the launch's mode >> 8 the logarithm of its lanes a row); 0 the generic window.
     int flux = 0;
+    bool totals = false; // there is a kernel `name`_t, which takes the contract's totals on the way
     int zchunk = 0; // planes a tile; 0: the program's
 };
 

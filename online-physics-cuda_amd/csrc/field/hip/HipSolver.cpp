@@ -71,9 +71,12 @@ constexpr int kTotals = 1024;      // doubles of conserved totals judged at once
 constexpr int kFillWaves = 2048;    // two waves a SIMD of MI355X: a generic window's launch shortens its z-chunks to reach it
 constexpr int kRanges = 1024;      // range checks judged at once (a record each: two counts and the first bad cell)
 constexpr std::size_t kNearCells = std::size_t{1} << 22; // cells up to which a distance line tries every pair
-// Cells from which a conduction window beats the direct gather (a step of few tiles is as long as a tile's
-// march: 64^3 6.4 us against 3.0, 96^3 7.0 against 7.0, 100^3 7.2 against 8.3, 128^3 7.8 against 9.7).
-constexpr std::size_t kRowCells = 900000;
+// Cells from which a conduction window beats the direct gather on a step that judges nothing (a step of few tiles is as
+// long as a tile's march: 64^3 3.6 us against 3.2, 256 x 200 x 10 4.8 against 4.7, 512^2 x 2 4.2 against 4.5, 300^2 x 7 5.8
+// against 6.3, 96^2 x 90 5.2 against 6.6). On one that does, the window takes the totals that the gather leaves to a pass of
+// their own, and is the faster at every size (a whole judged step: 16^3 57 us against 61, 64^3 56 against 61).
+constexpr std::size_t kRowCells = std::size_t{1} << 19;
+constexpr long long kRowTiles = 448; // tiles of a conduction window in blocks of eight waves, below which it takes four
 constexpr int kMaxWindowRegisters = 168; // a lane's registers that still leave a window gather three waves a SIMD
 
 struct Impl final : HipBackend {
@@ -266,8 +269,8 @@ struct Impl final : HipBackend {
     // and the store). nullptr otherwise.
     const hip::WindowKernel* fusable(const ir::Program& p, const hip::ProgramCode& code, int field) const
     {
-        const hip::WindowKernel* w = window_for(code);
-        if (w == nullptr || w->flux == 0 || p.writes.size() != 1 || p.writes[0] != field || law->fields[static_cast<std::size_t>(field)].clamp) {
+        const hip::WindowKernel* w = window_for(code, true);
+        if (w == nullptr || !w->totals || p.writes.size() != 1 || p.writes[0] != field || law->fields[static_cast<std::size_t>(field)].clamp) {
             return nullptr;
         }
         return w;
@@ -278,7 +281,7 @@ struct Impl final : HipBackend {
     // range into its record.
     void launch_gather(const hip::ProgramCode& code, double dt, FusedTotal* fused = nullptr)
     {
-        const hip::WindowKernel* w = window_for(code);
+        const hip::WindowKernel* w = window_for(code, fused != nullptr);
         if (w == nullptr) {
             // the direct gather, with 32-bit reads while the lattice (and its spacing) allows them
             last_gather = shape.cells() < (std::size_t{1} << 30) && spacing_flags() >= 3 ? code.gather + "_32" : code.gather;
@@ -289,7 +292,7 @@ struct Impl final : HipBackend {
         int zchunk = zchunk_override > 0 ? zchunk_override : (w->zchunk > 0 ? w->zchunk : code.zchunk);
         int tx = (shape.nx + 64 * w->vx - 1) / (64 * w->vx);
         int ty = (shape.ny + w->ty - 1) / w->ty;
-        const Tiling rows = w->flux == 3 ? row_tiling() : Tiling{};
+        const Tiling rows = w->flux == 3 ? row_tiling(w->block_y) : Tiling{};
         if (w->flux == 3) {
             zchunk = zchunk_override > 0 ? zchunk_override : rows.zchunk;
             tx = rows.tx;
@@ -357,19 +360,21 @@ struct Impl final : HipBackend {
     // MI355X, 128 MB (256^3) and 64 MB run faster in 16-plane chunks, 256 MB (512^2 x 128) and 250 MB (320^3) in 32.
     bool flux_cached() const { return 8.0 * static_cast<double>(shape.cells()) <= 160.0 * 1024 * 1024; }
 
-    // How the conduction window for any row length (flux 3) covers this lattice: 2^lanes_log2 lanes a row, four cells a lane, eight
-    // waves a block. The lanes whose tiles the lattice fills best, more lanes a row where they are as good (fewer halo
-    // rows); then chunks of planes while the launch has two tiles a CU, shorter down to 4 planes.
+    // How the conduction window for any row length (flux 3) covers this lattice: 2^lanes_log2 lanes a row, four cells a lane,
+    // eight or four waves a block. The lanes whose tiles the lattice fills best, more lanes a row where they are as good (fewer
+    // halo rows); then chunks of planes while the launch has two tiles a CU, shorter down to 4 planes. Blocks of four waves
+    // are for the lattices where that leaves the launch short of tiles: as many equal chunks as give two tiles a CU, of two
+    // planes or more (a chunk reads two planes beside its own: 512^2 x 2 in chunks of one takes 4.8 us, in one of two 4.2).
     struct Tiling {
         int lanes_log2 = 0, tx = 0, ty = 0, zchunk = 0;
         long long tiles = 0;
     };
-    Tiling row_tiling() const
+    Tiling row_tiling(int waves) const
     {
         Tiling best;
         double best_fill = 0.0;
         for (int lw = 6; lw >= 3; --lw) {
-            const int width = 4 << lw, rows = 512 >> lw;
+            const int width = 4 << lw, rows = (64 * waves) >> lw;
             const int tx = (shape.nx + width - 1) / width, ty = (shape.ny + rows - 1) / rows;
             const double fill = static_cast<double>(shape.nx) * shape.ny / (1.0 * tx * width * ty * rows);
             if (fill > best_fill * 1.03) {
@@ -381,6 +386,13 @@ struct Impl final : HipBackend {
         }
         best.zchunk = flux_cached() ? 16 : 32;
         auto tiles = [&] { return 1LL * best.tx * best.ty * ((shape.nz + best.zchunk - 1) / best.zchunk); };
+        if (waves == 4) {
+            const long long plane = 1LL * best.tx * best.ty;
+            const int parts = static_cast<int>(std::max<long long>(1, std::min<long long>((512 + plane - 1) / plane, shape.nz / 2)));
+            best.zchunk = std::min(best.zchunk, (shape.nz + parts - 1) / parts);
+            best.tiles = tiles();
+            return best;
+        }
         while (best.zchunk > 4 && tiles() < 512) {
             best.zchunk /= 2;
         }
@@ -389,16 +401,21 @@ struct Impl final : HipBackend {
     }
 
     // The window gather for this lattice. A conduction term: the flux-carrying window for rows of whole quads that fill
-    // one 256-wide tile while the lattice sits in the last-level cache and the launch has two tiles a CU; for any other
-    // row, size or number of tiles the one that takes every row (its chunks of planes shorten). Measured on MI355X a step,
-    // that form against what ran before: 100^3 6.6 us against 8.3, 128^3 7.4 against 12.3, 200^3 21.5 against 32.0,
-    // 256 x 128^2 10.9 against 15.4, 333 x 301 x 200 39 against 66, 501 x 333 x 290 89 against 117, 512 x 512 x 128 50
-    // against 69, 512^3 208 against 214, 1024 x 512 x 256 203 against 214. Any other term: four cells a lane where
+    // one 256-wide tile while the lattice sits in the last-level cache and its tiles of 16 planes fill whole rounds of one a
+    // CU, or come to more than two (256^2 x 240, 480 tiles: 25.2 us a step, judged 82, against the other form's 28.1 and 93;
+    // x 120, 256 tiles: 17.0 and 70 against 18.0 and 78; x 160, 320 tiles: 22.9 and 80 against 22.0 and 82); for any other row,
+    // size or number of tiles the one that takes every row (its chunks of planes shorten), in blocks of eight waves where
+    // those give the launch tiles enough, else, and on a step that is judged, of four. Measured on MI355X a step, the eight-wave form against what ran
+    // before: 200^3 21.5 us against 32.0, 256 x 128^2 11.1 against 19.9, 333 x 301 x 200 39 against 66, 501 x 333 x 290 89
+    // against 117, 512 x 512 x 128 50 against 69, 512^3 208 against 214, 1024 x 512 x 256 203 against 214; the four-wave form
+    // against the eight-wave one: 512^2 x 4 5.7 against 6.7, 700 x 500 x 5 8.2 against 11.1, 100^3 5.9 against 7.4, 512^2 x 10
+    // 9.5 against 10.3, 128^3 7.4 against 7.5 (and, from where the eight waves have 448 tiles, 256^2 x 60 11.3 against 10.9,
+    // 1000^2 x 1 6.2 against 5.7, 1024^2 x 2 8.1 against 7.2). Any other term: four cells a lane where
     // rows are whole float4s, else a cell a lane. Among windows of one kind, the tallest tile that still leaves at least
     // 512 tiles (two per CU) to spread (measured on MI355X, the generic window at z-chunks of 32: 256^3 29.1 us with 256x4
     // tiles against 31.2 with 256x2 and 39.9 with 256x6; 512^3 219 us with 256x6 against 251 and 253). FIELD_HIP_TILE
-    // (e.g. "4x2", "1x6", "h4x8" and "r4x8" for the two flux-carrying forms) picks one. None: the direct gather.
-    const hip::WindowKernel* window_for(const hip::ProgramCode& code) const
+    // (e.g. "4x2", "1x6", "h4x8", "r4x8" and "r4x4" for the flux-carrying forms) picks one. None: the direct gather.
+    const hip::WindowKernel* window_for(const hip::ProgramCode& code, bool judged) const
     {
         // A lattice one row high leaves a window's other rows idle: the direct gather (measured
         // on MI355X, Black-Scholes 4096 x 1 x 512: 16.8 us a pass against 23.8 through 256x2 tiles, and 9.6 with four planes a thread).
@@ -407,9 +424,10 @@ struct Impl final : HipBackend {
         }
         // A conduction term on a lattice of few cells: a step is as long as one tile's march (see kRowCells).
         const bool conduction = std::any_of(code.windows.begin(), code.windows.end(), [](const hip::WindowKernel& w) { return w.flux == 3; });
-        if (conduction && tile_vx == 0 && shape.cells() < kRowCells) {
+        if (conduction && tile_vx == 0 && !judged && shape.cells() < kRowCells) {
             return nullptr;
         }
+        const int row_waves = conduction && (judged || row_tiling(8).tiles < kRowTiles) ? 4 : 8;
         const hip::WindowKernel* best = nullptr;
         auto rank = [&](const hip::WindowKernel& w) {
             if (w.flux == 3) {
@@ -436,7 +454,7 @@ struct Impl final : HipBackend {
                 continue;
             }
             if (tile_vx > 0) {
-                if (w.vx == tile_vx && w.ty == tile_ty && w.flux == tile_flux) {
+                if (w.vx == tile_vx && w.flux == tile_flux && (judged && w.flux == 3 ? w.totals : w.ty == tile_ty)) {
                     return &w;
                 }
                 continue;
@@ -447,8 +465,12 @@ struct Impl final : HipBackend {
             const int zc = zchunk_override > 0 ? zchunk_override : (w.zchunk > 0 ? w.zchunk : code.zchunk);
             const long long tz = (shape.nz + zc - 1) / zc;
             const long long tiles = 1LL * ((shape.nx + 64 * w.vx - 1) / (64 * w.vx)) * ((shape.ny + w.ty - 1) / w.ty) * tz;
-            if (w.flux == 2 && (tiles < 512 || !flux_cached())) {
-                continue; // its chunks do not shorten: the other form's do (256 x 128^2: 11 us against 15)
+            // The whole-quad form's chunks do not shorten: the other form's do (256 x 128^2, 128 tiles: 11 us against 16).
+            if (w.flux == 2 && (!flux_cached() || tiles < 192 || (tiles > 256 && tiles < 384))) {
+                continue;
+            }
+            if (w.flux == 3 && w.block_y != row_waves) {
+                continue;
             }
             if (best == nullptr || rank(w) > rank(*best) || (rank(w) == rank(*best) && w.ty > best->ty && tiles >= 512)) {
                 best = &w;
