@@ -452,7 +452,7 @@ std::string literal(double v)
 
 class Generator {
 public:
-    Generator(const ir::Module& m, const Law& law, LawLayout& lay) : m_(m), law_(law), lay_(lay) {}
+    Generator(const ir::Module& m, const Law& law, LawLayout& lay, Fold fold) : m_(m), law_(law), lay_(lay), fold_(fold) {}
 
     std::string run(std::string& why)
     {
@@ -633,7 +633,7 @@ private:
     // `1 - 2 * a` beside `a`) would read that value's lattice, which the solve does not hold, so it stays stored too.
     std::set<int> folded_;
     static constexpr int kFoldOps = 12;
-    bool fold_cost(int id, int& ops, std::set<int>& fields, const std::set<int>& stages, bool root = true) const
+    bool fold_cost(int id, int& ops, bool& divides, std::set<int>& fields, const std::set<int>& stages, bool root = true) const
     {
         const ir::Inst& in = at(id);
         if (scalar(id)) {
@@ -649,25 +649,27 @@ private:
             if (!by_h(in) && !by_hh(in)) {
                 return false;
             }
+            divides = true;
             break;
         default: return false;
         }
         if (++ops > kFoldOps) {
             return false;
         }
-        return std::all_of(in.args.begin(), in.args.end(), [&](int a) { return fold_cost(a, ops, fields, stages, false); });
+        return std::all_of(in.args.begin(), in.args.end(), [&](int a) { return fold_cost(a, ops, divides, fields, stages, false); });
     }
     void fold_coefficients(std::set<int>& stages)
     {
         const std::set<int> all = stages;
-        std::vector<char> lines(m_.insts.size(), 0), other(m_.insts.size(), 0);
+        std::vector<char> lines(m_.insts.size(), 0), other(m_.insts.size(), 0); // lines: a bit an axis
         for (std::size_t id = 0; id < m_.insts.size(); ++id) {
             if (!used(static_cast<int>(id))) {
                 continue;
             }
             const ir::Inst& in = m_.insts[id];
             for (std::size_t q = 0; q < in.args.size(); ++q) {
-                (in.op == Op::Tridiag && in.index != 0 && q < 3 ? lines : other)[static_cast<std::size_t>(in.args[q])] = 1;
+                char& as = (in.op == Op::Tridiag && q < 3 ? lines : other)[static_cast<std::size_t>(in.args[q])];
+                as = static_cast<char>(as | (in.op == Op::Tridiag && q < 3 ? 1 << in.index : 1));
             }
         }
         for (const auto* progs : {&m_.terms, &m_.learned, &m_.derives}) {
@@ -680,9 +682,13 @@ private:
         for (auto it = stages.begin(); it != stages.end();) {
             const int id = *it;
             int ops = 0;
+            bool divides = false;
             std::set<int> fields;
-            const bool fold = at(id).op != Op::Tridiag && lines[static_cast<std::size_t>(id)] && !other[static_cast<std::size_t>(id)] &&
-                !scalar(id) && fold_cost(id, ops, fields, all) && fields.size() <= 2;
+            bool fold = at(id).op != Op::Tridiag && lines[static_cast<std::size_t>(id)] && !other[static_cast<std::size_t>(id)] &&
+                !scalar(id) && fold_cost(id, ops, divides, fields, all) && fields.size() <= 2;
+            for (int axis = 0; axis < 3; ++axis) {
+                fold = fold && ((lines[static_cast<std::size_t>(id)] >> axis & 1) == 0 || (divides ? fold_.divided : fold_.plain)[axis]);
+            }
             if (fold) {
                 folded_.insert(id);
                 it = stages.erase(it);
@@ -1427,7 +1433,8 @@ private:
                 fetch << "    const double s_" << names[q] << " = " << d(arg) << ";\n";
             } else if (folded_.count(arg) != 0) {
                 int ops = 0;
-                fold_cost(arg, ops, leaves, {});
+                bool divides = false;
+                fold_cost(arg, ops, divides, leaves, {});
             } else {
                 cell.push_back({names[q], arg, -1});
             }
@@ -2888,17 +2895,18 @@ private:
     const ir::Module& m_;
     const Law& law_;
     LawLayout& lay_;
+    const Fold fold_;
     std::ostringstream out_;
     std::vector<char> live_;
 };
 
 } // namespace
 
-std::string generate(const ir::Module& m, const Law& law, LawLayout& layout, std::string& why)
+std::string generate(const ir::Module& m, const Law& law, LawLayout& layout, std::string& why, Fold fold)
 {
     layout = LawLayout{};
     try {
-        return Generator(m, law, layout).run(why);
+        return Generator(m, law, layout, fold).run(why);
     } catch (const std::exception& e) {
         why = e.what();
         return "";

@@ -110,8 +110,14 @@ struct LawLayout {
     int kernel_arg_bytes = 0; // sizeof the generated argument struct
 };
 
+// Whether tridiagonal lines along an axis compute cheap coefficients themselves instead of reading stored ones: those without
+// a division by the spacing, and those with one (the lattice's and its spacing's rule).
+struct Fold {
+    bool plain[3] = {false, true, true};
+    bool divided[3] = {false, true, true};
+};
 // The translation unit of a law, or "" with `why` when it uses an op this backend does not run yet.
-std::string generate(const ir::Module& m, const Law& law, LawLayout& layout, std::string& why);
+std::string generate(const ir::Module& m, const Law& law, LawLayout& layout, std::string& why, Fold fold = {});
 
 // hipRTC options every generated source is compiled with (see the prelude for why each is there).
 std::vector<std::string> compile_options();

@@ -4,7 +4,7 @@ import re
 import numpy as np
 import pytest
 
-HEAD = "field T init 0 range -10 10\nfield w init 1 range 0 10 static\nparam k = 0.05\nterm t\n  let a = k * w * dt / (h * h)\n"
+HEAD = "field T init 0 range -10 10\nfield w init 1 range 0 10 static\nparam k = 0.05\nterm t\n  let a = k * w * dt / {by}\n"
 # Coefficients built from one another: `a` is one itself (stored for the others that read it), or only a part of them.
 FORMS = {
     "shared": ("a", "1 - 2 * a", "a"),
@@ -14,10 +14,10 @@ FORMS = {
 }
 
 
-def law_text(form, axis):
+def law_text(form, axis, by="(h * h)"):
     low, mid, up = FORMS[form]
     lets = "  let c = 0 - a\n" if "c" in low else ""
-    return HEAD + lets + f"  d T = (tridiag_{axis}({low}, {mid}, {up}, T) - T) / dt\n"
+    return HEAD.format(by=by) + lets + f"  d T = (tridiag_{axis}({low}, {mid}, {up}, T) - T) / dt\n"
 
 
 @pytest.mark.parametrize("axis", ["y", "z"])
@@ -41,25 +41,28 @@ def test_a_folded_coefficient_reaches_no_stored_lattice(form, axis):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("h", [0.25, 0.3], ids=["pow2", "any_h"])
+@pytest.mark.parametrize("fold", ["0", "1"], ids=["stored", "computed"])
+@pytest.mark.parametrize("h,by,dt", [(0.25, "(h * h)", 0.125), (0.3, "(h * h)", 0.125), (0.3 * 2.0 ** -110, "h", 0.25 * 2.0 ** -110)],
+                         ids=["pow2", "any_h", "past_the_reciprocal"])
 @pytest.mark.parametrize("axis", ["y", "z"])
 @pytest.mark.parametrize("form", FORMS)
-def test_coefficients_built_from_one_another_solve_as_given_ones(device, form, axis, h):
+def test_coefficients_built_from_one_another_solve_as_given_ones(device, monkeypatch, form, axis, h, by, dt, fold):
     """The same coefficients, rounded to float node by node as the law's, given as fields of their own: the same bits."""
     import field_hip
 
-    shape, dt, f32 = (17, 21, 19), 0.125, np.float32
+    monkeypatch.setenv("FIELD_HIP_FOLD", fold)
+    shape, f32 = (17, 21, 19), np.float32
     n = int(np.prod(shape))
     rng = np.random.default_rng(3)
     t0, w = rng.uniform(-1, 1, n).astype(f32), rng.uniform(0.5, 2.0, n).astype(f32)
-    s = field_hip.Solver(field_hip.Law(law_text(form, axis)), shape, h)
+    s = field_hip.Solver(field_hip.Law(law_text(form, axis, by)), shape, h)
     s.set_field("T", t0)
     s.set_field("w", w)
     s.step(dt)
 
     r = lambda v: np.asarray(v, np.float64).astype(f32)  # a node: doubles, one rounding to float
     d = lambda v: v.astype(np.float64)
-    a = r(d(r(d(r(0.05 * d(w))) * dt)) / (h * h))
+    a = r(d(r(d(r(0.05 * d(w))) * dt)) / (h * h if by != "h" else h))
     c = r(0.0 - d(a))
     two = lambda v: r(2.0 * d(v))
     low, mid, up = {
