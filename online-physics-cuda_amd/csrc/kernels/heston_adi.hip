@@ -747,9 +747,10 @@ struct fe_heston {
 
     // The members that take their steps together before the next ones begin. A pass reads what the one before wrote, three
     // lattices of 4 bytes a cell: at 16M cells those are 192 MB, and part of each is still in the 256 MB last-level cache.
-    // 2048 options (three classes), 64 steps: 62.2 ms in one piece, 59.9 at 16M, 61 at 32M; at 8M and below the passes no
-    // longer fill the card (62.5 and more).
-    static constexpr long long kChunkCells = 1LL << 24;
+    // A part has at least kPartCells, because the passes of a smaller one no longer fill the card: 512 x 256, 32 steps, 130
+    // options 4.5 ms in one part of 17M cells and 5.4 in two, 200 options 6.7 and 7.1, 250 options (33M) 8.8 and 8.2, 300
+    // options 11.0 in one, 9.9 in two, 10.7 in three. 2048 options of three classes, 64 steps: 62.2 ms in one part a class, 59.9 so.
+    static constexpr long long kPartCells = 14LL << 20;
 
     void build_tasks(Class& c)
     {
@@ -759,7 +760,7 @@ struct fe_heston {
         for (const int o : c.members) {
             cells += 1LL * c.nx * host_opts[static_cast<std::size_t>(o)].ny;
         }
-        const long long parts = (cells + kChunkCells - 1) / kChunkCells, most = parts > 0 ? (cells + parts - 1) / parts : 0;
+        const long long parts = std::max(1LL, cells / kPartCells), most = (cells + parts - 1) / parts;
         c.chunks.clear();
         for (const int o : c.members) {
             const int ny = host_opts[static_cast<std::size_t>(o)].ny;

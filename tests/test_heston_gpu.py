@@ -163,14 +163,14 @@ def test_column_sweeps_in_lds_give_the_same_bits(device):
 
 @pytest.mark.parametrize("scheme", [0, 1], ids=["cs", "hv"])
 def test_a_class_stepped_in_parts_gives_the_bits_of_one_part(device, scheme):
-    """More than 2^24 cells of one class take their steps in several launches each; the options are independent, so the
+    """A class of many cells takes its steps in several launches each; the options are independent, so the
     same option has the same bits wherever it stands, run step by step, several at once or from a captured graph."""
     import field_hip
 
     few = draw(5, 31, ((512, 256),))
     ref = field_hip.HestonBatch(*few, 16, scheme)
     ref.step(4)
-    copies = 52  # 5 x 52 x 512 x 256 = 34M cells: three parts
+    copies = 52  # 5 x 52 x 512 x 256 = 34M cells: two parts
     b = field_hip.HestonBatch(np.tile(few[0], copies), np.tile(few[1], copies), np.tile(few[2], (copies, 1)), 16, scheme)
     b.step(1)
     b.step(3)
