@@ -283,8 +283,9 @@ struct Impl final : HipBackend {
     {
         const hip::WindowKernel* w = window_for(code, fused != nullptr);
         if (w == nullptr) {
-            // the direct gather, with 32-bit reads while the lattice (and its spacing) allows them
-            last_gather = shape.cells() < (std::size_t{1} << 30) && spacing_flags() >= 3 ? code.gather + "_32" : code.gather;
+            // the direct gather, with 32-bit reads while the lattice (a cell's index, and a row's bytes) and its spacing allow
+            // them: 1024^3, three reads off the cell, 11.8 ms four steps against 12.8
+            last_gather = shape.cells() < (std::size_t{1} << 31) && shape.nx < (1 << 30) && spacing_flags() >= 3 ? code.gather + "_32" : code.gather;
             launch_cells(last_gather, dt);
             return;
         }
