@@ -138,6 +138,12 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4))
             const int r = q / out, i = q % out, row = r0 + r;
             t0[r * dl + i] = row < rows ? T[(long long)row * out + i] : 0.0f;
         }
+        float mw[4]; // the weights of the rows whose outputs this lane holds
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int row = r0 + 4 * g4 + j;
+            mw[j] = M != nullptr && row < rows ? M[row] : 1.0f;
+        }
         __syncthreads();
         for (int k = 0; k < s.layers; ++k) {
             const int ni = s.sizes[k], no = s.sizes[k + 1], ni16 = pad16(ni), la = a_ld(ni), lo = a_ld(no);
@@ -175,7 +181,7 @@ __global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(4))
                             const int row = r0 + r;
                             float d = 0.0f;
                             if (row < rows) {
-                                const float m = M != nullptr ? M[row] : 1.0f;
+                                const float m = mw[j];
                                 const float e = pre * scale - t0[r * dl + col];
                                 loss += 0.5f * m * e * e;
                                 d = m * e * scale;
@@ -402,7 +408,8 @@ struct Pinned {
     }
 };
 
-// Rows, targets and row weights of at most this many floats are read by the pass itself from pinned host memory (each once),
+// Rows, targets and row weights of at most this many floats are read by the pass itself from pinned host memory (each once, a
+// row's weight once a wave: 1024 weighted rows 46 us a step, 47 with a read an output column),
 // where two copies of pageable memory and the loss's way back cost a step 25 us beside its kernels' 27 (1024 rows of 18 + 16
 // floats; 69 -> 43 us a step, 2048 rows 72 -> 47); past that the copy's rate counts and the rows are uploaded as before.
 constexpr std::size_t kStaged = 131072;
