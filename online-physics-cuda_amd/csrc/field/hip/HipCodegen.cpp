@@ -1583,8 +1583,9 @@ private:
                  << "    }\n}\n";
             if (!leaves.empty()) {
                 out_ << "extern \"C\" __global__ __launch_bounds__(64) void " << kernel << "(K k) {\n"
-                     << "    if (FE_POW2(k)) run_" << kernel << "<true, false>(k);\n"
-                     << "    else if ((k.flags & 4) != 0) run_" << kernel << "<false, false>(k);\n    else run_" << kernel << "<false, true>(k);\n}\n";
+                     << (fold_.pow2 ? "    if (FE_POW2(k)) { run_" + kernel + "<true, false>(k); return; }\n" : "")
+                     << (fold_.any ? "    if ((k.flags & 4) != 0) { run_" + kernel + "<false, false>(k); return; }\n" : "")
+                     << (fold_.past ? "    run_" + kernel + "<false, true>(k);\n" : "") << "}\n";
             }
             return;
         }

@@ -115,6 +115,8 @@ struct LawLayout {
 struct Fold {
     bool plain[3] = {false, true, true};
     bool divided[3] = {false, true, true};
+    // The solves' bodies to write: for a spacing that is a power of two, one that is not, one out of that division's range.
+    bool pow2 = true, any = true, past = true;
 };
 // The translation unit of a law, or "" with `why` when it uses an op this backend does not run yet.
 std::string generate(const ir::Module& m, const Law& law, LawLayout& layout, std::string& why, Fold fold = {});

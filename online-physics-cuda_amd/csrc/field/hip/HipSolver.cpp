@@ -518,6 +518,9 @@ struct Impl final : HipBackend {
             const int n = axis == 1 ? shape.ny : shape.nz;
             const std::size_t lines = shape.cells() / static_cast<std::size_t>(n);
             f.plain[axis] = forced != nullptr ? std::atoi(forced) != 0 : lines >= 8192 || n <= (lines >= 2048 ? 512 : 256);
+            f.pow2 = (spacing_flags() & 3) == 3; // one body: three took a law of two solves 1.06 s to compile, one 0.46
+            f.any = !f.pow2 && (spacing_flags() & 4) != 0;
+            f.past = !f.pow2 && !f.any;
             f.divided[axis] = forced != nullptr || (spacing_flags() & 3) == 3 ? f.plain[axis] : lines >= 32768 || n <= 48;
         }
         return f;
