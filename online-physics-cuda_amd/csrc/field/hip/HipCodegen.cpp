@@ -2188,7 +2188,9 @@ private:
     // double-buffered LDS tile (one barrier a plane), its z neighbours from a four-slot register ring loaded three
     // planes ahead. The tile's first and last row waves load its halo rows beside their own row, the others their own row
     // twice (two more waves that only load them measured slower: 256^3 29.4-36.4 us against 27.2). Its quads are vectors of
-    // the compiler's own: in structs of the HIP header's one of its releases kept a plane in private memory. The form for rows of
+    // the compiler's own: in structs of the HIP header's one of its releases kept a plane in private memory. Its step spills
+    // nothing in 120 registers, the step that takes the totals 16 (44 bytes of private memory a lane), and is the fastest there
+    // nevertheless (256^3 judged 83 us against 90 for row_flux_kernels' four waves, which spill none). The form for rows of
     // whole quads that fill a tile while the lattice sits in the last-level cache: at 256^3 27.9 us against 28.2-28.9
     // for row_flux_kernels' form, which wins past it (512 x 512 x 128: 49.9-52 us against 69).
     // The CPU's face sum, in its order (-x, +x, -y, +y, -z, +z; src/field/Law.cpp:986-1018), from fluxes computed once
@@ -2368,9 +2370,9 @@ private:
     // last-level cache and for few tiles (`_r_`). The fluxes, their sharing and their order are flux_kernels'; what differs is how a wave
     // covers rows. Its 64 lanes are W lanes a row (8, 16, 32 or 64, the launch's choice: mode >> 8 is its logarithm) on
     // 64 / W consecutive rows, four cells a lane, so a tile of TY waves is 4W cells by TY * 64 / W rows and the launch picks the
-    // W whose tiles the rows fill best. Eight waves (fewer halo rows) hold four waves a SIMD in 128 registers, four of which
-    // spill outside the planes' loop's loads; four waves (more tiles where the lattice gives few) may take 256 and spill none,
-    // and alone take the totals, whose sums would cost the eight 24 spilled registers a plane: 512 x 512 x 128 judged 127 us a
+    // W whose tiles the rows fill best. Eight waves (fewer halo rows) run four a SIMD in 128 registers, of which
+    // four spill (20 bytes of private memory a lane); four waves (more tiles where the lattice gives few) may take 256 and spill
+    // none, and alone take the totals, for which the eight would spill 24 more (68 bytes): 512 x 512 x 128 judged 127 us a
     // step against 133, 384^3 195 against 205, 256 x 256 x 160 78 against 82. Row starts are not 16-byte aligned (the quads are loaded as such; the card takes a
     // 4-byte aligned quad), and a row's last quad is read from the row's last four cells and moved up, the last cell
     // repeated behind it: its face to the cells that are not there then has a flux of +0, as a closed face's.

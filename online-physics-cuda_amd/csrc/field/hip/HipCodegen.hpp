@@ -83,8 +83,8 @@ struct WindowKernel {
 };
 
 struct ProgramCode {
-    std::string gather;     // empty: no equations. The direct gather: a thread a cell, blocks of 64 x 4 over (x, y),
-                            // one z-plane a block row; always there.
+    std::string gather;     // empty: no equations. The direct gather: a thread a cell, blocks of 64 cells of four rows (of
+                            // four planes where a plane has fewer); always there.
     bool window = false;    // window gathers exist (then one of them runs)
     int radius = 0;
     int zchunk = 0;

@@ -108,7 +108,7 @@ struct Impl final : HipBackend {
     // other): FIELD_HIP_TILE="<cells a lane>x<rows>", FIELD_HIP_ZCHUNK=<planes a tile>, FIELD_HIP_DIRECT=1,
     // FIELD_HIP_REMAP=0|1 (tiles in XCD runs), FIELD_HIP_STREAM=0|1 (streaming stores).
     int tile_vx = 0, tile_ty = 0, zchunk_override = 0, remap_override = -1, stream_override = -1;
-    int tile_flux = 0; // FIELD_HIP_TILE named a flux-carrying window: 2 "h4x8", 3 "r4x8"
+    int tile_flux = 0; // FIELD_HIP_TILE named a flux-carrying window: 2 "h4x8", 3 "r4x8", "r4x4"
     bool force_direct = false;
     std::string last_gather;
     std::vector<void*> own; // per field bound to a caller's buffer: its own array (else null)
@@ -419,7 +419,7 @@ struct Impl final : HipBackend {
     const hip::WindowKernel* window_for(const hip::ProgramCode& code, bool judged) const
     {
         // A lattice one row high leaves a window's other rows idle: the direct gather (measured
-        // on MI355X, Black-Scholes 4096 x 1 x 512: 16.8 us a pass against 23.8 through 256x2 tiles, and 9.6 with four planes a thread).
+        // on MI355X, Black-Scholes 4096 x 1 x 512: 16.8 us a pass against 23.8 through 256x2 tiles, and 9.6 in blocks of four planes).
         if (!code.window || code.windows.empty() || force_direct || spacing_flags() < 3 || (shape.ny == 1 && tile_vx == 0)) {
             return nullptr;
         }
@@ -483,7 +483,7 @@ struct Impl final : HipBackend {
     void read_overrides()
     {
         if (const char* t = std::getenv("FIELD_HIP_TILE")) {
-            tile_flux = t[0] == 'f' ? 1 : (t[0] == 'h' ? 2 : (t[0] == 'r' ? 3 : 0));
+            tile_flux = t[0] == 'h' ? 2 : (t[0] == 'r' ? 3 : 0);
             if (std::sscanf(t + (tile_flux != 0 ? 1 : 0), "%dx%d", &tile_vx, &tile_ty) != 2) {
                 tile_vx = tile_ty = 0;
                 tile_flux = 0;
@@ -557,7 +557,8 @@ struct Impl final : HipBackend {
     }
 
     // Generic window gathers that would run badly: private (scratch) memory, or more registers a lane than leave three waves a
-    // SIMD (four cells a lane of a law with many fields). The automatic choice passes them over.
+    // SIMD (four cells a lane of a law with many fields). The automatic choice passes them over. The conduction windows are
+    // not weighed: two of them spill a little and were measured to be the faster with it.
     std::set<std::string> heavy;
     void weigh_windows()
     {

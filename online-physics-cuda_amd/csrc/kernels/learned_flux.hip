@@ -65,7 +65,6 @@ __device__ __host__ __forceinline__ unsigned short to_bf16_bits(float f)
 
 // Round to nearest even: the hardware conversion (v_cvt_pk_bf16_f32 on gfx950), what to_bf16_bits computes by bits.
 __device__ __forceinline__ __bf16 bf(float f) { return static_cast<__bf16>(f); }
-__device__ __forceinline__ float unbf(__bf16 b) { return __builtin_bit_cast(float, static_cast<unsigned int>(__builtin_bit_cast(unsigned short, b)) << 16); }
 
 // GELU, tanh form: 0.5 z (1 + tanh u), u = sqrt(2 / pi) (z + 0.044715 z^3), computed as z s with s = 1 / (1 + e^(-2u))
 // (the same function: 0.5 (1 + tanh u) is the logistic of 2u), e^(-2u) as 2^(z (a + b z^2)) with the constants folded,
@@ -904,7 +903,7 @@ struct fe_lnet {
     int adam_step = 0;
     std::string error;
     hipStream_t stream() const { return static_cast<hipStream_t>(fe_hip_stream()); }
-    static constexpr int kFaceBlocks = 1024; // face kernels: waves in flight (a grid-stride loop over 16-row tiles)
+    static constexpr int kFaceBlocks = 1024; // face kernels: blocks of four waves, each looping over 32 rows (two tiles) a trip
     static constexpr int kTrainBlocks = 1024; // one wave a SIMD: the training pass holds 408 registers a lane
 };
 

@@ -127,6 +127,16 @@ def test_infinities_and_nan_at_tile_corners_follow_the_oracle(device, monkeypatc
     assert np.array_equal(got[~nan].view(np.uint32), want[~nan].view(np.uint32))
 
 
+def test_an_override_that_names_no_form_is_ignored(device, monkeypatch):
+    import field_hip
+
+    monkeypatch.setenv("FIELD_HIP_TILE", "f4x4")
+    solver = field_hip.Solver(field_hip.Law(LAW), (16, 16, 16), 1.0)
+    solver.set_field("T", np.random.default_rng(1).random(4096, dtype=np.float32))
+    solver.step(0.1)
+    assert solver.profile()["terms"][0]["kernel"].endswith("_r_4")
+
+
 @pytest.mark.parametrize("shape,judged,plain", [((16, 16, 16), "_r_4", "_32"), ((64, 64, 64), "_r_4", "_32"), ((512, 512, 2), "_r_4", "_r_4"),
                                                 ((3, 40, 40), "_32", "_32"), ((40, 1, 40), "_32", "_32")],
                          ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else v.strip("_"))
