@@ -2127,21 +2127,27 @@ private:
         for (const bool w32 : {false, true}) {
             const std::string w = w32 ? "true" : "false", fn = "d_" + code.gather + "<DirectT<" + w;
             g << "extern \"C\" __global__ void " << code.gather << (w32 ? "_32" : "") << "(K k) { CELL_HEAD\n";
-            if (by_spacing) {
-                g << "    if (!FE_POW2(k)) { " << fn << ", false>>(k, x, y, z); return; }\n";
-            }
+            std::string clear;
             if (w32) {
                 // A row clear of the y and z edges (the whole wave's, so no lanes part) takes the inner forms: no clamps, no
-                // face conditions, shift_t one read. A law that reads along x alone is clear of them everywhere.
-                std::string clear;
+                // face conditions, shift_t one read. A law that reads along x alone is clear of them everywhere. The test is
+                // two comparisons an axis where the law's ops make the same ones, which the compiler then drops (a pour of
+                // water over 144 x 144 x 48: 22.6 us, 26.3 behind the shorter test).
                 for (const auto& [axis, off] : {std::pair<std::string, int>{"y", off_y}, {"z", off_z}}) {
                     if (off > 0) {
-                        clear += (clear.empty() ? "" : " && ") + ("min(" + axis + ", k.n" + axis + " - 1 - " + axis + ") >= " + std::to_string(off));
+                        const std::string o = std::to_string(off), n = "k.n" + axis;
+                        clear += (clear.empty() ? "" : " && ") + (by_spacing ? axis + " >= " + o + " && " + axis + " + " + o + " < " + n
+                                                                            : "min(" + axis + ", " + n + " - 1 - " + axis + ") >= " + o);
                     }
                 }
-                g << "    " << (clear.empty() ? "" : "if (" + clear + ") ") << "{ if (" << fn << ", true, true>>(k, x, y, z)) return; }\n";
             }
-            g << "    " << fn << ", true>>(k, x, y, z);\n}\n";
+            const std::string general = fn + ", true>>(k, x, y, z);\n";
+            const std::string inner = !w32 ? "" : "if (" + (clear.empty() ? "" : clear + " && ") + fn + ", true, true>>(k, x, y, z)) return;\n";
+            if (by_spacing) {
+                g << "    if (FE_POW2(k)) {\n        " << inner << "        " << general << "    }\n    else " << fn << ", false>>(k, x, y, z);\n}\n";
+            } else {
+                g << "    " << inner << "    " << general << "}\n";
+            }
         }
         out_ << g.str();
         int radius = 0;
