@@ -398,13 +398,17 @@ struct Pinned {
         if (count <= n) {
             return;
         }
+        std::size_t size = 1024; // by doubling: calls of a few more rows each find room
+        while (size < count) {
+            size *= 2;
+        }
         if (p != nullptr) {
             hcheck(hipHostFree(p), "free");
             p = nullptr;
             n = 0;
         }
-        hcheck(hipHostMalloc(reinterpret_cast<void**>(&p), count * sizeof(float), hipHostMallocDefault), "pinned allocation");
-        n = count;
+        hcheck(hipHostMalloc(reinterpret_cast<void**>(&p), size * sizeof(float), hipHostMallocDefault), "pinned allocation");
+        n = size;
     }
 };
 
@@ -413,6 +417,7 @@ struct Pinned {
 // where two copies of pageable memory and the loss's way back cost a step 25 us beside its kernels' 27 (1024 rows of 18 + 16
 // floats; 69 -> 43 us a step, 2048 rows 72 -> 47); past that the copy's rate counts and the rows are uploaded as before.
 constexpr std::size_t kStaged = 131072;
+constexpr std::size_t kLossFloats = 16; // ahead of the rows in that memory: the loss, and the rows' alignment
 
 unsigned blocks_for(long long n, int per) { return static_cast<unsigned>((n + per - 1) / per); }
 
@@ -421,7 +426,7 @@ unsigned blocks_for(long long n, int per) { return static_cast<unsigned>((n + pe
 struct fe_nettrain {
     Shape s;
     Dev<float> w, m1, m2, x, t, m, partial, chunks, grad;
-    Pinned staged, loss;         // every call waits for its pass before it returns, so the next may write them
+    Pinned staged;               // the loss, then the rows: every call waits for its pass before it returns, so the next may write them
     const float *rx = nullptr, *rt = nullptr, *rm = nullptr; // the pass's rows, targets and row weights
     int adam_t = 0;
     std::string error;
@@ -448,7 +453,7 @@ struct fe_nettrain {
             sums = chunks.p;
         }
         hipLaunchKernelGGL(k_nt_fold, dim3(blocks_for(width, 256)), dim3(256), 0, st, sums, count, width, static_cast<float>(rows), grad.p, adam,
-            loss.p);
+            staged.p);
         hcheck(hipGetLastError(), "gradient launch");
     }
 
@@ -457,16 +462,19 @@ struct fe_nettrain {
         const hipStream_t st = stream();
         const std::size_t nr = static_cast<std::size_t>(rows), nx = nr * s.sizes[0], nt = nr * s.sizes[s.layers];
         if (nx + nt + nr <= kStaged) {
-            std::memcpy(staged.p, xs, nx * sizeof(float));
-            std::memcpy(staged.p + nx, ts, nt * sizeof(float));
+            staged.alloc(kLossFloats + nx + nt + nr);
+            float* const at = staged.p + kLossFloats;
+            std::memcpy(at, xs, nx * sizeof(float));
+            std::memcpy(at + nx, ts, nt * sizeof(float));
             if (ms != nullptr) {
-                std::memcpy(staged.p + nx + nt, ms, nr * sizeof(float));
+                std::memcpy(at + nx + nt, ms, nr * sizeof(float));
             }
-            rx = staged.p;
+            rx = at;
             rt = rx + nx;
             rm = ms != nullptr ? rt + nt : nullptr;
             return;
         }
+        staged.alloc(kLossFloats);
         x.put(xs, nx, st);
         t.put(ts, nt, st);
         if (ms != nullptr) {
@@ -551,8 +559,6 @@ fe_nettrain* fe_nettrain_create(const int* sizes, int count, int act, char* why,
         }
         image[static_cast<std::size_t>(2 * sizes[0])] = 1.0f;
         t->w.put(image.data(), image.size(), t->stream());
-        t->staged.alloc(kStaged);
-        t->loss.alloc(1);
         std::vector<float> zeros(static_cast<std::size_t>(s.trained), 0.0f);
         t->m1.put(zeros.data(), zeros.size(), t->stream());
         t->m2.put(zeros.data(), zeros.size(), t->stream());
@@ -618,7 +624,7 @@ int fe_nettrain_gradient(fe_nettrain* t, const float* x, const float* target, co
         }
         hcheck(hipStreamSynchronize(st), "sync");
         if (loss != nullptr) {
-            *loss = *t->loss.p;
+            *loss = *t->staged.p;
         }
         return 0;
     } catch (const std::exception& e) {
@@ -643,7 +649,7 @@ int fe_nettrain_step(fe_nettrain* t, const float* x, const float* target, const 
         const hipStream_t st = t->stream();
         hcheck(hipStreamSynchronize(st), "sync");
         if (loss != nullptr) {
-            *loss = *t->loss.p;
+            *loss = *t->staged.p;
         }
         return 0;
     } catch (const std::exception& e) {
