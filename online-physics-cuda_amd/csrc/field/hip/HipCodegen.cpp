@@ -2100,9 +2100,10 @@ private:
         }
         const int nt = static_cast<int>(targets.size());
         // The direct kernel: a thread a cell; `<gather>_32` the same with 32-bit addresses (lattices under 2^31 cells).
-        // False, and nothing written, for a cell the fast forms flag. A light law's waves are bound by their instructions
-        // ahead of the reads: addresses in 32 bits for the stores too, one test for the inner rows and none for the spacing where
-        // nothing divides by it give 256^3, three reads off the cell, 36.9 us against 40.3.
+        // False, and nothing written, for a cell the fast forms flag. A step is as long as its waves live, at full occupancy, and
+        // in a light law what a wave does ahead of its reads is a good part of that: addresses in 32 bits for the stores too,
+        // one test for the inner rows and none for the spacing where nothing divides by it take 256^3, three reads off the cell,
+        // from 40.3 us to 36.9.
         g << "template <class M> __device__ __forceinline__ bool d_" << code.gather << "(const K& k, int x, int y, int z)\n{\n"
           << "    const M m(k);\n    float o[" << nt << "], n[" << nt << "];\n    " << cellfn << "(k, m, x, y, z, o, n);\n"
           << "    if (m.bad) return false;\n";
